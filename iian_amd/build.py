@@ -19,6 +19,7 @@ ROOT = PKG.parent
 CSRC = PKG / "csrc"
 LIB = PKG / "libiian_pa.so"
 SOURCES = ["pa_abi.hip", "pa_decode.hip", "pa_decode_q8.hip", "pa_prefill.hip", "pa_prefill16.hip", "pa_general.hip",
+           "pa_gen_mfma.hip", "pa_gen_mfma_f32.hip", "pa_gen_mfma_q8.hip",
            "pa_kv_write.hip", "pa_batch.hip", "pa_rope.hip", "pa_runtime.hip"]
 ARCH = "gfx950"
 

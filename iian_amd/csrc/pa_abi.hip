@@ -45,6 +45,13 @@ constexpr int kF16DecodeWavesPerCuD256 = 3;
 // unit of work): 4 waves per CU measured best at Phi-3.5 shapes (414 us
 // against 420 at 3, 426 at 6, 455 at 2).
 constexpr int kF16DecodeWavesPerCuPairs = 4;
+// Matrix-core general path: decode waves per CU (its kernels hold two waves
+// per SIMD at head sizes up to 128, one above), alone and beside prefill
+// workgroups, and the prefill workgroups per CU a launch aims for.
+constexpr int kGenDecodeWavesPerCu = 8;
+constexpr int kGenMixedDecodeWavesPerCu = 4;
+constexpr int kGenDecodeWavesPerCuWide = 4;
+constexpr int kGenPrefillWgsPerCu = 2;
 constexpr int kQ8DecodeWavesPerCu = 8;
 constexpr int kMaxWavesPerCu = kQ8DecodeWavesPerCu;
 constexpr int kDefaultCus = 256;   // an MI355X, when the device cannot be queried
@@ -247,6 +254,17 @@ bool mfma_path(int type_k, int type_v, int head_dim, int head_dim_v, int bs_log2
            head_dim == head_dim_v && (head_dim == 64 || head_dim == 128 || head_dim == 256) && bs_log2 >= 3;
 }
 
+// The matrix-core general kernels (pa_gen_mfma.h): every pool type, the head
+// sizes of gen_mfma_chunks, blocks of whole 16-cell steps (a step's rows are
+// then consecutive), pool rows that 32-bit row numbers and 24-bit row lengths
+// address.
+bool gen_mfma_path(int head_dim, int head_dim_v, int32_t block_size, int32_t max_blocks, int32_t num_blocks,
+                   int64_t k_row, int64_t v_row, int64_t rows) {
+    return gen_mfma_chunks(head_dim, head_dim_v) && block_size % 16 == 0 &&
+           (int64_t) num_blocks * block_size <= ((int64_t) 1 << 32) && k_row < (1 << 24) && v_row < (1 << 24) &&
+           (int64_t) max_blocks * block_size <= INT32_MAX / 2 && rows <= (1 << 30);
+}
+
 // Any head size the general kernel stages (1 .. 1024; the reference's op
 // takes any, paged_attn.cpp:96-100); a Q8_0 head slice is whole 32-value
 // blocks.
@@ -366,6 +384,98 @@ int run_attention(hipStream_t st, const float *q, const void *k_pool, const void
                       (int64_t) max_query_len * gqa > kDecodeRowsMax ||
                       !(mfma_path(type_k, type_v, head_dim, head_dim_v, bs_log2) || f16_96)))
         return IIAN_PA_ERR_UNSUPPORTED;
+    if (!mfma_path(type_k, type_v, head_dim, head_dim_v, bs_log2) && !f16_96 &&
+        gen_mfma_path(head_dim, head_dim_v, block_size, max_blocks, num_blocks, kr, vr,
+                      (int64_t) n_tokens * gqa)) {
+        GenMfmaParams g = {};
+        AttnParams &a = g.a;
+        a.q = q;
+        a.k_pool = (const char *) k_pool;
+        a.v_pool = (const char *) v_pool;
+        a.bt = block_tables;
+        a.seq_lens = seq_lens;
+        a.qsl = query_start_loc;
+        a.pos = pos;
+        a.out = out;
+        a.err = err_flag;
+        a.k_row = kr;
+        g.v_row = vr;
+        a.max_blocks = max_blocks;
+        a.num_blocks = num_blocks;
+        a.T = n_tokens;
+        a.S = n_seqs;
+        a.H = n_head;
+        a.Hkv = n_head_kv;
+        a.gqa = gqa;
+        a.softcap = softcap;
+        a.causal = causal ? 1 : 0;
+        a.n_swa = n_swa;
+        a.max_q = max_query_len;
+        a.head_group = 1;
+        a.rec_heads = 1;
+        g.D = head_dim;
+        g.Dv = head_dim_v;
+        g.block_size = block_size;
+        g.bs_log2 = bs_log2;
+        g.sscale = softcap > 0.0f ? scale : scale * kLog2e;
+        // Rows: sequences with at most 16 rows per kv head go to the stream-K
+        // workers, the others to 64-row prefill workgroups.
+        const int64_t max_rows = (int64_t) max_query_len * gqa;
+        const bool decode_only = max_rows <= 16;
+        const bool no_decode =
+            !decode_only && ((int64_t) n_tokens - (int64_t) (n_seqs - 1) * max_query_len) * gqa > 16;
+        const int waves = head_dim > 128 ? kGenDecodeWavesPerCuWide
+                          : decode_only                        ? kGenDecodeWavesPerCu
+                                                               : kGenMixedDecodeWavesPerCu;
+        a.decode_rows = no_decode ? 0 : 16;
+        a.rec_rows = 16;
+        a.rec_stride = (int64_t) 16 * head_dim_v + kRecordPad;
+        a.sk_workers = no_decode ? 0 : waves * cus;
+        const size_t cap = src.scratch ? kScratchBytes : wl.total;
+        WorkspaceLayout xl = exact_layout(a);
+        if (a.sk_workers && xl.total > cap) {   // no room for decode records: every row unsplit or split by range
+            a.decode_rows = 0;
+            a.sk_workers = 0;
+            xl = exact_layout(a);
+        }
+        if (!a.sk_workers) xl = {};
+        g.n_dec_wgs = a.sk_workers / 4;
+        g.n_split = 1;
+        int64_t pre_wgs = 0;
+        size_t split_o = 0, need = xl.total;
+        if (a.decode_rows == 0 || !decode_only) {
+            // 64-row blocks the batch can hold: one more than rows/64 for
+            // every sequence that is not a decode one
+            const int64_t rows = (int64_t) n_tokens * gqa;
+            const int64_t n_rb = rows / 64 + std::min<int64_t>(n_seqs, rows / (a.decode_rows + 1));
+            // Ranges per row block: until the launch holds about
+            // kGenPrefillWgsPerCu workgroups per CU, each range at least 8
+            // tiles of the longest table, the records inside the workspace
+            const int64_t full = std::max<int64_t>(1, rows / 64) * n_head_kv;
+            const int64_t max_tiles = ((int64_t) max_blocks * block_size + kTile - 1) / kTile;
+            int64_t ns = ((int64_t) kGenPrefillWgsPerCu * cus + full - 1) / full;
+            ns = std::min<int64_t>({ns, std::max<int64_t>(1, max_tiles / 8), 16});
+            const size_t per_split = (size_t) n_tokens * n_head * (head_dim_v + 2) * sizeof(float);
+            if (ns > 1)
+                ns = std::min<int64_t>(ns, (int64_t) ((cap - std::min(cap, align256(xl.total) + 512)) / per_split));
+            g.n_split = (int) std::max<int64_t>(ns, 1);
+            pre_wgs = n_rb * n_head_kv * g.n_split;
+            if (g.n_split > 1) {
+                split_o = align256(xl.total);
+                need = split_o + align256((size_t) n_tokens * n_head * g.n_split * head_dim_v * sizeof(float)) +
+                       (size_t) n_tokens * n_head * g.n_split * 2 * sizeof(float);
+            }
+        }
+        const int rc = ws_resolve(src, st, need, &ws);
+        if (rc) return rc;
+        a.part_o = (float *) (ws + xl.o);
+        a.part_ml = (float *) (ws + xl.ml);
+        a.seg_info = (int2 *) (ws + xl.seg);
+        g.split_o = (float *) (ws + split_o);
+        g.split_ml = (float *) (ws + split_o +
+                                align256((size_t) n_tokens * n_head * g.n_split * head_dim_v * sizeof(float)));
+        return launch_gen_mfma(g, type_k, type_v, pre_wgs, st) == hipSuccess ? IIAN_PA_OK : IIAN_PA_ERR_HIP;
+    }
     if (!mfma_path(type_k, type_v, head_dim, head_dim_v, bs_log2) && !f16_96) {
         // General fp32 path.  Cell indices within a sequence and pool rows
         // are int32 / int64 there.

@@ -1,0 +1,741 @@
+// pa_gen_mfma.h - matrix-core attention for the pool types and head sizes the
+// f16 / Q8_0 kernels are not built for (pa_gen_mfma_*.hip, one file per K type).
+//
+// K and V each F32, F16 or Q8_0 in any pairing, head sizes up to 256 (D a
+// multiple of 8, Dv of 4, gen_mfma_chunks), blocks of a multiple of 16 cells,
+// Dv != D.  Precision is that of
+// pa_general_kernel, which keeps every other combination: nothing of the
+// computation drops below 32 bits.
+//
+//   K F32 or Q8_0  S^T = K Q^T on v_mfma_f32_16x16x4_f32; a Q8_0 value is
+//                  q * fp32(d), exactly dequantize_row_q8_0 (ggml-quants.c:553-567)
+//   K F16          K is exact in f16, and q goes in as three f16 terms (11 + 11
+//                  + 11 bits, each rounded toward zero: the whole fp32 value)
+//                  on v_mfma_f32_16x16x32_f16: 3 x 16 cycles per 32 dims where
+//                  the fp32 form takes 8 x 32
+//   V F32 or Q8_0  O += P V on the fp32 MFMA, P in fp32
+//   V F16          V exact, P as two f16 terms (22 bits), on the f16 MFMA
+//
+// Work split.  One wave owns 16 query rows (r = j*gqa + g) of one (sequence,
+// kv head) and walks 32-cell tiles (16 when V is not F16) straight from the block table: K rows are
+// the A operand of S^T as they lie in memory (lane (n, g): cell n, dims
+// 8g .. 8g+7 of each 32), S^T's result layout (lane (n, g): cells 4g .. 4g+3
+// of row n) is PV's A operand, and V rows are read 4 dims per lane, so
+// nothing passes through LDS and no two waves wait for each other.  The next
+// tile's K loads go out after QK^T, its V loads after PV, its table entries
+// one tile earlier still.
+//   - sequences with at most 16 rows per kv head (decode): stream-K, as the
+//     f16 decode kernel (pa_common.h): every wave of the first n_dec_wgs
+//     workgroups takes an equal range of the call's (sequence, kv head, tile)
+//     line and leaves partial records for the merge;
+//   - the others (prefill chunks): a 4-wave workgroup takes 64 consecutive rows
+//     and one of n_split ranges of their tiles.  Its waves read the same tiles
+//     at about the same time, so the CU's L1 serves three of the four.
+// Both kinds run in one launch, so the memory-bound decode waves share the CUs
+// with the chunks' MFMAs.  One merge launch follows when anything was split.
+//
+// What bounds it: decode, HBM; chunks over F32 or Q8_0, the fp32 MFMA (64
+// flop per cycle and SIMD); chunks over F16, the L1 (16 KB of K and V per 640
+// MFMA cycles at head size 128).  Measured against pa_general_kernel (one
+// MI355X, whole calls): 32 decodes of 512-8192 cells over F32 pools, H32/Hkv8/
+// D128, 215 -> 158 us (5.2 TB/s); 2 chunks and 16 decodes over F32 1448 -> 211
+// us; 2 chunks and 16 decodes over F16 at H32/Hkv32/D80 9030 -> 156 us.
+// Distance from a 64-bit result there: 6.5e-7 -> 4.1e-7 (F32), 6.3e-7 ->
+// 5.7e-7 (F16, D80).
+#pragma once
+
+#include "pa_common.h"
+#include "pa_launch.h"
+#include "pa_merge.h"
+
+namespace iian_pa {
+
+constexpr int kGmWaves = 4;
+constexpr int kGmRows = 16;                       // query rows per wave
+constexpr int kGmBlockRows = kGmWaves * kGmRows;  // rows per prefill workgroup
+
+struct __attribute__((packed, aligned(2))) u32x2_a2 {
+    uint32_t x, y;
+};
+struct __attribute__((packed, aligned(2))) u32_a2 {
+    uint32_t x;
+};
+
+template <int KT>
+struct GmK {   // 8 dims of one cell
+    u32x4 a;
+};
+template <>
+struct GmK<0> {
+    u32x4 a, b;
+};
+template <>
+struct GmK<8> {
+    uint32_t x, y;
+    uint16_t d;
+};
+template <int VT>
+struct GmV {   // 4 dims of one cell
+    u32x4 a;
+};
+template <>
+struct GmV<1> {
+    u32x2 a;
+};
+template <>
+struct GmV<8> {
+    uint32_t x;
+    uint16_t d;
+};
+
+// A load at a wave-uniform base plus a lane's 32-bit offset (the saddr form:
+// no vector address arithmetic).
+template <typename T>
+__device__ __forceinline__ T gm_ld(const char *base, uint32_t off) {
+    return *(const T *) (base + off);
+}
+
+__device__ __forceinline__ float gm_f16(uint32_t h) { return (float) __builtin_bit_cast(_Float16, (uint16_t) h); }
+
+// f32 value of dim e (0..7) of a F32 or Q8_0 K chunk.
+template <int KT>
+__device__ __forceinline__ float gm_k_f32(const GmK<KT> &k, int e) {
+    if constexpr (KT == 0) {
+        return __uint_as_float(e < 4 ? k.a[e] : k.b[e - 4]);
+    } else {
+        const uint32_t w = e < 4 ? k.x : k.y;
+        return (float) (int8_t) (w >> (8 * (e & 3))) * gm_f16(k.d);
+    }
+}
+template <int VT>
+__device__ __forceinline__ float gm_v_f32(const GmV<VT> &v, int e) {
+    if constexpr (VT == 0) return __uint_as_float(v.a[e]);
+    else return (float) (int8_t) (v.x >> (8 * e)) * gm_f16(v.d);
+}
+
+// One stretch of work of a wave: 16 rows from row0 of (sequence s, kv head
+// hk) over the cells [cb, ce) (ce <= the sequence's length).
+struct GmPiece {
+    int s, hk, q0, M, row0;
+    int pmin, pmax;   // positions of the wave's rows (pmax also stands in for rows past M)
+    int cb, ce;
+    int mode;         // 0: normalised output, 1: stream-K record rec, 2: record z of each row's n_split
+    int rec;
+};
+
+// x = h + m + l exactly, each f16 rounded toward zero.  x is scaled below
+// 2^15 by the caller.  m and l are kept non-zero (2^-24) where h alone is
+// exact, so that an infinite K element times the three terms gives one signed
+// infinity, as its fp32 product does, and never inf * 0.  The differences
+// pass through empty asm: folded into a mixed-precision FMA with a negated
+// operand they have come out wrong (see split_f16x8).
+__device__ __forceinline__ void gm_split3(float x, _Float16 &h, _Float16 &m, _Float16 &l) {
+    typedef __fp16 h2 __attribute__((ext_vector_type(2)));
+    const uint32_t tiny = (__float_as_uint(x) >> 16 & 0x8000u) | 1u;   // +-2^-24 as f16
+    auto rtz = [](float v) { return __builtin_bit_cast(uint16_t, (__fp16) __builtin_amdgcn_cvt_pkrtz(v, 0.f)[0]); };
+    uint16_t a = rtz(x);
+    float fa = gm_f16(a);
+    asm volatile("" : "+v"(fa));
+    float r1 = x - fa;
+    asm volatile("" : "+v"(r1));
+    uint16_t b = rtz(r1);
+    float fb = gm_f16(b);
+    asm volatile("" : "+v"(fb));
+    float r2 = r1 - fb;
+    asm volatile("" : "+v"(r2));
+    uint16_t c = rtz(r2);
+    if (x != 0.f) {
+        if ((a & 0x7fff) == 0x7c00) b = c = 0;   // an infinite q: one term
+        if ((b & 0x7fff) == 0) b = (uint16_t) tiny;
+        if ((c & 0x7fff) == 0) c = (uint16_t) tiny;
+    }
+    h = __builtin_bit_cast(_Float16, a);
+    m = __builtin_bit_cast(_Float16, b);
+    l = __builtin_bit_cast(_Float16, c);
+}
+
+// NK: 32-dim chunks of K (D <= 32 NK), NV: 64-dim blocks of V (Dv <= 64 NV).
+template <int KT, int VT, int NK, int NV>
+__device__ __forceinline__ void gm_piece(const GenMfmaParams &p, const GmPiece &vp) {
+    const AttnParams &a = p.a;
+    // wave-uniform, and known to be: the tile loop's control and addresses are scalar
+    GmPiece pc;
+    pc.s = __builtin_amdgcn_readfirstlane(vp.s);
+    pc.hk = __builtin_amdgcn_readfirstlane(vp.hk);
+    pc.q0 = __builtin_amdgcn_readfirstlane(vp.q0);
+    pc.M = __builtin_amdgcn_readfirstlane(vp.M);
+    pc.row0 = __builtin_amdgcn_readfirstlane(vp.row0);
+    pc.pmin = __builtin_amdgcn_readfirstlane(vp.pmin);
+    pc.pmax = __builtin_amdgcn_readfirstlane(vp.pmax);
+    pc.cb = __builtin_amdgcn_readfirstlane(vp.cb);
+    pc.ce = __builtin_amdgcn_readfirstlane(vp.ce);
+    pc.mode = __builtin_amdgcn_readfirstlane(vp.mode);
+    pc.rec = __builtin_amdgcn_readfirstlane(vp.rec);
+    constexpr bool KF16 = KT == 1, VF16 = VT == 1;
+    constexpr int NT = VF16 ? 2 : 1;       // 16-cell steps per tile: the f16 PV wants 32 cells per MFMA
+    constexpr int TC = 16 * NT, CV = 4 * NT;   // cells per tile, and V cells per lane
+    // D > 32 (NK - 1) and Dv > 64 (NV - 1) except in the wide kernels (NK = 8,
+    // D > 128), whose later chunks and blocks are skipped when past the size
+    constexpr int JOPT = NK == 8 ? 4 : NK, BOPT = NK == 8 ? 1 : NV;
+    const int lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15;
+    const int D = p.D, Dv = p.Dv;
+    const int rown = pc.row0 + n;
+    const bool rlive = rown < pc.M;
+    int prow = pc.pmax;
+
+    // ---- q of row n, dims 32j + 8g + e ----
+    float qf[KF16 ? 1 : NK][8];
+    f16x8 q3[KF16 ? NK : 1][3];
+    float cs = p.sscale;   // multiplies the raw dot product
+    {
+        const float *qp = nullptr;
+        if (rlive) {
+            const int t = pc.q0 + rown / a.gqa, h = pc.hk * a.gqa + rown % a.gqa;
+            prow = a.pos[t];
+            qp = a.q + ((int64_t) t * a.H + h) * D + 8 * g;
+        }
+        float qv[NK][8];
+#pragma unroll
+        for (int j = 0; j < NK; j++) {
+            float4 u = make_float4(0.f, 0.f, 0.f, 0.f), v = u;
+            if (rlive && 32 * j + 8 * g < D) {
+                u = *(const float4 *) (qp + 32 * j);
+                v = *(const float4 *) (qp + 32 * j + 4);
+            }
+            qv[j][0] = u.x; qv[j][1] = u.y; qv[j][2] = u.z; qv[j][3] = u.w;
+            qv[j][4] = v.x; qv[j][5] = v.y; qv[j][6] = v.z; qv[j][7] = v.w;
+        }
+        if constexpr (KF16) {
+            // scale the row to a largest |q| in [2^14, 2^15): the three f16
+            // terms then hold every element down to 2^-38 of the largest
+            float mx = 0.f;
+#pragma unroll
+            for (int j = 0; j < NK; j++)
+#pragma unroll
+                for (int e = 0; e < 8; e++) mx = fmaxf(mx, fabsf(qv[j][e]));
+            mx = fmaxf(mx, __shfl_xor(mx, 16));
+            mx = fmaxf(mx, __shfl_xor(mx, 32));
+            const int ex = mx > 0.f && mx < INFINITY ? max(__builtin_amdgcn_frexp_expf(mx), -100) : 15;
+            const float up = __uint_as_float((uint32_t) (127 + 15 - ex) << 23);
+            cs *= __uint_as_float((uint32_t) (127 - 15 + ex) << 23);
+#pragma unroll
+            for (int j = 0; j < NK; j++)
+#pragma unroll
+                for (int e = 0; e < 8; e++) {
+                    _Float16 h, m, l;
+                    gm_split3(qv[j][e] * up, h, m, l);
+                    q3[j][0][e] = h;
+                    q3[j][1][e] = m;
+                    q3[j][2][e] = l;
+                }
+        } else {
+#pragma unroll
+            for (int j = 0; j < NK; j++)
+#pragma unroll
+                for (int e = 0; e < 8; e++) qf[j][e] = qv[j][e];
+        }
+    }
+
+    // ---- loads: a block holds a whole number of 16-cell steps (the host
+    // checks it), so a step's rows are consecutive: its base is scalar work
+    // and a lane's offset from it one 24-bit multiply-add ----
+    const int last = pc.ce - 1;
+    typedef const __attribute__((address_space(4))) int32_t *bt_ptr;   // the table is not written during the launch
+    const bt_ptr bt = (bt_ptr) (uintptr_t) (a.bt + (int64_t) pc.s * a.max_blocks);
+    struct Step {
+        uint32_t row;   // pool row of the step's first cell
+        uint32_t lim;   // last readable cell of the step
+    };
+    struct StepId {
+        int c0, off;
+        int32_t id;
+    };
+    // table entry of the step at cell c (past the range: the last one again)
+    auto step_id = [&](int c) {
+        StepId e;
+        e.c0 = (int) min((uint32_t) c, (uint32_t) (last & ~15));
+        int b = p.bs_log2 >= 0 ? e.c0 >> p.bs_log2 : e.c0 / p.block_size;
+        if (b >= a.max_blocks) {
+            if (a.err && lane == 0) atomicOr(a.err, 2);
+            b = a.max_blocks - 1;
+        }
+        e.off = e.c0 - b * p.block_size;
+        if (e.off >= p.block_size) e.off = 0;
+        e.id = bt[__builtin_amdgcn_readfirstlane(b)];
+        return e;
+    };
+    auto step_of = [&](const StepId &e) {
+        int32_t id = e.id;
+        if ((uint32_t) id >= (uint32_t) a.num_blocks) {
+            if (a.err && lane == 0) atomicOr(a.err, 2);
+            id = 0;
+        }
+        // (the branches around the flags hide that these are wave-uniform)
+        id = __builtin_amdgcn_readfirstlane(id);
+        return Step{(uint32_t) id * (uint32_t) p.block_size + (uint32_t) __builtin_amdgcn_readfirstlane(e.off),
+                    (uint32_t) (last - e.c0)};
+    };
+
+    GmK<KT> kr[NT][NK];
+    GmV<VT> vr[CV][NV];
+    constexpr int KE = KT == 0 ? 4 : 2, VE = VT == 0 ? 4 : 2;   // bytes per element (F32, F16)
+    // lane offsets inside a row: K dims 8g of chunk 0 and of the last chunk
+    // (lanes past D reread its last 8 dims, and their K is taken as zero)
+    const int kd_last = min(32 * (NK - 1) + 8 * g, D - 8);
+    const uint32_t k_lane = KT == 8 ? pc.hk * (D / 32) * 34 + 2 + 8 * g : (pc.hk * D + 8 * g) * KE;
+    const uint32_t k_last = KT == 8 ? 0 : (pc.hk * D + kd_last) * KE;
+    // V dims 4n of block 0 and of the last block (columns past Dv are never stored)
+    const int vd_last = min(64 * (NV - 1) + 4 * n, Dv - 4);
+    const uint32_t v_head = VT == 8 ? pc.hk * (Dv / 32) * 34 : pc.hk * Dv * VE;
+    const uint32_t v_lane = VT == 8 ? v_head + 34 * (n >> 3) : v_head + 4 * n * VE;
+    const uint32_t v_last = VT == 8 ? v_head + 34 * (vd_last >> 5) : v_head + vd_last * VE;
+    auto load_k = [&](const Step (&st)[NT]) {
+#pragma unroll
+        for (int t = 0; t < NT; t++) {
+            const char *base = a.k_pool + pool_off(st[t].row, a.k_row);
+            const uint32_t c = __umul24(min((uint32_t) n, st[t].lim), (uint32_t) a.k_row);
+#pragma unroll
+            for (int j = 0; j < NK; j++) {
+                if (j >= JOPT && 32 * j >= D) continue;   // wave-uniform
+                if constexpr (KT == 8) {
+                    const u32x2_a2 v = gm_ld<u32x2_a2>(base, c + k_lane + 34 * j);
+                    kr[t][j].x = v.x;
+                    kr[t][j].y = v.y;
+                    kr[t][j].d = gm_ld<uint16_t>(base, c + (k_lane - 2 - 8 * g) + 34 * j);
+                } else {
+                    const bool edge = j == NK - 1 && JOPT == NK;
+                    const uint32_t off = edge ? c + k_last : c + k_lane + 32 * j * KE;
+                    if constexpr (JOPT < NK) {   // wide kernels: any chunk may be the last
+                        const uint32_t o2 = j >= JOPT ? c + (pc.hk * D + min(32 * j + 8 * g, D - 8)) * KE : off;
+                        kr[t][j].a = gm_ld<u32x4>(base, o2);
+                        if constexpr (KT == 0) kr[t][j].b = gm_ld<u32x4>(base, o2 + 16);
+                    } else {
+                        kr[t][j].a = gm_ld<u32x4>(base, off);
+                        if constexpr (KT == 0) kr[t][j].b = gm_ld<u32x4>(base, off + 16);
+                    }
+                }
+            }
+        }
+    };
+    auto load_v = [&](const Step (&st)[NT]) {
+#pragma unroll
+        for (int t = 0; t < NT; t++) {
+            const char *base = a.v_pool + pool_off(st[t].row, p.v_row);
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const uint32_t c = __umul24(min((uint32_t) (4 * g + i), st[t].lim), (uint32_t) p.v_row);
+#pragma unroll
+                for (int b = 0; b < NV; b++) {
+                    GmV<VT> &v = vr[4 * t + i][b];
+                    if (b >= BOPT && 64 * b >= Dv) continue;   // wave-uniform
+                    if constexpr (VT == 8) {
+                        const int vd = min(64 * b + 4 * n, Dv - 4);
+                        const uint32_t off = b == NV - 1 ? c + v_last
+                                             : BOPT < NV ? c + v_head + 34 * (vd >> 5) : c + v_lane + 68 * b;
+                        v.d = gm_ld<uint16_t>(base, off);
+                        v.x = gm_ld<u32_a2>(base, off + 2 + ((4 * n) & 31)).x;
+                    } else {
+                        const uint32_t off = b == NV - 1 ? c + v_last
+                                             : BOPT < NV ? c + v_head + min(64 * b + 4 * n, Dv - 4) * VE
+                                                         : c + v_lane + 64 * b * VE;
+                        if constexpr (VT == 0) v.a = gm_ld<u32x4>(base, off);
+                        else v.a = gm_ld<u32x2>(base, off);
+                    }
+                }
+            }
+        }
+    };
+
+    // m_ref: the row's reference in log2 units, 7 below the largest score it
+    // was last moved to, so that P lies in [0, 2^15] (the range in which two
+    // f16 terms hold 22 bits of every P down to 2^-32 of the largest)
+    float m_ref = -INFINITY, m_sub = 0.f, l_run = 0.f;   // m_sub: m_ref, or 0 while no cell was visible
+    f32x4 o[4 * NV];
+#pragma unroll
+    for (int i = 0; i < 4 * NV; i++) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    if (pc.cb < pc.ce) {
+        Step st[NT];
+        StepId nxt[NT];
+#pragma unroll
+        for (int t = 0; t < NT; t++) st[t] = step_of(step_id(pc.cb + 16 * t));
+#pragma unroll
+        for (int t = 0; t < NT; t++) nxt[t] = step_id(pc.cb + TC + 16 * t);
+        load_k(st);
+        load_v(st);
+        for (int tile = pc.cb; tile < pc.ce; tile += TC) {
+            const bool has_next = tile + TC < pc.ce;
+            // S^T = K Q^T: lane (n, g) gets cells 16t + 4g + i of row n
+            f32x4 sacc[NT];
+#pragma unroll
+            for (int t = 0; t < NT; t++) sacc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int j = 0; j < NK; j++) {
+                if (j >= JOPT && 32 * j >= D) continue;   // wave-uniform
+                if constexpr (KT != 8) {
+                    if (j == NK - 1 || j >= JOPT) {   // q is zero past D: K must be finite there
+                        const bool in = 32 * j + 8 * g < D;
+#pragma unroll
+                        for (int t = 0; t < NT; t++)
+#pragma unroll
+                            for (int i = 0; i < 4; i++) {
+                                kr[t][j].a[i] = in ? kr[t][j].a[i] : 0u;
+                                if constexpr (KT == 0) kr[t][j].b[i] = in ? kr[t][j].b[i] : 0u;
+                            }
+                    }
+                }
+                if constexpr (KF16) {
+#pragma unroll
+                    for (int u = 2; u >= 0; u--)
+#pragma unroll
+                        for (int t = 0; t < NT; t++)
+                            sacc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, kr[t][j].a),
+                                                                             q3[j][u], sacc[t], 0, 0, 0);
+                } else {
+                    // 16 dims to a chain: short chains round less, and two of
+                    // them run side by side
+                    f32x4 part[2][NT];
+#pragma unroll
+                    for (int t = 0; t < NT; t++) part[0][t] = part[1][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int e = 0; e < 8; e++)
+#pragma unroll
+                        for (int t = 0; t < NT; t++)
+                            part[e & 1][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(gm_k_f32<KT>(kr[t][j], e), qf[j][e],
+                                                                                  part[e & 1][t], 0, 0, 0);
+#pragma unroll
+                    for (int t = 0; t < NT; t++) sacc[t] += part[0][t] + part[1][t];
+                }
+            }
+            if (has_next) {
+#pragma unroll
+                for (int t = 0; t < NT; t++) {
+                    st[t] = step_of(nxt[t]);
+                    nxt[t] = step_id(tile + 2 * TC + 16 * t);
+                }
+                load_k(st);
+            }
+
+            // online softmax, exp2 domain; P in registers
+            float x[CV];
+#pragma unroll
+            for (int t = 0; t < NT; t++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) x[4 * t + i] = sacc[t][i] * cs;
+            if (a.softcap > 0.f) {
+#pragma unroll
+                for (int e = 0; e < CV; e++) x[e] = a.softcap * tanhf(x[e] / a.softcap) * kLog2e;
+            }
+            const bool full = tile + TC <= pc.ce && (!a.causal || tile + TC - 1 <= pc.pmin) &&
+                              (a.n_swa <= 0 || pc.pmax - tile < a.n_swa);
+            if (!full) {
+                const CellWindow cw = cell_window(tile, TC, pc.ce, prow, a.causal, a.n_swa);
+#pragma unroll
+                for (int e = 0; e < CV; e++) x[e] = cell_visible(cw, 16 * (e >> 2) + 4 * g + (e & 3)) ? x[e] : -INFINITY;
+            }
+            float mx = x[0];
+#pragma unroll
+            for (int e = 1; e < CV; e++) mx = fmaxf(mx, x[e]);
+            if (__builtin_amdgcn_ballot_w64(mx > m_ref + 15.f)) {   // some row's reference moves
+                mx = wave_max(mx);
+                const float mn = mx > m_ref + 15.f ? mx - 7.f : m_ref;
+                const float alpha = mn == m_ref ? 1.f : __builtin_amdgcn_exp2f(m_ref - mn);
+                m_ref = mn;
+                m_sub = mn == -INFINITY ? 0.f : mn;
+                l_run *= alpha;
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const float al = __shfl(alpha, 4 * g + i);   // of O row 4g + i
+#pragma unroll
+                    for (int b = 0; b < 4 * NV; b++) o[b][i] *= al;
+                }
+            }
+            float pv[CV];
+#pragma unroll
+            for (int e = 0; e < CV; e++) {
+                pv[e] = __builtin_amdgcn_exp2f(x[e] - m_sub);
+                l_run += pv[e];
+            }
+
+            // O += P V
+            if constexpr (VF16) {
+                u32x4 ph, pl;
+#pragma unroll
+                for (int w = 0; w < 4; w++) {
+                    const float p0 = pv[2 * w], p1 = pv[2 * w + 1];
+                    const auto hh = __builtin_amdgcn_cvt_pkrtz(p0, p1);
+                    float h0 = (float) hh[0], h1 = (float) hh[1];
+                    asm volatile("" : "+v"(h0), "+v"(h1));
+                    float r0 = p0 - h0, r1 = p1 - h1;
+                    asm volatile("" : "+v"(r0), "+v"(r1));
+                    ph[w] = __builtin_bit_cast(uint32_t, hh);
+                    pl[w] = pack_f16x2(r0, r1);
+                }
+#pragma unroll
+                for (int b = 0; b < NV; b++) {
+                    if (b >= BOPT && 64 * b >= Dv) continue;   // wave-uniform
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        u32x4 vb;
+                        const uint32_t sel = (e & 1) ? 0x07060302u : 0x05040100u;
+#pragma unroll
+                        for (int w = 0; w < 4; w++)
+                            vb[w] = __builtin_amdgcn_perm(vr[2 * w + 1][b].a[e >> 1], vr[2 * w][b].a[e >> 1], sel);
+                        f32x4 &acc = o[4 * b + e];
+                        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, pl),
+                                                                     __builtin_bit_cast(f16x8, vb), acc, 0, 0, 0);
+                        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, ph),
+                                                                     __builtin_bit_cast(f16x8, vb), acc, 0, 0, 0);
+                    }
+                }
+            } else {
+#pragma unroll
+                for (int b = 0; b < NV; b++) {   // the tile's cells, then one add
+                    if (b >= BOPT && 64 * b >= Dv) continue;   // wave-uniform
+                    f32x4 part[4];
+#pragma unroll
+                    for (int e = 0; e < 4; e++) part[e] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int c = 0; c < CV; c++)
+#pragma unroll
+                        for (int e = 0; e < 4; e++)
+                            part[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(pv[c], gm_v_f32<VT>(vr[c][b], e), part[e],
+                                                                           0, 0, 0);
+#pragma unroll
+                    for (int e = 0; e < 4; e++) o[4 * b + e] += part[e];
+                }
+            }
+            if (has_next) load_v(st);
+        }
+    }
+
+    // ---- output: lane (n, g) holds rows 4g + i, dims 64b + 4n + e ----
+    float l = l_run;
+    l += __shfl_xor(l, 16);
+    l += __shfl_xor(l, 32);
+    // (an empty split range has only its (m, l) = (-inf, 0): the merge skips its O)
+    const bool no_o = pc.mode == 2 && pc.cb >= pc.ce;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const float lr = __shfl(l, 4 * g + i);
+        const int r = pc.row0 + 4 * g + i;
+        if (r >= pc.M || no_o) continue;
+        const int64_t orow = (int64_t) (pc.q0 + r / a.gqa) * a.H + pc.hk * a.gqa + r % a.gqa;
+        float *op;
+        float f = 1.f;
+        if (pc.mode == 0) {
+            op = a.out + orow * Dv;
+            f = lr > 0.f ? 1.f / lr : 0.f;
+        } else if (pc.mode == 1) {
+            op = rec_o(a, pc.rec, 0, r - pc.row0, Dv);
+        } else {
+            op = p.split_o + (orow * p.n_split + pc.rec) * Dv;
+        }
+#pragma unroll
+        for (int b = 0; b < NV; b++) {
+            const int d = 64 * b + 4 * n;
+            if (d < Dv)
+                *(float4 *) (op + d) = make_float4(o[4 * b][i] * f, o[4 * b + 1][i] * f, o[4 * b + 2][i] * f,
+                                                   o[4 * b + 3][i] * f);
+        }
+    }
+    if (pc.mode != 0 && g == 0 && rlive) {
+        float *ml;
+        if (pc.mode == 1) {
+            ml = rec_ml(a, pc.rec, 0, n);
+        } else {
+            const int64_t orow = (int64_t) (pc.q0 + rown / a.gqa) * a.H + pc.hk * a.gqa + rown % a.gqa;
+            ml = p.split_ml + 2 * (orow * p.n_split + pc.rec);
+        }
+        *(float2 *) ml = make_float2(m_ref, l);
+    }
+}
+
+// The pieces of a stream-K worker, one next() at a time (the line and its
+// cuts: pa_common.h; a loop around one gm_piece, so that the kernel holds one
+// copy of it).
+struct GmPieceIter {
+    int start, end, base, incl, nt, per;
+    __device__ __forceinline__ void init(const AttnParams &a, int worker) {
+        const int lane = threadIdx.x & 63;
+        const SeqWindow w0 = seq_window(a, lane);
+        nt = w0.nt;
+        int total = wave_sum_i(nt);
+        bool over = w0.nq > a.max_q;
+        for (int b = 64; b < a.S; b += 64) {
+            const SeqWindow wb = seq_window(a, b + lane);
+            total += wave_sum_i(wb.nt);
+            over |= wb.nq > a.max_q;
+        }
+        if (worker == 0 && __builtin_amdgcn_ballot_w64(over) && lane == 0 && a.err) atomicOr(a.err, 4);
+        total = __builtin_amdgcn_readfirstlane(total) * a.Hkv;
+        per = max(kMinPieceTiles, (total + a.sk_workers - 1) / a.sk_workers);
+        start = worker * per;
+        end = min(total, start + per);
+        base = 0;
+        incl = wave_incl_scan(nt * a.Hkv);
+    }
+    __device__ __forceinline__ bool next(const AttnParams &a, int worker, GmPiece &pc) {
+        if (start >= end) return false;
+        const int lane = threadIdx.x & 63;
+        uint64_t hit = __builtin_amdgcn_ballot_w64(incl > start);
+        while (!hit) {
+            const int carry = __shfl(incl, 63);
+            base += 64;
+            nt = seq_window(a, base + lane).nt;
+            incl = carry + wave_incl_scan(nt * a.Hkv);
+            hit = __builtin_amdgcn_ballot_w64(incl > start);
+        }
+        const int ls = __builtin_ctzll(hit);
+        const int s = base + ls;
+        const SeqWindow w = seq_window(a, s);
+        const int excl = __builtin_amdgcn_readfirstlane(__shfl(incl, ls)) - w.nt * a.Hkv;
+        const int off = start - excl;
+        pc.s = s;
+        pc.hk = off / w.nt;
+        const int t0 = off % w.nt;
+        const int t1 = min(w.nt, t0 + (end - start));
+        const int seg_start = excl + pc.hk * w.nt;
+        const int seg = s * a.Hkv + pc.hk;
+        const int pieces = (seg_start + w.nt - 1) / per - seg_start / per + 1;
+        pc.rec = worker + seg;
+        pc.mode = pieces > 1 ? 1 : 0;
+        pc.q0 = w.q0;
+        pc.M = w.nq * a.gqa;
+        pc.row0 = 0;
+        pc.pmin = w.pmin;
+        pc.pmax = w.pmax;
+        pc.cb = w.c_lo + t0 * kTile;
+        pc.ce = min(w.c_hi, w.c_lo + t1 * kTile);
+        if (t0 == 0 && lane == 0) a.seg_info[seg] = make_int2(pc.rec, pieces);
+        start = seg_start + t1;
+        return true;
+    }
+};
+
+// Row blocks (64 rows) of sequence s when it is a prefill sequence, else 0.
+__device__ __forceinline__ int gm_row_blocks(const AttnParams &a, int s, int &q0, int &nq) {
+    q0 = nq = 0;
+    if (s >= a.S) return 0;
+    q0 = min(max(a.qsl[s], 0), a.T);
+    nq = min(max(a.qsl[s + 1], q0), a.T) - q0;
+    const int64_t M = (int64_t) nq * a.gqa;
+    return M > a.decode_rows ? (int) ((M + kGmBlockRows - 1) / kGmBlockRows) : 0;
+}
+
+// The piece of this wave of a prefill workgroup: workgroup b takes row block
+// `rest / n_split` of the batch's (sequences in order, each one's last rows,
+// which see the most cells, first), kv head hk and split range rest %
+// n_split.  Consecutive workgroups go to consecutive XCDs, so with a multiple
+// of 8 kv heads every row block and range of one head runs on one XCD and
+// shares its K and V through that L2.  False when the wave has no rows.
+__device__ __forceinline__ bool gm_prefill_piece(const GenMfmaParams &p, int b, GmPiece &pc) {
+    const AttnParams &a = p.a;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    pc.hk = b % a.Hkv;
+    const int rest = b / a.Hkv;
+    const int z = rest % p.n_split;
+    const int rbl = rest / p.n_split;
+    int base = 0, q0, nq;
+    int nrb = gm_row_blocks(a, lane, q0, nq);
+    int incl = wave_incl_scan(nrb);
+    uint64_t hit;
+    while (!(hit = __builtin_amdgcn_ballot_w64(incl > rbl))) {
+        const int carry = __shfl(incl, 63);
+        base += 64;
+        if (base >= a.S) return false;
+        nrb = gm_row_blocks(a, base + lane, q0, nq);
+        incl = carry + wave_incl_scan(nrb);
+    }
+    const int ls = __builtin_ctzll(hit);
+    pc.s = base + ls;
+    pc.q0 = __builtin_amdgcn_readfirstlane(__shfl(q0, ls));
+    nq = __builtin_amdgcn_readfirstlane(__shfl(nq, ls));
+    nrb = __builtin_amdgcn_readfirstlane(__shfl(nrb, ls));
+    const int rb = nrb - 1 - (rbl - (__builtin_amdgcn_readfirstlane(__shfl(incl, ls)) - nrb));
+    // a sequence with more query tokens than the caller's max_query_len (its
+    // rows are attended all the same)
+    if (pc.hk == 0 && z == 0 && rb == 0 && threadIdx.x == 0 && nq > a.max_q && a.err) atomicOr(a.err, 4);
+    pc.M = nq * a.gqa;
+    const int R0 = rb * kGmBlockRows;
+    pc.row0 = R0 + wave * kGmRows;
+    if (pc.row0 >= pc.M) return false;
+    // positions of the block's rows (at most 64 tokens) and of the wave's
+    const int j0 = R0 / a.gqa, j1 = (min(pc.M, R0 + kGmBlockRows) - 1) / a.gqa;
+    const int w0 = pc.row0 / a.gqa, w1 = (min(pc.M, pc.row0 + kGmRows) - 1) / a.gqa;
+    int mn = INT32_MAX, mx = INT32_MIN, wmn = INT32_MAX, wmx = INT32_MIN;
+    const int j = j0 + lane;
+    if (j <= j1) {
+        const int ps = a.pos[pc.q0 + j];
+        mn = mx = ps;
+        if (j >= w0 && j <= w1) wmn = wmx = ps;
+    }
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) {
+        mn = min(mn, __shfl_xor(mn, o));
+        mx = max(mx, __shfl_xor(mx, o));
+        wmn = min(wmn, __shfl_xor(wmn, o));
+        wmx = max(wmx, __shfl_xor(wmx, o));
+    }
+    mn = __builtin_amdgcn_readfirstlane(mn);
+    mx = __builtin_amdgcn_readfirstlane(mx);
+    pc.pmin = __builtin_amdgcn_readfirstlane(wmn);
+    pc.pmax = __builtin_amdgcn_readfirstlane(wmx);
+    const int L = max(a.seq_lens[pc.s], 0);
+    const int hi = a.causal ? min(L, max(mx + 1, 0)) : L;
+    const int lo = a.n_swa > 0 ? min(max(0, mn - a.n_swa + 1) & ~(kTile - 1), hi) : 0;
+    const int nt = (hi - lo + kTile - 1) / kTile;
+    const int per = (nt + p.n_split - 1) / p.n_split;
+    pc.cb = lo + min(nt, z * per) * kTile;
+    pc.ce = min(hi, lo + min(nt, (z + 1) * per) * kTile);
+    // the part of the range this wave's own rows can see
+    if (a.causal) pc.ce = min(pc.ce, max(pc.pmax + 1, 0));
+    if (a.n_swa > 0) pc.cb = max(pc.cb, max(0, pc.pmin - a.n_swa + 1) & ~(kTile - 1));
+    pc.mode = p.n_split > 1 ? 2 : 0;
+    pc.rec = z;
+    return true;
+}
+
+template <int KT, int VT, int NK, int NV>
+__global__ __launch_bounds__(kGmWaves * 64, NK <= 4 ? 2 : 1) void pa_gen_mfma_kernel(GenMfmaParams p) {
+    const bool pre = (int) blockIdx.x >= p.n_dec_wgs;
+    const int worker = __builtin_amdgcn_readfirstlane(blockIdx.x * kGmWaves + (threadIdx.x >> 6));
+    GmPiece pc;
+    GmPieceIter it;
+    bool go;
+    if (pre) {
+        go = gm_prefill_piece(p, blockIdx.x - p.n_dec_wgs, pc);
+    } else {
+        it.init(p.a, worker);
+        go = it.next(p.a, worker, pc);
+    }
+    while (go) {
+        gm_piece<KT, VT, NK, NV>(p, pc);
+        go = !pre && it.next(p.a, worker, pc);
+    }
+}
+
+template <int KT, int VT>
+static hipError_t launch_gen_mfma_v(const GenMfmaParams &p, unsigned wgs, hipStream_t stream) {
+    const dim3 grid(wgs), block(kGmWaves * 64);
+    switch (gen_mfma_chunks(p.D, p.Dv)) {
+        case 2: hipLaunchKernelGGL((pa_gen_mfma_kernel<KT, VT, 2, 1>), grid, block, 0, stream, p); break;
+        case 3: hipLaunchKernelGGL((pa_gen_mfma_kernel<KT, VT, 3, 2>), grid, block, 0, stream, p); break;
+        case 4: hipLaunchKernelGGL((pa_gen_mfma_kernel<KT, VT, 4, 2>), grid, block, 0, stream, p); break;
+        case 8: hipLaunchKernelGGL((pa_gen_mfma_kernel<KT, VT, 8, 4>), grid, block, 0, stream, p); break;
+        default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+
+template <int KT>
+static hipError_t launch_gen_mfma_k(const GenMfmaParams &p, int type_v, unsigned wgs, hipStream_t stream) {
+    switch (type_v) {
+        case 0: return launch_gen_mfma_v<KT, 0>(p, wgs, stream);
+        case 1: return launch_gen_mfma_v<KT, 1>(p, wgs, stream);
+        case 8: return launch_gen_mfma_v<KT, 8>(p, wgs, stream);
+        default: return hipErrorInvalidValue;
+    }
+}
+
+}  // namespace iian_pa

@@ -1,0 +1,73 @@
+// pa_gen_mfma.hip - launch and merge of the matrix-core general path
+// (pa_gen_mfma.h), and its F16-K kernels (one K type per file).
+#include "pa_gen_mfma.h"
+
+#include <algorithm>
+
+namespace iian_pa {
+
+// One launch merges everything the call split.  Workgroups [0, n_seg_wgs) take
+// the decode segments: WPR = 1, a workgroup per segment and a wave per row;
+// WPR = 4, a workgroup per row, its waves sharing the row's records (chosen
+// when the call has few segments, whose records are then many).  The rest take
+// the split prefill rows, a wave each.
+template <int WPR>
+__global__ __launch_bounds__(256) void pa_gen_merge_kernel(GenMfmaParams p, int n_seg_wgs, int seg_rows) {
+    __shared__ __attribute__((aligned(16))) float comb[WPR > 1 ? 4 * 258 : 4];
+    const AttnParams &a = p.a;
+    const int wave = threadIdx.x >> 6;
+    if ((int) blockIdx.x < n_seg_wgs) {
+        const int seg = WPR > 1 ? blockIdx.x / seg_rows : blockIdx.x;
+        const int s = seg / a.Hkv, hk = seg - s * a.Hkv;
+        const int2 info = a.seg_info[seg];
+        const int q0 = min(max(a.qsl[s], 0), a.T);
+        const int nq = min(max(a.qsl[s + 1], q0), a.T) - q0;
+        if (nq <= 0 || (int64_t) nq * a.gqa > a.decode_rows || info.y <= 1) return;
+        const int M = nq * a.gqa;
+        // (WPR = 4: one row per workgroup, so its barrier is met once)
+        for (int r = WPR > 1 ? blockIdx.x % seg_rows : wave; r < M; r += WPR > 1 ? kGmRows : 4) {
+            const int64_t orow = (int64_t) (q0 + r / a.gqa) * a.H + hk * a.gqa + r % a.gqa;
+            merge_row<WPR>(rec_o(a, info.x, 0, r, p.Dv), a.rec_stride, rec_ml(a, info.x, 0, r), 2 * (int64_t) a.rec_rows,
+                           info.y, p.Dv, a.out + orow * p.Dv, comb);
+        }
+        return;
+    }
+    const int64_t row = (int64_t) (blockIdx.x - n_seg_wgs) * 4 + wave;
+    if (row >= (int64_t) a.T * a.H) return;
+    const int t = (int) (row / a.H);
+    int lo = 0, hi = a.S - 1;   // the last s with qsl[s] <= t
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (a.qsl[mid] <= t) lo = mid; else hi = mid - 1;
+    }
+    const int q0 = min(max(a.qsl[lo], 0), a.T), nq = min(max(a.qsl[lo + 1], q0), a.T) - q0;
+    // rows of a decode sequence, and of none, have no split records
+    if (t < q0 || t >= q0 + nq || (int64_t) nq * a.gqa <= a.decode_rows) return;
+    merge_row<1>(p.split_o + row * p.n_split * p.Dv, p.Dv, p.split_ml + 2 * row * p.n_split, 2, p.n_split, p.Dv,
+                 a.out + row * p.Dv, comb);
+}
+
+hipError_t launch_gen_mfma(const GenMfmaParams &p, int type_k, int type_v, int64_t n_prefill_wgs, hipStream_t stream) {
+    const int64_t wgs = p.n_dec_wgs + n_prefill_wgs;
+    const int64_t seg = p.n_dec_wgs ? (int64_t) p.a.S * p.a.Hkv : 0;
+    // few segments: their records are many (on average more than 16 each)
+    const bool wide = seg * 16 <= p.a.sk_workers;
+    const int seg_rows = (int) std::min<int64_t>(kGmRows, (int64_t) p.a.max_q * p.a.gqa);
+    const int64_t seg_wgs = wide ? seg * seg_rows : seg;
+    const int64_t row_wgs = n_prefill_wgs && p.n_split > 1 ? ((int64_t) p.a.T * p.a.H + 3) / 4 : 0;
+    if (wgs <= 0 || wgs > INT32_MAX || seg_wgs + row_wgs > INT32_MAX) return hipErrorInvalidValue;
+    hipError_t e;
+    switch (type_k) {
+        case 0: e = launch_gen_mfma_f32(p, type_v, (unsigned) wgs, stream); break;
+        case 1: e = launch_gen_mfma_k<1>(p, type_v, (unsigned) wgs, stream); break;
+        case 8: e = launch_gen_mfma_q8(p, type_v, (unsigned) wgs, stream); break;
+        default: return hipErrorInvalidValue;
+    }
+    if (e != hipSuccess || seg_wgs + row_wgs == 0) return e;
+    const dim3 grid((unsigned) (seg_wgs + row_wgs));
+    if (wide) hipLaunchKernelGGL(pa_gen_merge_kernel<4>, grid, dim3(256), 0, stream, p, (int) seg_wgs, seg_rows);
+    else hipLaunchKernelGGL(pa_gen_merge_kernel<1>, grid, dim3(256), 0, stream, p, (int) seg_wgs, seg_rows);
+    return hipGetLastError();
+}
+
+}  // namespace iian_pa

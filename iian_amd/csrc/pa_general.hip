@@ -1,8 +1,9 @@
 // pa_general.hip - paged attention for every pool-type and head-size combination
-// the MFMA kernels are not built for: F32 pools, mixed K/V types (F32, F16,
-// Q8_0 in any pairing), any head size from 1 to 1024 (Phi-3's 96, 80, ...;
-// Q8_0 pools in multiples of 32), Dv != D, and block sizes that are not a
-// power of two >= 8.  Head sizes that are not multiples of 4 are staged in
+// no matrix-core kernel is built for (pa_gen_mfma.h takes head sizes in (32,
+// 256] in multiples of 8 over blocks of a multiple of 16 cells): head sizes up
+// to 32, above 256 (up to 1024) or not a multiple of 8, and other block sizes,
+// over F32, F16 and Q8_0 pools in any pairing (Q8_0 in multiples of 32),
+// Dv != D.  Head sizes that are not multiples of 4 are staged in
 // LDS rows padded with zeros to the next multiple of 4 (the reference's
 // dot and axpy loops run to any D, paged_attn.cpp:39,50), with element-wise
 // global loads and stores, since their rows are not 16-byte aligned.

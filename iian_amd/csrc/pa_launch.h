@@ -30,6 +30,19 @@ struct GenParams {
     int32_t causal, n_swa;
 };
 
+// Everything the matrix-core general kernels (pa_gen_mfma.h) read, by value.
+struct GenMfmaParams {
+    AttnParams a;               // k_row, the decode rows' records, segment table; bs_log2 and qscale unused
+    int64_t v_row;              // bytes per V pool row (a.k_row: K's)
+    float *split_o;             // prefill split records: [T*H][n_split][Dv]
+    float *split_ml;            // [T*H][n_split] of (m in log2 units, l)
+    int32_t D, Dv, block_size;
+    int32_t bs_log2;            // -1: block_size is not a power of two
+    int32_t n_dec_wgs;          // leading workgroups that hold stream-K workers (a.sk_workers / 4)
+    int32_t n_split;            // ranges per prefill row block
+    float sscale;               // of the dot product: scale (before a softcap) or scale * log2 e
+};
+
 // Waves per segment workgroup of the f16 segment decode kernel
 // (pa_decode_seg_kernel, p.seg_waves), by head size, and the most tiles per
 // wave a sliding-window call may give it.
@@ -97,6 +110,21 @@ hipError_t launch_general(const GenParams &p, int type_k, int type_v, hipStream_
 size_t general_lds_bytes(int tile_cells, int D, int Dv, int rows_per_block);
 int general_tile_cells(int D, int Dv);
 int general_rows_per_block(int max_rows);
+
+// Matrix-core general path (pa_gen_mfma.hip): any K/V types, blocks of a
+// multiple of 16 cells.  gen_mfma_chunks: the 32-dim K chunks of the kernel
+// that takes head sizes D (a multiple of 8) and Dv (of 4), or 0: D in (32, 64],
+// (64, 96], (96, 128] or (128, 256], Dv up to 64, 128, 128 or 256.
+// n_prefill_wgs: prefill workgroups (64-row blocks x kv heads x n_split), 0
+// when no sequence can have more than 16 rows.
+inline int gen_mfma_chunks(int D, int Dv) {
+    if (D % 8 || Dv % 4 || D <= 32 || D > 256) return 0;
+    const int nk = D <= 64 ? 2 : D <= 96 ? 3 : D <= 128 ? 4 : 8;
+    return Dv <= (nk == 2 ? 64 : nk == 8 ? 256 : 128) ? nk : 0;
+}
+hipError_t launch_gen_mfma(const GenMfmaParams &p, int type_k, int type_v, int64_t n_prefill_wgs, hipStream_t stream);
+hipError_t launch_gen_mfma_f32(const GenMfmaParams &p, int type_v, unsigned wgs, hipStream_t stream);
+hipError_t launch_gen_mfma_q8(const GenMfmaParams &p, int type_v, unsigned wgs, hipStream_t stream);
 
 hipError_t launch_kv_write(const float *rows, int64_t n_rows, int64_t row_elems, const int64_t *slots, void *pool,
                            int64_t n_cells, int type, int32_t *err, hipStream_t stream);
