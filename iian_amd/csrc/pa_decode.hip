@@ -32,6 +32,7 @@
 #include "pa_common.h"
 #include "pa_launch.h"
 #include "pa_decode_body.h"
+#include "pa_merge.h"
 
 namespace iian_pa {
 
@@ -46,20 +47,19 @@ __global__ __launch_bounds__(64, (D * NRT <= 128) ? 2 : 1) void pa_decode_f16_ke
     });
 }
 
-// Log-sum-exp merge of the stream-K partials: one workgroup per (sequence, kv
-// head), wave i merging rows i, i+4, ...: out = sum_j 2^(m_j - m) O_j /
-// sum_j 2^(m_j - m) l_j over the segment's pieces j, m = max_j m_j.  A separate
-// launch: the kernel boundary is what makes the partials written on other XCDs
-// visible (their L2s are not coherent within a launch, and a device-scope
-// fence per piece costs an L2 write-back).
-template <int D>
-__global__ __launch_bounds__(256) void pa_merge_kernel(AttnParams p) {
-    constexpr int DL = (D + 63) / 64;   // dims per lane (head size 96: 2 dims on lanes 0..47)
-    constexpr bool ALL = D % 64 == 0;   // every lane has dims
+// Log-sum-exp merge of the stream-K partials (merge_row, pa_merge.h).  A
+// separate launch: the kernel boundary is what makes the partials written on
+// other XCDs visible (their L2s are not coherent within a launch, and a
+// device-scope fence per piece costs an L2 write-back).
+// WPR = 1: one workgroup per (sequence, kv head or head group), wave i merging
+// rows i, i+4, ...  WPR = 4: one workgroup per row, blockIdx.z, whose 4 waves
+// share its records, for calls with few segments and so many records in each.
+template <int WPR>
+__global__ __launch_bounds__(256) void pa_merge_kernel(AttnParams p, int D) {
+    __shared__ __attribute__((aligned(16))) float comb[WPR > 1 ? 4 * 258 : 4];
     // blockIdx.y: the kv head, or the head group of head_group kv heads
     // (rows r of a group's segment: row r % M of its head r / M)
     const int s = blockIdx.x, hg = blockIdx.y;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const bool grouped = p.rec_heads > 1;
     // the segment table entry and the query range in one round trip: the
     // exit test below reads all three without short-circuit, so the entry is
@@ -71,81 +71,31 @@ __global__ __launch_bounds__(256) void pa_merge_kernel(AttnParams p) {
     const int M = nq * p.gqa;
     if ((nq <= 0) | (M > p.decode_rows) | (info.y <= 1)) return;
     const int hr = grouped ? hg : 0;
-    const int rec0 = info.x, ns = info.y;
-    const bool dl_live = ALL || lane * DL < D;
-    for (int r = wave; r < M * p.head_group; r += 4) {
+    const int rows = M * p.head_group;
+    for (int r = WPR > 1 ? (int) blockIdx.z : (int) (threadIdx.x >> 6); r < rows; r += WPR > 1 ? rows : 4) {
         const int hl = r / M, rh = r - hl * M;
         const int t = q0 + rh / p.gqa, h = (hg * p.head_group + hl) * p.gqa + rh % p.gqa;
-        // the first 8 partial O rows are loaded together with the (m, l) of
-        // pieces lane, lane + 64, ...; the first (m, l) chunk stays in registers
-        float v0[8][DL];
-#pragma unroll
-        for (int u = 0; u < 8; u++) {
-            const float *op = rec_o(p, rec0 + min(u, ns - 1), hr, r, D) + lane * DL;
-#pragma unroll
-            for (int i = 0; i < DL; i++) v0[u][i] = dl_live ? op[i] : 0.f;
-        }
-        float2 ml0 = make_float2(-INFINITY, 0.f);
-        if (lane < ns) ml0 = *(const float2 *) rec_ml(p, rec0 + lane, hr, r);
-        float mx = ml0.x;
-        for (int j = lane + 64; j < ns; j += 64) mx = fmaxf(mx, rec_ml(p, rec0 + j, hr, r)[0]);
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
-        float acc[DL];
-#pragma unroll
-        for (int i = 0; i < DL; i++) acc[i] = 0.f;
-        float lpart = 0.f;
-        if (mx != -INFINITY) {
-            for (int c0 = 0; c0 < ns; c0 += 64) {
-                const int nc = min(64, ns - c0);
-                const float2 ml = c0 == 0 ? ml0 : (lane < nc ? *(const float2 *) rec_ml(p, rec0 + c0 + lane, hr, r)
-                                                             : make_float2(-INFINITY, 0.f));
-                const float wl = lane < nc ? __builtin_amdgcn_exp2f(ml.x - mx) : 0.f;   // 0 for an empty piece
-                lpart += wl * ml.y;
-                // partial O rows in batches of 8, all loads of a batch issued before use
-                for (int j0 = 0; j0 < nc; j0 += 8) {
-                    float v[8][DL];
-                    if (c0 == 0 && j0 == 0) {
-#pragma unroll
-                        for (int u = 0; u < 8; u++)
-#pragma unroll
-                            for (int i = 0; i < DL; i++) v[u][i] = v0[u][i];
-                    } else {
-#pragma unroll
-                        for (int u = 0; u < 8; u++) {
-                            const float *op = rec_o(p, rec0 + c0 + min(j0 + u, nc - 1), hr, r, D) + lane * DL;
-#pragma unroll
-                            for (int i = 0; i < DL; i++) v[u][i] = dl_live ? op[i] : 0.f;
-                        }
-                    }
-#pragma unroll
-                    for (int u = 0; u < 8; u++) {
-                        const float wgt = j0 + u < nc ? __shfl(wl, min(j0 + u, 63)) : 0.f;
-#pragma unroll
-                        for (int i = 0; i < DL; i++) acc[i] += wgt * v[u][i];
-                    }
-                }
-            }
-        }
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) lpart += __shfl_xor(lpart, o);
-        const float inv = lpart > 0.f ? 1.f / lpart : 0.f;
-        float *out = p.out + ((int64_t) t * p.H + h) * D + lane * DL;
-        if (dl_live)
-#pragma unroll
-            for (int i = 0; i < DL; i++) out[i] = acc[i] * inv;
+        merge_row<WPR>(rec_o(p, info.x, hr, r, D), p.rec_stride, rec_ml(p, info.x, hr, r),
+                       2 * (int64_t) p.rec_heads * p.rec_rows, info.y, D, p.out + ((int64_t) t * p.H + h) * D, comb);
     }
 }
 
+// A workgroup per row where the call has at most one segment per 8 stream-K
+// workers, and so 8 records or more per segment on average: merge_row's batch
+// covers 8 records of a row with one wave, 32 with four.  Measured at H32/Hkv8/
+// D128 f16, whole calls (before: one wave per row, 8 records a batch, at any
+// count): 2 sequences of 26K-30K cells 57.8 -> 53.4 us (the merge 10.2 -> 5.8),
+// 4 of 512-8192 cells 22.7 -> 19.2, 16 37.9 -> 37.6 (38.5 with a wave per row),
+// 24 and more unchanged; 4 Q8_0 spec-verify sequences of 4K 40.6 -> 28.9 us.
 hipError_t launch_merge(const AttnParams &p, int head_dim, hipStream_t stream) {
-    const dim3 grid(p.S, p.Hkv / p.head_group);
-    switch (head_dim) {
-        case 64: hipLaunchKernelGGL((pa_merge_kernel<64>), grid, dim3(256), 0, stream, p); break;
-        case 96: hipLaunchKernelGGL((pa_merge_kernel<96>), grid, dim3(256), 0, stream, p); break;
-        case 128: hipLaunchKernelGGL((pa_merge_kernel<128>), grid, dim3(256), 0, stream, p); break;
-        case 256: hipLaunchKernelGGL((pa_merge_kernel<256>), grid, dim3(256), 0, stream, p); break;
-        default: return hipErrorInvalidValue;
-    }
+    if (head_dim % 4 || head_dim > 256) return hipErrorInvalidValue;
+    const int groups = p.Hkv / p.head_group;
+    const int64_t segs = p.rec_heads > 1 ? p.S : (int64_t) p.S * groups;
+    const dim3 block(256);
+    if (segs * 8 <= p.sk_workers)
+        hipLaunchKernelGGL(pa_merge_kernel<4>, dim3(p.S, groups, p.rec_rows), block, 0, stream, p, head_dim);
+    else
+        hipLaunchKernelGGL(pa_merge_kernel<1>, dim3(p.S, groups), block, 0, stream, p, head_dim);
     return hipGetLastError();
 }
 

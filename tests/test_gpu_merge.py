@@ -1,0 +1,49 @@
+"""The merge launch of the decode kernels on both sides of its rule (a
+workgroup per row up to one segment per 8 stream-K workers, a wave per row
+above), for every head size and record layout: one head, head pairs at head
+size 96, grouped Q8_0 records, two 16-row tiles.  Bar: the 2e-3 of the f16
+kernels (P is rounded to f16 there), as the other decode tests."""
+import zlib
+
+import numpy as np
+import pytest
+import torch
+
+from helpers import Q8_0, make_case, row_rel_err
+from test_gpu_parity import TOL, banner, gpu_attention, oracle_attention
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def pa():
+    assert torch.cuda.is_available(), "GPU tests need an MI355X"
+    import iian_amd
+    iian_amd._lib.load()
+    return iian_amd
+
+
+CASES = {
+    "d64_one_sequence": (14, 2, 64, [6000], [1], {}),
+    "d96_pairs": (32, 32, 96, [5000], [1], {}),
+    "d96_verify": (8, 2, 96, [5000, 40], [5, 1], {}),
+    "d128_verify5_two_tiles": (32, 8, 128, [7000, 2100], [5, 5], {}),
+    "d128_few_records": (32, 8, 128, [90, 70], [1, 1], {}),
+    "d128_24_sequences": (8, 8, 128, [1000 + 40 * s for s in range(24)], [1] * 24, {}),   # 192 segments, 1536 workers
+    "d128_25_sequences": (8, 8, 128, [1000 + 40 * s for s in range(25)], [1] * 25, {}),
+    "d256_one_sequence": (16, 8, 256, [9000], [1], {}),
+    "q8_d64_one_sequence": (14, 2, 64, [6000], [1], {"k_type": Q8_0}),
+    "q8_d128_verify5": (32, 8, 128, [7000, 300], [5, 5], {"k_type": Q8_0}),
+    "q8_d128_33_sequences": (8, 8, 128, [600 + 10 * s for s in range(33)], [1] * 33, {"k_type": Q8_0}),
+}
+
+
+@pytest.mark.parametrize("name", sorted(CASES))
+def test_merge_matches_oracle(pa, oracle, name):
+    H, Hkv, D, lens, nq, kw = CASES[name]
+    banner(f"merge {name}")
+    c = make_case(np.random.default_rng(zlib.crc32(name.encode())), H, Hkv, D, lens, nq,
+                  quantize=oracle.quantize_q8_0, **kw)
+    got = gpu_attention(pa, c)
+    e = row_rel_err(got, oracle_attention(oracle, c))
+    assert np.isfinite(got).all() and e.max() <= TOL, (name, e.max())
