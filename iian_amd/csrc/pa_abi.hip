@@ -52,6 +52,10 @@ constexpr int kGenDecodeWavesPerCu = 8;
 constexpr int kGenMixedDecodeWavesPerCu = 4;
 constexpr int kGenDecodeWavesPerCuWide = 4;
 constexpr int kGenPrefillWgsPerCu = 2;
+// Split prefill row blocks (prefill_splits): the rounds of D = 256 workgroups
+// a launch of about one round is cut into, and the most ranges per row block.
+constexpr int kSplitRoundsD256 = 3;
+constexpr int kMaxSplits = 16;
 constexpr int kQ8DecodeWavesPerCu = 8;
 constexpr int kMaxWavesPerCu = kQ8DecodeWavesPerCu;
 constexpr int kDefaultCus = 256;   // an MI355X, when the device cannot be queried
@@ -263,6 +267,43 @@ bool gen_mfma_path(int head_dim, int head_dim_v, int32_t block_size, int32_t max
     return gen_mfma_chunks(head_dim, head_dim_v) && block_size % 16 == 0 &&
            (int64_t) num_blocks * block_size <= ((int64_t) 1 << 32) && k_row < (1 << 24) && v_row < (1 << 24) &&
            (int64_t) max_blocks * block_size <= INT32_MAX / 2 && rows <= (1 << 30);
+}
+
+// Ranges a prefill row block is cut into at most (split_range, pa_common.h),
+// with `room` bytes of workspace left for their records.  A launch whose row
+// blocks take at most half of the device's workgroup slots is cut to fill
+// them; more ranges than that only add starts and records (one 256-token chunk
+// over 10K cells at H16/Hkv8/D256: 481 us uncut, 87 with one workgroup per CU,
+// 136 with two rounds of them).  D <= 128 kernels hold two workgroups per CU,
+// less the decode workers of a mixed launch (4 chunks' worth of slots taken
+// from 2 chunks of 512 beside 32 decodes cost 365 -> 390 us).  At D = 256,
+// where a workgroup has its CU alone and the longest one decides a launch of
+// about one round, such a launch is planned for 3 rounds and the kernel cuts it
+// when the batch is uneven (8 chunks of 256 over 4K-16K cells 784 -> 614 us; 2
+// rounds 0-3% either way on other lengths).  Measured besides, whole calls: 8 Q8_0
+// kv heads, chunks of 504 and 361 tokens over 1.6K-2.7K cells beside 24
+// decodes, two layers, 394 -> 301 us; one chunk of 250 tokens over 8.5K cells at
+// H32/Hkv8/D128 231 -> 96 us; full launches unchanged.
+int prefill_splits(AttnParams &p, int head_dim, bool mixed_one_launch, int64_t max_rows, int32_t block_size,
+                   int cus, size_t room) {
+    const int64_t rows = (int64_t) p.T * p.gqa;
+    const int64_t blocks = std::max<int64_t>(1, rows / kPrefillBlockRows) * p.Hkv;
+    // slots: the workgroups of this kernel the device holds at once
+    const int64_t slots = head_dim == 256 ? cus : 2 * cus - (mixed_one_launch ? p.sk_workers / 4 : 0);
+    int64_t ns = slots / blocks;
+    p.split_balance = 0;
+    if (head_dim == 256 && 2 * blocks > slots && p.n_swa <= 0 && p.S <= 64) {
+        ns = kSplitRoundsD256 * slots / blocks;
+        p.split_balance = 1;   // the kernel looks whether the batch is uneven
+    }
+    int64_t cells = (int64_t) p.max_blocks * block_size;
+    if (p.n_swa > 0) cells = std::min<int64_t>(cells, (int64_t) p.n_swa + max_rows / p.gqa);
+    ns = std::min<int64_t>({ns, cells / kSplitMinCells, kMaxSplits});
+    // records: n_split - 1 O rows and n_split (m, l) per output row
+    const size_t out_rows = (size_t) p.T * p.H;
+    while (ns > 1 && align256(out_rows * (ns - 1) * head_dim * sizeof(float)) + out_rows * ns * 2 * sizeof(float) > room)
+        ns--;
+    return (int) std::max<int64_t>(ns, 1);
 }
 
 // Any head size the general kernel stages (1 .. 1024; the reference's op
@@ -641,8 +682,24 @@ int run_attention(hipStream_t st, const float *q, const void *k_pool, const void
         p.sk_workers = 0;
     }
     const WorkspaceLayout xl = exact_layout(p);
-    const int rc = ws_resolve(src, st, xl.total, &ws);
+    size_t need = xl.total;
+    const size_t split_at = align256(xl.total);
+    size_t split_o = 0;
+    p.n_split = 1;
+    if (!decode_only) {
+        const size_t cap = src.scratch ? kScratchBytes : wl.total;
+        p.n_split = prefill_splits(p, head_dim, mixed_one_launch, max_rows, block_size, cus,
+                                   cap - std::min(split_at, cap));
+        if (p.n_split > 1) {
+            const size_t rows = (size_t) n_tokens * n_head;
+            split_o = align256(rows * (p.n_split - 1) * head_dim_v * sizeof(float));
+            need = split_at + split_o + rows * p.n_split * 2 * sizeof(float);
+        }
+    }
+    const int rc = ws_resolve(src, st, need, &ws);
     if (rc) return rc;
+    p.split_o = (float *) (ws + split_at);
+    p.split_ml = (float *) (ws + split_at + split_o);
     p.part_o = (float *) (ws + xl.o);
     p.part_ml = (float *) (ws + xl.ml);
     p.seg_info = (int2 *) (ws + xl.seg);

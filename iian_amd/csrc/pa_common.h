@@ -59,6 +59,10 @@ struct AttnParams {
     int32_t cus_per_xcd;        // CUs per XCD: workgroups b and b + 8*cus_per_xcd of a launch share a CU
     int32_t head_group;         // kv heads per f16 decode segment: 1, or 2 (head size 96, rows per head <= 8)
     int32_t rec_rows;           // rows of a partial record per kv-head slot: decode_rows * head_group
+    int32_t n_split;            // > 1: prefill row blocks are cut into up to n_split ranges of their tiles
+    int32_t split_balance;      // cut for balance only: not when the batch is even (pa_prefill16_kernel)
+    float *split_o;             // their records past the first: [T*H][n_split - 1][D] (the first is in `out`)
+    float *split_ml;            // [T*H][n_split] of (m in log2 units, l)
 };
 
 __device__ __forceinline__ float wave_max(float v) {
@@ -229,6 +233,41 @@ __device__ __forceinline__ float *rec_o(const AttnParams &p, int rec, int hr, in
 }
 __device__ __forceinline__ float *rec_ml(const AttnParams &p, int rec, int hr, int r) {
     return p.part_ml + (((int64_t) rec * p.rec_heads + hr) * p.rec_rows + r) * 2;
+}
+
+// ---- Split prefill row blocks ----
+//
+// A launch with few prefill row blocks leaves CUs idle, or waits for the
+// longest one.  Its row blocks are then cut into equal ranges of their tiles,
+// one workgroup each, whose partial results a launch after it merges
+// (pa_split_merge_kernel): as many as kSplitMinCells cells each allow, at most
+// n_split.  A row block of up to kSplitMinCells cells is never cut, so its rows do
+// not depend on the batch or on how the launch was planned.
+constexpr int kSplitMinCells = 1024;
+
+struct SplitRange {
+    int n;        // ranges of this row block
+    int lo, hi;   // cells of range z (empty when z >= n)
+};
+// Range z of the cells [c_lo, c_hi) in whole tiles of `tile` cells.
+__device__ __forceinline__ SplitRange split_range(int c_lo, int c_hi, int z, int n_split, int tile) {
+    const int cells = max(c_hi - c_lo, 0);
+    SplitRange r;
+    r.n = min(n_split, max(1, (cells + kSplitMinCells - 1) / kSplitMinCells));
+    const int nt = (cells + tile - 1) / tile, per = (nt + r.n - 1) / r.n;
+    r.lo = min(c_hi, c_lo + z * per * tile);
+    r.hi = z < r.n ? min(c_hi, c_lo + (z + 1) * per * tile) : r.lo;
+    return r;
+}
+
+// The (m, l) of output row `orow`, range z.  Range 0 of an uncut row block
+// writes the finished row and l = -1.
+__device__ __forceinline__ float2 *split_ml_at(const AttnParams &p, int64_t orow, int z) {
+    return (float2 *) p.split_ml + orow * p.n_split + z;
+}
+// Where range z's O row goes.
+__device__ __forceinline__ float *split_o_at(const AttnParams &p, int64_t orow, int z, int dv) {
+    return z == 0 ? p.out + orow * dv : p.split_o + (orow * (p.n_split - 1) + z - 1) * dv;
 }
 
 // ---- Merge of a split segment inside the launch (mixed prefill launch) ----

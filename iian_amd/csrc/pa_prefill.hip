@@ -40,6 +40,8 @@
 #include "pa_mfma.h"
 #include "pa_decode_body.h"
 
+#include <algorithm>
+
 #ifndef IIAN_PA_PREFILL_LO8
 #define IIAN_PA_PREFILL_LO8 1
 #endif
@@ -68,7 +70,9 @@ struct PrefillOcc {
 // instead of the decode rows waiting for the prefill tail.  Split decode segments are merged inside the launch (arrive_last):
 // the decode workers finish long before the prefill workgroups, so the merge
 // costs the launch nothing, and the call is one launch.
-template <int D, int NW, int KVT, bool MIXED>
+//
+// SPLIT: row blocks cut into ranges of their tiles (split_range, pa_common.h).
+template <int D, int NW, int KVT, bool MIXED, bool SPLIT>
 __global__ __launch_bounds__(NW * 64, PrefillOcc<D>::kWavesPerSimd) void pa_prefill_kernel(AttnParams p, int n_rb,
                                                                                           int n_dec) {
     int bid = blockIdx.x;
@@ -115,10 +119,14 @@ __global__ __launch_bounds__(NW * 64, PrefillOcc<D>::kWavesPerSimd) void pa_pref
     // early ones and get the CU to themselves sooner (Qwen3-8B chunked prefill
     // 133.3-134.0 against 137.2-137.3 us; with decode rows 164.8-165.9 against
     // 173.5-173.7 us).  Per pair, so every row block is taken once.
+    // (a cut row block's ranges lie n_rb slots apart: the row blocks of one
+    // range, which read the same cells, stay together)
     const int slot = bid >> 3;
-    const int pair_x = slot / n_rb;
+    const int per_pair = SPLIT ? n_rb * p.n_split : n_rb;
+    const int pair_x = slot / per_pair;
     const int pair = (bid & 7) + 8 * pair_x;
     const int rb = (((pair_x * n_rb) / p.cus_per_xcd) & 1) ? n_rb - 1 - slot % n_rb : slot % n_rb;
+    const int z = SPLIT ? slot % per_pair / n_rb : 0;
     if (pair >= p.S * p.Hkv) return;
     const int s = pair / p.Hkv;
     const int hk = pair % p.Hkv;
@@ -134,7 +142,7 @@ __global__ __launch_bounds__(NW * 64, PrefillOcc<D>::kWavesPerSimd) void pa_pref
     const int M = nq * p.gqa;
     // more query tokens than the caller's max_query_len: rows past this
     // launch's row blocks stay unwritten, so flag it (bit 2)
-    if (rb == 0 && hk == 0 && threadIdx.x == 0 && nq > p.max_q && p.err) atomicOr(p.err, 4);
+    if (rb == 0 && z == 0 && hk == 0 && threadIdx.x == 0 && nq > p.max_q && p.err) atomicOr(p.err, 4);
     if (M <= p.decode_rows) return;
     const int R0 = rb * ROWS;
     if (R0 >= M) return;
@@ -175,6 +183,20 @@ __global__ __launch_bounds__(NW * 64, PrefillOcc<D>::kWavesPerSimd) void pa_pref
     int c_lo = 0;
     if (p.n_swa > 0) c_lo = max(0, wg_min - p.n_swa + 1);
     c_lo &= ~(kTile - 1);
+
+    SplitRange sr = {1, c_lo, c_hi};
+    if constexpr (SPLIT) {
+        sr = split_range(c_lo, c_hi, z, p.n_split, PT);
+        if (z >= sr.n) {   // no such range: an empty record, where the row block is cut
+            if (sr.n == 1) return;
+            for (int r = R0 + tid; r < min(M, R0 + ROWS); r += NW * 64)
+                *split_ml_at(p, (int64_t) (q0 + r / p.gqa) * p.H + hk * p.gqa + r % p.gqa, z) =
+                    make_float2(-INFINITY, 0.f);
+            return;
+        }
+        c_lo = sr.lo;
+        c_hi = sr.hi;
+    }
 
     // Q^T B operands of query row n (pre-scaled f16 hi/lo pairs, dims
     // 16kk + 8hh .. +7), its position and running state.  The pair carries q
@@ -609,12 +631,68 @@ __global__ __launch_bounds__(NW * 64, PrefillOcc<D>::kWavesPerSimd) void pa_pref
         const int row = Rw + rr;
         if (row < M) {
             const int t = q0 + row / p.gqa, h = hk * p.gqa + row % p.gqa;
-            const float inv = lr > 0.f ? 1.f / lr : 0.f;
-            float *op = p.out + ((int64_t) t * p.H + h) * D + n;
+            const int64_t orow = (int64_t) t * p.H + h;
+            const bool part = SPLIT && sr.n > 1;   // unnormalised, for the merge
+            const float inv = part ? 1.f : lr > 0.f ? 1.f / lr : 0.f;
+            float *op = (part ? split_o_at(p, orow, z, D) : p.out + orow * D) + n;
 #pragma unroll
             for (int m = 0; m < NO; m++) op[32 * m] = o[m][r] * inv;
+            if constexpr (SPLIT) {
+                const float mr = __shfl(m_run, rr);
+                if (n == 0) *split_ml_at(p, orow, z) = make_float2(mr, part ? lr : -1.f);
+            }
         }
     }
+}
+
+// The split row blocks' merge: out = sum_z 2^(m_z - m) O_z / sum_z 2^(m_z - m)
+// l_z over the ranges of each row of a prefill sequence, range 0's O taken from
+// `out` itself.  One round trip of (m, l) and one of the O rows; a lane holds 4
+// dims, so a row takes lpr = 16, 32 or 64 lanes and a wave 64 / lpr rows.  Rows
+// the launch did not cover (past cover_rows of a sequence) are left alone.
+__global__ __launch_bounds__(256) void pa_split_merge_kernel(AttnParams p, int D, int lpr, int cover_rows) {
+    const int lane = threadIdx.x & 63, sub = lane / lpr, d = 4 * (lane & (lpr - 1));
+    const int64_t row = ((int64_t) blockIdx.x * 4 + (threadIdx.x >> 6)) * (64 / lpr) + sub;
+    if (row >= (int64_t) p.T * p.H) return;
+    // an uncut row block wrote the finished row (looked at first: rows the
+    // launch did not cover hold anything here, and are left alone below)
+    if (split_ml_at(p, row, 0)->y < 0.f) return;
+    const int t = (int) (row / p.H), h = (int) (row - (int64_t) t * p.H);
+    int lo = 0, hi = p.S - 1;   // the last s with qsl[s] <= t
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (p.qsl[mid] <= t) lo = mid; else hi = mid - 1;
+    }
+    const int q0 = min(max(p.qsl[lo], 0), p.T), nq = min(max(p.qsl[lo + 1], q0), p.T) - q0;
+    if (t < q0 || t >= q0 + nq || nq * p.gqa <= p.decode_rows || (t - q0) * p.gqa + h % p.gqa >= cover_rows) return;
+    float mx = -INFINITY;
+    for (int z = 0; z < p.n_split; z++) mx = fmaxf(mx, split_ml_at(p, row, z)->x);
+    if (d >= D) return;
+    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+    float ls = 0.f;
+    for (int z = 0; z < p.n_split; z++) {
+        const float2 ml = *split_ml_at(p, row, z);
+        if (ml.x == -INFINITY) continue;   // no visible cell, or no such range: its O may hold anything
+        const float w = __builtin_amdgcn_exp2f(ml.x - mx);
+        const float4 v = *(const float4 *) (split_o_at(p, row, z, D) + d);
+        ls = fmaf(w, ml.y, ls);
+        acc.x = fmaf(w, v.x, acc.x);
+        acc.y = fmaf(w, v.y, acc.y);
+        acc.z = fmaf(w, v.z, acc.z);
+        acc.w = fmaf(w, v.w, acc.w);
+    }
+    const float inv = ls > 0.f ? 1.f / ls : 0.f;
+    *(float4 *) (p.out + row * D + d) = make_float4(acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv);
+}
+
+hipError_t launch_split_merge(const AttnParams &p, int head_dim, int cover_rows, hipStream_t stream) {
+    const int lpr = head_dim <= 64 ? 16 : head_dim <= 128 ? 32 : 64;
+    if (head_dim % 4 || head_dim > 256) return hipErrorInvalidValue;
+    const int64_t rows_per_wg = 4 * (64 / lpr);
+    const int64_t wgs = ((int64_t) p.T * p.H + rows_per_wg - 1) / rows_per_wg;
+    if (wgs > INT32_MAX) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(pa_split_merge_kernel, dim3((unsigned) wgs), dim3(256), 0, stream, p, head_dim, lpr, cover_rows);
+    return hipGetLastError();
 }
 
 template <int D, int NW, int KVT, bool MIXED>
@@ -622,12 +700,18 @@ static hipError_t launch_prefill_t(const AttnParams &p, int max_rows, hipStream_
     constexpr int ROWS = NW * 32;
     const int n_rb = (max_rows + ROWS - 1) / ROWS;
     const int pairs_per_xcd = (p.S * p.Hkv + 7) / 8;
-    const int64_t n_pf = 8 * (int64_t) pairs_per_xcd * n_rb;
+    static_assert(ROWS == kPrefillBlockRows, "the host plans 128-row blocks");
+    const int64_t n_pf = 8 * (int64_t) pairs_per_xcd * n_rb * std::max(1, p.n_split);
     const int64_t n_dec = MIXED ? ((p.sk_workers + NW - 1) / NW + 7) / 8 * 8 : 0;
     const int64_t nwg = n_dec + n_pf;
     if (nwg > INT32_MAX) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((pa_prefill_kernel<D, NW, KVT, MIXED>), dim3((unsigned) nwg), dim3(NW * 64), 0, stream, p, n_rb,
-                       (int) n_dec);
+    const dim3 grid((unsigned) nwg), block(NW * 64);
+    if (p.n_split > 1) {
+        hipLaunchKernelGGL((pa_prefill_kernel<D, NW, KVT, MIXED, true>), grid, block, 0, stream, p, n_rb, (int) n_dec);
+        const hipError_t e = hipGetLastError();
+        return e != hipSuccess ? e : launch_split_merge(p, D, n_rb * ROWS, stream);
+    }
+    hipLaunchKernelGGL((pa_prefill_kernel<D, NW, KVT, MIXED, false>), grid, block, 0, stream, p, n_rb, (int) n_dec);
     return hipGetLastError();
 }
 

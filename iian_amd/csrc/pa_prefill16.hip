@@ -28,6 +28,8 @@
 #include "pa_launch.h"
 #include "pa_mfma.h"
 
+#include <algorithm>
+
 namespace iian_pa {
 
 // The lo product of q in bf8 (f16 pools; pa_mfma.h): one
@@ -68,7 +70,8 @@ __device__ __forceinline__ f16x8 lds_tr_b16x8_16(const char *p0, const char *p1)
 // values in f16 plus the block scales d as f32 in LDS, applied per cell after
 // each QK^T k-step MFMA (k-step = block), so q*d enters the scores exactly;
 // V as f16(q*d), the correctly rounded dequantised value.
-template <int D, int NRT, int NW, int KVT>
+// SPLIT: row blocks cut into ranges of their tiles (split_range, pa_common.h).
+template <int D, int NRT, int NW, int KVT, bool SPLIT>
 // Waves per SIMD asked of the register allocator: four for f16 at D = 128 (two
 // 8-wave workgroups per CU in 128 VGPRs), else two up to D = 128, one at 256.
 __global__ __launch_bounds__(NW * 64, (D == 128 && KVT == 1) ? 4 : (D <= 128 ? 2 : 1)) void pa_prefill16_kernel(
@@ -93,8 +96,11 @@ __global__ __launch_bounds__(NW * 64, (D == 128 && KVT == 1) ? 4 : (D <= 128 ? 2
     // few sequences of a batch are prefill chunks) land on different XCDs.
     const int bid = blockIdx.x;
     const int slot = bid >> 3;
-    const int pair = (bid & 7) + 8 * (slot / n_rb);
-    const int rb = slot % n_rb;
+    // (a cut row block's ranges lie n_rb slots apart: the row blocks of one
+    // range, which read the same cells, stay together)
+    const int per_pair = SPLIT ? n_rb * p.n_split : n_rb;
+    const int pair = (bid & 7) + 8 * (slot / per_pair);
+    const int rb = slot % n_rb, z = SPLIT ? slot % per_pair / n_rb : 0;
     if (pair >= p.S * p.Hkv) return;
 
     // wave index in a scalar register, so that the tile-load rows derived from
@@ -111,6 +117,7 @@ __global__ __launch_bounds__(NW * 64, (D == 128 && KVT == 1) ? 4 : (D <= 128 ? 2
     // shuffles cost the window-bounded prefill 2-3%).
     const int hk = pair % p.Hkv;
     int s = pair / p.Hkv, L, q0, nq;
+    int n_split = SPLIT ? p.n_split : 1;   // ranges a row block may be cut into
     if (p.S <= 64 && p.n_swa <= 0) {
         int ll = 0, a = 0, nql = 0, key = -1;
         if (lane < p.S) {
@@ -123,6 +130,27 @@ __global__ __launch_bounds__(NW * 64, (D == 128 && KVT == 1) ? 4 : (D <= 128 ? 2
         for (int j = 0; j < p.S; j++) {
             const int kj = __builtin_amdgcn_readlane(key, j);
             rank += (kj > key || (kj == key && j < lane)) ? 1 : 0;
+        }
+        if (SPLIT && p.split_balance) {
+            // The call has about as many workgroups as CUs: uncut, it takes the
+            // longest of them, or its rounds of average ones.  Cut only when
+            // that is well above an even share of the cells (records and the
+            // pieces' starts cost an even batch 12%: 8 chunks of 256 tokens
+            // over 6000 cells each 356 against 400 us; over 4K-16K cells 784
+            // us uncut, 627 cut).
+            const float rows = key >= 0 ? (float) ((nql * p.gqa + ROWS - 1) / ROWS) : 0.f;
+            float blocks = rows, cells = rows * (float) max(key, 0), longest = (float) max(key, 0);
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) {
+                blocks += __shfl_xor(blocks, o);
+                cells += __shfl_xor(cells, o);
+                longest = fmaxf(longest, __shfl_xor(longest, o));
+            }
+            const float cus = 8.f * (float) p.cus_per_xcd, wgs = blocks * (float) p.Hkv;
+            const float share = cells * (float) p.Hkv / cus;
+            const float uncut = fmaxf(longest, ceilf(wgs / cus) * (cells / fmaxf(blocks, 1.f)));
+            if (!__builtin_amdgcn_ballot_w64(uncut > 1.2f * share)) n_split = 1;
+            if (z >= n_split) return;
         }
         const uint64_t hit = __builtin_amdgcn_ballot_w64(lane < p.S && rank == s);
         s = __builtin_amdgcn_readfirstlane(hit ? (int) __builtin_ctzll(hit) : s);
@@ -137,7 +165,7 @@ __global__ __launch_bounds__(NW * 64, (D == 128 && KVT == 1) ? 4 : (D <= 128 ? 2
     const int M = nq * p.gqa;
     // more query tokens than the caller's max_query_len: rows past this
     // launch's row blocks stay unwritten, so flag it (bit 2)
-    if (rb == 0 && hk == 0 && tid == 0 && nq > p.max_q && p.err) atomicOr(p.err, 4);
+    if (rb == 0 && z == 0 && hk == 0 && tid == 0 && nq > p.max_q && p.err) atomicOr(p.err, 4);
     if (M <= p.decode_rows) return;
     const int R0 = rb * ROWS;
     if (R0 >= M) return;
@@ -173,6 +201,20 @@ __global__ __launch_bounds__(NW * 64, (D == 128 && KVT == 1) ? 4 : (D <= 128 ? 2
     int c_lo = 0;
     if (p.n_swa > 0) c_lo = max(0, wg_min - p.n_swa + 1);
     c_lo &= ~(kTile - 1);
+
+    SplitRange sr = {1, c_lo, c_hi};
+    if constexpr (SPLIT) {
+        sr = split_range(c_lo, c_hi, z, n_split, kTile);
+        if (z >= sr.n) {   // no such range: an empty record, where the row block is cut
+            if (sr.n == 1) return;
+            for (int r = R0 + tid; r < min(M, R0 + ROWS); r += NW * 64)
+                *split_ml_at(p, (int64_t) (q0 + r / p.gqa) * p.H + hk * p.gqa + r % p.gqa, z) =
+                    make_float2(-INFINITY, 0.f);
+            return;
+        }
+        c_lo = sr.lo;
+        c_hi = sr.hi;
+    }
 
     // Q^T B operands (pre-scaled f16 hi/lo pairs; measured: +4-6% time, the
     // score error of a single f16 q removed), row positions, running state
@@ -448,10 +490,13 @@ __global__ __launch_bounds__(NW * 64, (D == 128 && KVT == 1) ? 4 : (D <= 128 ? 2
             const float lr = __shfl(l, 4 * g + i);
             if (r < M) {
                 const int t = q0 + r / p.gqa, h = hk * p.gqa + r % p.gqa;
-                const float inv = lr > 0.f ? 1.f / lr : 0.f;
-                float *op = p.out + ((int64_t) t * p.H + h) * D + n;
+                const int64_t orow = (int64_t) t * p.H + h;
+                const bool part = SPLIT && sr.n > 1;   // unnormalised, for the merge
+                const float inv = part ? 1.f : lr > 0.f ? 1.f / lr : 0.f;
+                float *op = (part ? split_o_at(p, orow, z, D) : p.out + orow * D) + n;
 #pragma unroll
                 for (int m = 0; m < NPV; m++) op[16 * m] = o[rt][m][i] * inv;
+                if (SPLIT && n == 4 * g + i) *split_ml_at(p, orow, z) = make_float2(m_run[rt], part ? lr : -1.f);
             }
         }
     }
@@ -459,11 +504,19 @@ __global__ __launch_bounds__(NW * 64, (D == 128 && KVT == 1) ? 4 : (D <= 128 ? 2
 
 template <int D, int NRT, int NW, int KVT>
 static hipError_t launch_prefill16_t(const AttnParams &p, int max_rows, hipStream_t stream) {
+    static_assert(NW * NRT * 16 == kPrefillBlockRows, "the host plans 128-row blocks");
     constexpr int ROWS = NW * NRT * 16;
     const int n_rb = (max_rows + ROWS - 1) / ROWS;
     const int pairs_per_xcd = (p.S * p.Hkv + 7) / 8;
-    const int nwg = 8 * pairs_per_xcd * n_rb;
-    hipLaunchKernelGGL((pa_prefill16_kernel<D, NRT, NW, KVT>), dim3(nwg), dim3(NW * 64), 0, stream, p, n_rb);
+    const int64_t nwg = 8 * (int64_t) pairs_per_xcd * n_rb * std::max(1, p.n_split);
+    if (nwg > INT32_MAX) return hipErrorInvalidValue;
+    const dim3 grid((unsigned) nwg), block(NW * 64);
+    if (p.n_split > 1) {
+        hipLaunchKernelGGL((pa_prefill16_kernel<D, NRT, NW, KVT, true>), grid, block, 0, stream, p, n_rb);
+        const hipError_t e = hipGetLastError();
+        return e != hipSuccess ? e : launch_split_merge(p, D, n_rb * ROWS, stream);
+    }
+    hipLaunchKernelGGL((pa_prefill16_kernel<D, NRT, NW, KVT, false>), grid, block, 0, stream, p, n_rb);
     return hipGetLastError();
 }
 
