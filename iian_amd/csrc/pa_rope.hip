@@ -46,6 +46,7 @@ constexpr int kRopeWaves = 4;           // waves (head rows in flight) per workg
 constexpr int kRopeMaxPairs = kRopeWaves * 64;   // n_dims / 2: one table entry per thread
 constexpr int kRopeQ8MaxDim = 512;      // largest head row staged for a Q8_0 pool
 constexpr int kRopeTargetWgs = 2048;    // workgroups a launch aims for
+constexpr int kRopeVecWgs = 1024;       // and one of the vector kernel
 
 __device__ __forceinline__ float rope_ramp(float low, float high, int i0) {
     const float y = (float) (i0 / 2) - low;
@@ -231,11 +232,161 @@ __global__ __launch_bounds__(kRopeWaves * 64) void pa_rope_kv_write_kernel(RopeP
     }
 }
 
+// ---- The common form: whole heads rotated, D = Dv, 16-byte aligned rows ----
+//
+// The kernel above keeps one row of a wave in flight, so a prefill step waits
+// for a memory round trip per row (a 1903-token step of H32/Hkv8/D128, 86 MB:
+// 25.6 us).  Here a lane moves 4 elements of each half of its row (two
+// 16-byte loads), lpr lanes share a row, and a wave has kRopeU groups of 64/lpr
+// rows in flight; the first of them are requested before the (cos, sin) table
+// is computed, which then costs no time of its own (17.6 us, 4.9 TB/s).  Two
+// groups and 64 registers, eight workgroups per CU, beat three at six (that
+// step 20.4 us: its 1903 workgroups then need a second round).
+// A Q8_0 block is 8 neighbouring lanes' values, quantised without LDS.  The
+// arithmetic is the same, and so is every bit.
+constexpr int kRopeU = 2;
+
+// Values v of elements e .. e+3 of head h of pool row `slot`.
+template <int T>
+__device__ __forceinline__ void rope_store4(void *pool, int64_t slot, int Hkv, int h, int D, int e, const float4 &v) {
+    const int64_t base = (slot * Hkv + h) * (int64_t) D + e;
+    if constexpr (T == 0) {
+        *(float4 *) ((float *) pool + base) = v;
+    } else if constexpr (T == 1) {
+        *(u32x2 *) ((_Float16 *) pool + base) = u32x2{pack_f16x2(v.x, v.y), pack_f16x2(v.z, v.w)};
+    } else {
+        float amax = fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
+#pragma unroll
+        for (int o = 1; o < 8; o <<= 1) amax = fmaxf(amax, __shfl_xor(amax, o));
+        const float d = amax / 127.f;
+        const float id = amax != 0.f ? 127.f / amax : 0.f;
+        const float x[4] = {v.x, v.y, v.z, v.w};
+        int q[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) q[i] = min(127, max(-128, (int) __builtin_rintf(x[i] * id))) & 0xff;
+        uint16_t *blk = (uint16_t *) ((uint8_t *) pool + (slot * Hkv + h) * (int64_t) (D / 32 * 34) + 34 * (e >> 5));
+        uint16_t *dst = blk + 1 + ((e & 31) >> 1);
+        dst[0] = (uint16_t) (q[0] | (q[1] << 8));
+        dst[1] = (uint16_t) (q[2] | (q[3] << 8));
+        if ((e & 31) == 0) blk[0] = __builtin_bit_cast(uint16_t, (_Float16) d);
+    }
+}
+
+// Token blockIdx.x, rows [blockIdx.y * rows_per_wg, +rows_per_wg) of its
+// nq + 2 Hkv rows, as above.  lpr = 1 << lpr_log2 >= D / 8 lanes per row.
+template <int KT, int VT>
+__global__ __launch_bounds__(kRopeWaves * 64, 8) void pa_rope_vec_kernel(RopeParams p, int nq, int rows_per_wg,
+                                                                      int lpr_log2) {
+#pragma clang fp contract(off)
+    __shared__ __attribute__((aligned(16))) float2 cs_tab[kRopeMaxPairs];
+    const int t = blockIdx.x, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int rpt = nq + 2 * p.Hkv, D = p.D, half = D >> 1;
+    const int r0 = blockIdx.y * rows_per_wg, r1 = min(rpt, r0 + rows_per_wg);
+    const int i = lane & ((1 << lpr_log2) - 1), sub = lane >> lpr_log2, rps = 64 >> lpr_log2;
+    const bool act = 4 * i < half;
+    const int64_t slot = p.slots[t];
+    const bool slot_ok = slot >= 0 && slot < p.n_cells;
+    if (blockIdx.y == 0 && threadIdx.x == 0 && !slot_ok && p.err) atomicOr(p.err, 1);
+    const bool ne = p.mode != 0;
+    float4 xa[kRopeU], xb[kRopeU];
+    auto row_of = [&](int rb, int u) { return rb + (u * kRopeWaves + wave) * rps + sub; };
+    auto load = [&](int rb) {
+#pragma unroll
+        for (int u = 0; u < kRopeU; u++) {
+            const int r = row_of(rb, u);
+            if (r < r1 && act) {
+                const float *src = r < nq           ? p.q_in + ((int64_t) t * p.H + r) * D
+                                   : r < nq + p.Hkv ? p.k_rows + ((int64_t) t * p.Hkv + (r - nq)) * D
+                                                    : p.v_rows + ((int64_t) t * p.Hkv + (r - nq - p.Hkv)) * D;
+                xa[u] = *(const float4 *) (src + 4 * i);
+                xb[u] = *(const float4 *) (src + half + 4 * i);
+            }
+        }
+    };
+    load(r0);
+    if (r0 < nq + p.Hkv) {   // workgroup-uniform: some row rotates
+        const int j = threadIdx.x;
+        if (j < half) {
+            float theta = (float) p.pos[t];
+            for (int k = 0; k < j; k++) theta *= p.theta_scale;
+            cs_tab[j] = rope_cs(p, theta, j);
+        }
+        __syncthreads();
+    }
+    for (int rb = r0; rb < r1; rb += kRopeU * kRopeWaves * rps) {
+        if (rb != r0) load(rb);
+#pragma unroll
+        for (int u = 0; u < kRopeU; u++) {
+            const int r = row_of(rb, u);
+            if (r >= r1 || !act) continue;
+            float4 a = xa[u], b = xb[u];
+            if (r < nq + p.Hkv) {
+                if (ne) {   // pairs (e, e + half)
+                    const float4 c0 = *(const float4 *) &cs_tab[4 * i], c1 = *(const float4 *) &cs_tab[4 * i + 2];
+                    const float2 y0 = rope_rotate(a.x, b.x, c0.x, c0.y), y1 = rope_rotate(a.y, b.y, c0.z, c0.w);
+                    const float2 y2 = rope_rotate(a.z, b.z, c1.x, c1.y), y3 = rope_rotate(a.w, b.w, c1.z, c1.w);
+                    a = make_float4(y0.x, y1.x, y2.x, y3.x);
+                    b = make_float4(y0.y, y1.y, y2.y, y3.y);
+                } else {    // pairs (2e, 2e + 1)
+                    const float4 ca = *(const float4 *) &cs_tab[2 * i], cb = *(const float4 *) &cs_tab[half / 2 + 2 * i];
+                    const float2 y0 = rope_rotate(a.x, a.y, ca.x, ca.y), y1 = rope_rotate(a.z, a.w, ca.z, ca.w);
+                    const float2 y2 = rope_rotate(b.x, b.y, cb.x, cb.y), y3 = rope_rotate(b.z, b.w, cb.z, cb.w);
+                    a = make_float4(y0.x, y0.y, y1.x, y1.y);
+                    b = make_float4(y2.x, y2.y, y3.x, y3.y);
+                }
+            }
+            if (r < nq) {
+                float *qo = p.q_out + ((int64_t) t * p.H + r) * D;
+                *(float4 *) (qo + 4 * i) = a;
+                *(float4 *) (qo + half + 4 * i) = b;
+            } else if (slot_ok) {
+                if (r < nq + p.Hkv) {
+                    rope_store4<KT>(p.k_pool, slot, p.Hkv, r - nq, D, 4 * i, a);
+                    rope_store4<KT>(p.k_pool, slot, p.Hkv, r - nq, D, half + 4 * i, b);
+                } else {
+                    rope_store4<VT>(p.v_pool, slot, p.Hkv, r - nq - p.Hkv, D, 4 * i, a);
+                    rope_store4<VT>(p.v_pool, slot, p.Hkv, r - nq - p.Hkv, D, half + 4 * i, b);
+                }
+            }
+        }
+    }
+}
+
+// The vector kernel's form: every pair of whole heads rotated (n_dims = D =
+// Dv), 4-element pieces within each half (and whole Q8_0 blocks), 16-byte
+// aligned rows.  (An f16 pool's pieces are 8 bytes, which the ABI requires.)
+static bool rope_vec_ok(const RopeParams &p, int type_k, int type_v) {
+    const bool q8 = type_k == 8 || type_v == 8;
+    uintptr_t al = (uintptr_t) p.k_rows | (uintptr_t) p.v_rows | (uintptr_t) p.q_in | (uintptr_t) p.q_out;
+    if (type_k == 0) al |= (uintptr_t) p.k_pool;
+    if (type_v == 0) al |= (uintptr_t) p.v_pool;
+    return p.n_dims == p.D && p.Dv == p.D && p.D % (q8 ? 64 : 8) == 0 && p.D <= 512 && al % 16 == 0;
+}
+
+template <int KT, int VT>
+static hipError_t launch_rope_vec(const RopeParams &p, hipStream_t stream) {
+    const int nq = p.q_in ? p.H : 0;
+    const int64_t rpt = nq + 2 * (int64_t) p.Hkv;
+    int lpr_log2 = 0;
+    while ((8 << lpr_log2) < p.D) lpr_log2++;
+    // rows per workgroup: a whole token's when the step has tokens enough for
+    // kRopeVecWgs workgroups, else fewer, in whole passes of the 4 waves
+    const int64_t pass = kRopeWaves * (64 >> lpr_log2);
+    const int64_t want = (p.T * rpt + kRopeVecWgs - 1) / kRopeVecWgs;
+    const int64_t rows_per_wg = std::min((rpt + pass - 1) / pass, std::max<int64_t>(1, (want + pass - 1) / pass)) * pass;
+    const int64_t chunks = (rpt + rows_per_wg - 1) / rows_per_wg;
+    if (chunks > 65535 || rpt > INT32_MAX / 2) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((pa_rope_vec_kernel<KT, VT>), dim3((unsigned) p.T, (unsigned) chunks), dim3(kRopeWaves * 64), 0,
+                       stream, p, nq, (int) rows_per_wg, lpr_log2);
+    return hipGetLastError();
+}
+
 // Rows per workgroup: a multiple of the 4 waves, sized so that the launch
 // holds about kRopeTargetWgs workgroups (one row per wave when the step has
 // few tokens, a whole token per workgroup when it has thousands).
 template <int KT, int VT>
 static hipError_t launch_rope_t(const RopeParams &p, hipStream_t stream) {
+    if (rope_vec_ok(p, KT, VT)) return launch_rope_vec<KT, VT>(p, stream);
     const int nq = p.q_in ? p.H : 0;
     const int64_t rpt = nq + 2 * (int64_t) p.Hkv;
     const int64_t per_wave_all = (rpt + kRopeWaves - 1) / kRopeWaves;
