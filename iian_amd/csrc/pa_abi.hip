@@ -45,12 +45,19 @@ constexpr int kF16DecodeWavesPerCuD256 = 3;
 // unit of work): 4 waves per CU measured best at Phi-3.5 shapes (414 us
 // against 420 at 3, 426 at 6, 455 at 2).
 constexpr int kF16DecodeWavesPerCuPairs = 4;
-// Matrix-core general path: decode waves per CU (its kernels hold two waves
-// per SIMD at head sizes up to 128, one above), alone and beside prefill
-// workgroups, and the prefill workgroups per CU a launch aims for.
+// Matrix-core general path.  Decode waves per CU: its kernels hold two waves
+// per SIMD at head sizes up to 128 and one above; beside prefill workgroups 3
+// measured best (2 chunks + 16 decodes, H32/Hkv8/D128 F32: 187 us at 2 and 3,
+// 195 at 4, 203 at 6, 207 at 8; H16/Hkv16/D96 F32 153, 140, 154, 160, 173;
+// H32/Hkv32/D80 F16 128, 122, 122, 132, 141).  Prefill workgroups per CU a
+// launch is split for: F16 chunks are quick, and their records cost more than
+// a second workgroup per CU gives (2 chunks of 500 at H32/Hkv32/D80: 82 us at
+// 1, 97 at 2, 110 at 4); over F32 two balance better (the step above 207 at 1,
+// 195 at 2 and 4, with 4 decode waves).
 constexpr int kGenDecodeWavesPerCu = 8;
-constexpr int kGenMixedDecodeWavesPerCu = 4;
+constexpr int kGenMixedDecodeWavesPerCu = 3;
 constexpr int kGenDecodeWavesPerCuWide = 4;
+constexpr int kGenPrefillWgsPerCuF16 = 1;
 constexpr int kGenPrefillWgsPerCu = 2;
 // Split prefill row blocks (prefill_splits): the rounds of D = 256 workgroups
 // a launch of about one round is cut into, and the most ranges per row block.
@@ -269,6 +276,15 @@ bool gen_mfma_path(int head_dim, int head_dim_v, int32_t block_size, int32_t max
            (int64_t) max_blocks * block_size <= INT32_MAX / 2 && rows <= (1 << 30);
 }
 
+// Records of row blocks cut into ns ranges: ns - 1 O rows (range 0's is in the
+// output) and ns (m, l) per output row.
+size_t split_o_bytes(size_t out_rows, int64_t ns, int head_dim_v) {
+    return align256(out_rows * (size_t) (ns - 1) * head_dim_v * sizeof(float));
+}
+size_t split_bytes(size_t out_rows, int64_t ns, int head_dim_v) {
+    return split_o_bytes(out_rows, ns, head_dim_v) + out_rows * (size_t) ns * 2 * sizeof(float);
+}
+
 // Ranges a prefill row block is cut into at most (split_range, pa_common.h),
 // with `room` bytes of workspace left for their records.  A launch whose row
 // blocks take at most half of the device's workgroup slots is cut to fill
@@ -299,10 +315,8 @@ int prefill_splits(AttnParams &p, int head_dim, bool mixed_one_launch, int64_t m
     int64_t cells = (int64_t) p.max_blocks * block_size;
     if (p.n_swa > 0) cells = std::min<int64_t>(cells, (int64_t) p.n_swa + max_rows / p.gqa);
     ns = std::min<int64_t>({ns, cells / kSplitMinCells, kMaxSplits});
-    // records: n_split - 1 O rows and n_split (m, l) per output row
     const size_t out_rows = (size_t) p.T * p.H;
-    while (ns > 1 && align256(out_rows * (ns - 1) * head_dim * sizeof(float)) + out_rows * ns * 2 * sizeof(float) > room)
-        ns--;
+    while (ns > 1 && split_bytes(out_rows, ns, head_dim) > room) ns--;
     return (int) std::max<int64_t>(ns, 1);
 }
 
@@ -481,9 +495,9 @@ int run_attention(hipStream_t st, const float *q, const void *k_pool, const void
         }
         if (!a.sk_workers) xl = {};
         g.n_dec_wgs = a.sk_workers / 4;
-        g.n_split = 1;
+        a.n_split = 1;
         int64_t pre_wgs = 0;
-        size_t split_o = 0, need = xl.total;
+        size_t split_at = 0, need = xl.total;
         if (a.decode_rows == 0 || !decode_only) {
             // 64-row blocks the batch can hold: one more than rows/64 for
             // every sequence that is not a decode one
@@ -494,27 +508,24 @@ int run_attention(hipStream_t st, const float *q, const void *k_pool, const void
             // tiles of the longest table, the records inside the workspace
             const int64_t full = std::max<int64_t>(1, rows / 64) * n_head_kv;
             const int64_t max_tiles = ((int64_t) max_blocks * block_size + kTile - 1) / kTile;
-            int64_t ns = ((int64_t) kGenPrefillWgsPerCu * cus + full - 1) / full;
+            const bool f16 = type_k == IIAN_PA_TYPE_F16 && type_v == IIAN_PA_TYPE_F16;
+            int64_t ns = ((int64_t) (f16 ? kGenPrefillWgsPerCuF16 : kGenPrefillWgsPerCu) * cus + full - 1) / full;
             ns = std::min<int64_t>({ns, std::max<int64_t>(1, max_tiles / 8), 16});
-            const size_t per_split = (size_t) n_tokens * n_head * (head_dim_v + 2) * sizeof(float);
-            if (ns > 1)
-                ns = std::min<int64_t>(ns, (int64_t) ((cap - std::min(cap, align256(xl.total) + 512)) / per_split));
-            g.n_split = (int) std::max<int64_t>(ns, 1);
-            pre_wgs = n_rb * n_head_kv * g.n_split;
-            if (g.n_split > 1) {
-                split_o = align256(xl.total);
-                need = split_o + align256((size_t) n_tokens * n_head * g.n_split * head_dim_v * sizeof(float)) +
-                       (size_t) n_tokens * n_head * g.n_split * 2 * sizeof(float);
-            }
+            const size_t out_rows = (size_t) n_tokens * n_head;
+            split_at = align256(xl.total);
+            const size_t room = cap - std::min(split_at, cap);
+            while (ns > 1 && split_bytes(out_rows, ns, head_dim_v) > room) ns--;
+            a.n_split = (int) std::max<int64_t>(ns, 1);
+            pre_wgs = n_rb * n_head_kv * a.n_split;
+            if (a.n_split > 1) need = split_at + split_bytes(out_rows, a.n_split, head_dim_v);
         }
         const int rc = ws_resolve(src, st, need, &ws);
         if (rc) return rc;
         a.part_o = (float *) (ws + xl.o);
         a.part_ml = (float *) (ws + xl.ml);
         a.seg_info = (int2 *) (ws + xl.seg);
-        g.split_o = (float *) (ws + split_o);
-        g.split_ml = (float *) (ws + split_o +
-                                align256((size_t) n_tokens * n_head * g.n_split * head_dim_v * sizeof(float)));
+        a.split_o = (float *) (ws + split_at);
+        a.split_ml = (float *) (ws + split_at + split_o_bytes((size_t) n_tokens * n_head, a.n_split, head_dim_v));
         return launch_gen_mfma(g, type_k, type_v, pre_wgs, st) == hipSuccess ? IIAN_PA_OK : IIAN_PA_ERR_HIP;
     }
     if (!mfma_path(type_k, type_v, head_dim, head_dim_v, bs_log2) && !f16_96) {
@@ -684,22 +695,17 @@ int run_attention(hipStream_t st, const float *q, const void *k_pool, const void
     const WorkspaceLayout xl = exact_layout(p);
     size_t need = xl.total;
     const size_t split_at = align256(xl.total);
-    size_t split_o = 0;
     p.n_split = 1;
     if (!decode_only) {
         const size_t cap = src.scratch ? kScratchBytes : wl.total;
         p.n_split = prefill_splits(p, head_dim, mixed_one_launch, max_rows, block_size, cus,
                                    cap - std::min(split_at, cap));
-        if (p.n_split > 1) {
-            const size_t rows = (size_t) n_tokens * n_head;
-            split_o = align256(rows * (p.n_split - 1) * head_dim_v * sizeof(float));
-            need = split_at + split_o + rows * p.n_split * 2 * sizeof(float);
-        }
+        if (p.n_split > 1) need = split_at + split_bytes((size_t) n_tokens * n_head, p.n_split, head_dim_v);
     }
     const int rc = ws_resolve(src, st, need, &ws);
     if (rc) return rc;
     p.split_o = (float *) (ws + split_at);
-    p.split_ml = (float *) (ws + split_at + split_o);
+    p.split_ml = (float *) (ws + split_at + split_o_bytes((size_t) n_tokens * n_head, p.n_split, head_dim_v));
     p.part_o = (float *) (ws + xl.o);
     p.part_ml = (float *) (ws + xl.ml);
     p.seg_info = (int2 *) (ws + xl.seg);

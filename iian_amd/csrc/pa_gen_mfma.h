@@ -17,31 +17,34 @@
 //   V F16          V exact, P as two f16 terms (22 bits), on the f16 MFMA
 //
 // Work split.  One wave owns 16 query rows (r = j*gqa + g) of one (sequence,
-// kv head) and walks 32-cell tiles (16 when V is not F16) straight from the block table: K rows are
-// the A operand of S^T as they lie in memory (lane (n, g): cell n, dims
-// 8g .. 8g+7 of each 32), S^T's result layout (lane (n, g): cells 4g .. 4g+3
-// of row n) is PV's A operand, and V rows are read 4 dims per lane, so
-// nothing passes through LDS and no two waves wait for each other.  The next
-// tile's K loads go out after QK^T, its V loads after PV, its table entries
-// one tile earlier still.
+// kv head) and walks 32-cell tiles (16 when V is not F16) through the block
+// table: K rows are the A operand of S^T as they lie in memory (lane (n, g):
+// cell n, dims 8g .. 8g+7 of each 32), S^T's result layout (lane (n, g): cells
+// 4g .. 4g+3 of row n) is PV's A operand, and V rows are read 4 dims per lane.
 //   - sequences with at most 16 rows per kv head (decode): stream-K, as the
 //     f16 decode kernel (pa_common.h): every wave of the first n_dec_wgs
 //     workgroups takes an equal range of the call's (sequence, kv head, tile)
-//     line and leaves partial records for the merge;
+//     line, reads its operands from memory itself, the next tile's K after
+//     QK^T and its V after PV, and leaves partial records for the merge;
 //   - the others (prefill chunks): a 4-wave workgroup takes 64 consecutive rows
-//     and one of n_split ranges of their tiles.  Its waves read the same tiles
-//     at about the same time, so the CU's L1 serves three of the four.
+//     and one of n_split ranges of their tiles, each tile staged once in LDS
+//     for the four waves (F32 and F16 pools; over Q8_0 the waves read for
+//     themselves).
 // Both kinds run in one launch, so the memory-bound decode waves share the CUs
 // with the chunks' MFMAs.  One merge launch follows when anything was split.
 //
-// What bounds it: decode, HBM; chunks over F32 or Q8_0, the fp32 MFMA (64
-// flop per cycle and SIMD); chunks over F16, the L1 (16 KB of K and V per 640
-// MFMA cycles at head size 128).  Measured against pa_general_kernel (one
-// MI355X, whole calls): 32 decodes of 512-8192 cells over F32 pools, H32/Hkv8/
-// D128, 215 -> 158 us (5.2 TB/s); 2 chunks and 16 decodes over F32 1448 -> 211
-// us; 2 chunks and 16 decodes over F16 at H32/Hkv32/D80 9030 -> 156 us.
-// Distance from a 64-bit result there: 6.5e-7 -> 4.1e-7 (F32), 6.3e-7 ->
-// 5.7e-7 (F16, D80).
+// What bounds it: decode, HBM.  Chunks over F32, the fp32 MFMA (64 flop per
+// cycle and SIMD; busy 55% of the CUs' time at 2 chunks of 449 and 356 tokens,
+// H32/Hkv8/D128); chunks over F16, VALU work between short MFMAs (about 300
+// instructions and 34 MFMAs per tile at D = 80).  Without the staging each wave
+// read every tile itself, and the vector memory address unit, 30 cycles per
+// instruction, was busy 65% of a D = 80 launch (156 against 122 us).
+//
+// Measured against pa_general_kernel (one MI355X, whole calls): 32 decodes of
+// 512-8192 cells over F32 pools, H32/Hkv8/D128, 215 -> 158 us (5.2 TB/s); those
+// 2 chunks and 16 decodes over F32 1448 -> 186 us; 2 chunks of 500 and 16
+// decodes over F16 at H32/Hkv32/D80 9030 -> 122 us.  Distance from a 64-bit
+// result there: 6.5e-7 -> 4.1e-7 (F32), 6.3e-7 -> 5.7e-7 (F16, D80).
 #pragma once
 
 #include "pa_common.h"
@@ -118,7 +121,8 @@ __device__ __forceinline__ float gm_v_f32(const GmV<VT> &v, int e) {
 struct GmPiece {
     int s, hk, q0, M, row0;
     int pmin, pmax;   // positions of the wave's rows (pmax also stands in for rows past M)
-    int cb, ce;
+    int cb, ce;       // staged pieces: the workgroup's range
+    int wcb, wce;     // and the wave's part of it
     int mode;         // 0: normalised output, 1: stream-K record rec, 2: record z of each row's n_split
     int rec;
 };
@@ -154,9 +158,24 @@ __device__ __forceinline__ void gm_split3(float x, _Float16 &h, _Float16 &m, _Fl
     l = __builtin_bit_cast(_Float16, c);
 }
 
+// The LDS tile of a prefill workgroup, two buffers of it: rows of the kernel's
+// largest head size, so that every read is a lane base plus an immediate.  K
+// rows are padded by 16 bytes (16 rows read at one offset start 4 banks apart,
+// in some order), V rows by 32 (rows 4 apart start 32 banks apart).
+constexpr int gm_k_stride(int kt, int nk) { return 32 * nk * (kt == 0 ? 4 : 2) + 16; }
+constexpr int gm_v_stride(int vt, int nv) { return 64 * nv * (vt == 0 ? 4 : 2) + 32; }
+__host__ __device__ constexpr bool gm_staged_types(int kt, int vt) { return kt != 8 && vt != 8; }
+// (V rows of whole 16-byte pieces: the host asks before it plans)
+__host__ __device__ inline bool gm_staged(int kt, int vt, int Dv) { return gm_staged_types(kt, vt) && (vt == 0 || Dv % 8 == 0); }
+__host__ __device__ constexpr int gm_tile(int vt) { return vt == 1 ? 32 : 16; }
+
 // NK: 32-dim chunks of K (D <= 32 NK), NV: 64-dim blocks of V (Dv <= 64 NV).
-template <int KT, int VT, int NK, int NV>
-__device__ __forceinline__ void gm_piece(const GenMfmaParams &p, const GmPiece &vp) {
+// STAGED: the workgroup's waves walk [cb, ce) together, each tile staged in
+// LDS once for the four of them (through registers, two buffers, one barrier
+// per tile), and a wave skips the tiles outside its own rows' [wcb, wce);
+// otherwise the wave reads its operands from memory itself.
+template <int KT, int VT, int NK, int NV, bool STAGED>
+__device__ __forceinline__ void gm_piece(const GenMfmaParams &p, const GmPiece &vp, char *lds) {
     const AttnParams &a = p.a;
     // wave-uniform, and known to be: the tile loop's control and addresses are scalar
     GmPiece pc;
@@ -169,6 +188,10 @@ __device__ __forceinline__ void gm_piece(const GenMfmaParams &p, const GmPiece &
     pc.pmax = __builtin_amdgcn_readfirstlane(vp.pmax);
     pc.cb = __builtin_amdgcn_readfirstlane(vp.cb);
     pc.ce = __builtin_amdgcn_readfirstlane(vp.ce);
+    if constexpr (STAGED) {
+        pc.wcb = __builtin_amdgcn_readfirstlane(vp.wcb);
+        pc.wce = __builtin_amdgcn_readfirstlane(vp.wce);
+    }
     pc.mode = __builtin_amdgcn_readfirstlane(vp.mode);
     pc.rec = __builtin_amdgcn_readfirstlane(vp.rec);
     constexpr bool KF16 = KT == 1, VF16 = VT == 1;
@@ -346,6 +369,79 @@ __device__ __forceinline__ void gm_piece(const GenMfmaParams &p, const GmPiece &
         }
     };
 
+    // ---- staging (STAGED): pass u of a step copies its 16-byte pieces tid +
+    // 256u; past the step's last piece a thread repeats it ----
+    constexpr int KP = STAGED ? (32 * NK * KE + 255) / 256 : 1, VP = STAGED ? (64 * NV * VE + 255) / 256 : 1;
+    constexpr int kst = gm_k_stride(KT, NK), vst = gm_v_stride(VT, NV), vat = TC * kst, bufb = TC * (kst + vst);
+    uint32_t kgo[KP], klo[KP], vgo[VP], vlo[VP];   // cell << 24 | row offset, LDS offset
+    u32x4 ksr[STAGED ? NT * KP : 1], vsr[STAGED ? NT * VP : 1];
+    if constexpr (STAGED) {
+        const int tid = threadIdx.x, kc = D * KE / 16, vc = Dv * VE / 16;
+#pragma unroll
+        for (int u = 0; u < KP; u++) {
+            const int i = min(tid + 256 * u, 16 * kc - 1), cell = i / kc, c = i - cell * kc;
+            kgo[u] = (uint32_t) cell << 24 | (uint32_t) (pc.hk * D * KE + 16 * c);
+            klo[u] = cell * kst + 16 * c;
+        }
+#pragma unroll
+        for (int u = 0; u < VP; u++) {
+            const int i = min(tid + 256 * u, 16 * vc - 1), cell = i / vc, c = i - cell * vc;
+            vgo[u] = (uint32_t) cell << 24 | (uint32_t) (pc.hk * Dv * VE + 16 * c);
+            vlo[u] = vat + cell * vst + 16 * c;
+        }
+    }
+    auto stage_load = [&](const Step (&st)[NT]) {
+#pragma unroll
+        for (int t = 0; t < NT; t++) {
+            const char *kb = a.k_pool + pool_off(st[t].row, a.k_row), *vb = a.v_pool + pool_off(st[t].row, p.v_row);
+#pragma unroll
+            for (int u = 0; u < KP; u++)
+                ksr[t * KP + u] = gm_ld<u32x4>(kb, __umul24(min(kgo[u] >> 24, st[t].lim), (uint32_t) a.k_row) +
+                                                       (kgo[u] & 0xffffffu));
+#pragma unroll
+            for (int u = 0; u < VP; u++)
+                vsr[t * VP + u] = gm_ld<u32x4>(vb, __umul24(min(vgo[u] >> 24, st[t].lim), (uint32_t) p.v_row) +
+                                                       (vgo[u] & 0xffffffu));
+        }
+    };
+    auto stage_store = [&](int buf) {
+        char *b = lds + buf * bufb;
+#pragma unroll
+        for (int t = 0; t < NT; t++) {
+#pragma unroll
+            for (int u = 0; u < KP; u++) *(u32x4 *) (b + 16 * t * kst + klo[u]) = ksr[t * KP + u];
+#pragma unroll
+            for (int u = 0; u < VP; u++) *(u32x4 *) (b + 16 * t * vst + vlo[u]) = vsr[t * VP + u];
+        }
+    };
+    // this wave's operands of the tile in buffer buf
+    auto lds_k = [&](int buf) {
+        const char *b = lds + buf * bufb + n * kst + 8 * g * KE, *bl = lds + buf * bufb + n * kst + kd_last * KE;
+#pragma unroll
+        for (int t = 0; t < NT; t++)
+#pragma unroll
+            for (int j = 0; j < NK; j++) {
+                if (j >= JOPT && 32 * j >= D) continue;   // wave-uniform
+                const char *src = (JOPT < NK && j >= JOPT ? b + (min(32 * j + 8 * g, D - 8) - 8 * g) * KE
+                                   : j == NK - 1          ? bl : b + 32 * j * KE) + 16 * t * kst;
+                if constexpr (KT != 8) kr[t][j].a = *(const u32x4 *) src;
+                if constexpr (KT == 0) kr[t][j].b = *(const u32x4 *) (src + 16);
+            }
+    };
+    auto lds_v = [&](int buf) {
+        const char *b = lds + buf * bufb + vat + 4 * g * vst + 4 * n * VE, *be = b + (vd_last - 4 * n) * VE;
+#pragma unroll
+        for (int c = 0; c < CV; c++)
+#pragma unroll
+            for (int bl = 0; bl < NV; bl++) {
+                if (bl >= BOPT && 64 * bl >= Dv) continue;   // wave-uniform
+                const char *src = (bl == NV - 1 ? be : BOPT < NV ? b + (min(64 * bl + 4 * n, Dv - 4) - 4 * n) * VE
+                                                                 : b + 64 * bl * VE) + (16 * (c >> 2) + (c & 3)) * vst;
+                if constexpr (VT == 0) vr[c][bl].a = *(const u32x4 *) src;
+                else if constexpr (VT == 1) vr[c][bl].a = *(const u32x2 *) src;
+            }
+    };
+
     // m_ref: the row's reference in log2 units, 7 below the largest score it
     // was last moved to, so that P lies in [0, 2^15] (the range in which two
     // f16 terms hold 22 bits of every P down to 2^-32 of the largest)
@@ -361,10 +457,31 @@ __device__ __forceinline__ void gm_piece(const GenMfmaParams &p, const GmPiece &
         for (int t = 0; t < NT; t++) st[t] = step_of(step_id(pc.cb + 16 * t));
 #pragma unroll
         for (int t = 0; t < NT; t++) nxt[t] = step_id(pc.cb + TC + 16 * t);
-        load_k(st);
-        load_v(st);
+        int buf = 0;
+        if constexpr (STAGED) {
+            stage_load(st);
+            stage_store(0);
+            __syncthreads();
+        } else {
+            load_k(st);
+            load_v(st);
+        }
         for (int tile = pc.cb; tile < pc.ce; tile += TC) {
             const bool has_next = tile + TC < pc.ce;
+            bool mine = true;   // some row of this wave sees a cell of the tile
+            if constexpr (STAGED) {
+                if (has_next) {
+#pragma unroll
+                    for (int t = 0; t < NT; t++) {
+                        st[t] = step_of(nxt[t]);
+                        nxt[t] = step_id(tile + 2 * TC + 16 * t);
+                    }
+                    stage_load(st);
+                }
+                mine = tile < pc.wce && tile + TC > pc.wcb;
+                if (mine) lds_k(buf);
+            }
+            if (mine) {
             // S^T = K Q^T: lane (n, g) gets cells 16t + 4g + i of row n
             f32x4 sacc[NT];
 #pragma unroll
@@ -407,7 +524,7 @@ __device__ __forceinline__ void gm_piece(const GenMfmaParams &p, const GmPiece &
                     for (int t = 0; t < NT; t++) sacc[t] += part[0][t] + part[1][t];
                 }
             }
-            if (has_next) {
+            if (!STAGED && has_next) {
 #pragma unroll
                 for (int t = 0; t < NT; t++) {
                     st[t] = step_of(nxt[t]);
@@ -415,6 +532,7 @@ __device__ __forceinline__ void gm_piece(const GenMfmaParams &p, const GmPiece &
                 }
                 load_k(st);
             }
+            if constexpr (STAGED) lds_v(buf);
 
             // online softmax, exp2 domain; P in registers
             float x[CV];
@@ -505,7 +623,13 @@ __device__ __forceinline__ void gm_piece(const GenMfmaParams &p, const GmPiece &
                     for (int e = 0; e < 4; e++) o[4 * b + e] += part[e];
                 }
             }
-            if (has_next) load_v(st);
+            if (!STAGED && has_next) load_v(st);
+            }
+            if constexpr (STAGED) {
+                if (has_next) stage_store(buf ^ 1);
+                __syncthreads();
+                buf ^= 1;
+            }
         }
     }
 
@@ -529,7 +653,7 @@ __device__ __forceinline__ void gm_piece(const GenMfmaParams &p, const GmPiece &
         } else if (pc.mode == 1) {
             op = rec_o(a, pc.rec, 0, r - pc.row0, Dv);
         } else {
-            op = p.split_o + (orow * p.n_split + pc.rec) * Dv;
+            op = split_o_at(a, orow, pc.rec, Dv);
         }
 #pragma unroll
         for (int b = 0; b < NV; b++) {
@@ -545,7 +669,7 @@ __device__ __forceinline__ void gm_piece(const GenMfmaParams &p, const GmPiece &
             ml = rec_ml(a, pc.rec, 0, n);
         } else {
             const int64_t orow = (int64_t) (pc.q0 + rown / a.gqa) * a.H + pc.hk * a.gqa + rown % a.gqa;
-            ml = p.split_ml + 2 * (orow * p.n_split + pc.rec);
+            ml = (float *) split_ml_at(a, orow, pc.rec);
         }
         *(float2 *) ml = make_float2(m_ref, l);
     }
@@ -629,13 +753,13 @@ __device__ __forceinline__ int gm_row_blocks(const AttnParams &a, int s, int &q0
 // n_split.  Consecutive workgroups go to consecutive XCDs, so with a multiple
 // of 8 kv heads every row block and range of one head runs on one XCD and
 // shares its K and V through that L2.  False when the wave has no rows.
-__device__ __forceinline__ bool gm_prefill_piece(const GenMfmaParams &p, int b, GmPiece &pc) {
+__device__ __forceinline__ bool gm_prefill_piece(const GenMfmaParams &p, int b, bool staged, GmPiece &pc) {
     const AttnParams &a = p.a;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     pc.hk = b % a.Hkv;
     const int rest = b / a.Hkv;
-    const int z = rest % p.n_split;
-    const int rbl = rest / p.n_split;
+    const int z = rest % a.n_split;
+    const int rbl = rest / a.n_split;
     int base = 0, q0, nq;
     int nrb = gm_row_blocks(a, lane, q0, nq);
     int incl = wave_incl_scan(nrb);
@@ -659,10 +783,10 @@ __device__ __forceinline__ bool gm_prefill_piece(const GenMfmaParams &p, int b, 
     pc.M = nq * a.gqa;
     const int R0 = rb * kGmBlockRows;
     pc.row0 = R0 + wave * kGmRows;
-    if (pc.row0 >= pc.M) return false;
+    if (pc.row0 >= pc.M && !staged) return false;   // (a staged workgroup's waves all walk its tiles)
     // positions of the block's rows (at most 64 tokens) and of the wave's
     const int j0 = R0 / a.gqa, j1 = (min(pc.M, R0 + kGmBlockRows) - 1) / a.gqa;
-    const int w0 = pc.row0 / a.gqa, w1 = (min(pc.M, pc.row0 + kGmRows) - 1) / a.gqa;
+    const int w0 = pc.row0 / a.gqa, w1 = (min(pc.M, pc.row0 + kGmRows) - 1) / a.gqa;   // (none: no lane's token)
     int mn = INT32_MAX, mx = INT32_MIN, wmn = INT32_MAX, wmx = INT32_MIN;
     const int j = j0 + lane;
     if (j <= j1) {
@@ -685,47 +809,73 @@ __device__ __forceinline__ bool gm_prefill_piece(const GenMfmaParams &p, int b, 
     const int hi = a.causal ? min(L, max(mx + 1, 0)) : L;
     const int lo = a.n_swa > 0 ? min(max(0, mn - a.n_swa + 1) & ~(kTile - 1), hi) : 0;
     const int nt = (hi - lo + kTile - 1) / kTile;
-    const int per = (nt + p.n_split - 1) / p.n_split;
+    const int per = (nt + a.n_split - 1) / a.n_split;
     pc.cb = lo + min(nt, z * per) * kTile;
     pc.ce = min(hi, lo + min(nt, (z + 1) * per) * kTile);
     // the part of the range this wave's own rows can see
-    if (a.causal) pc.ce = min(pc.ce, max(pc.pmax + 1, 0));
-    if (a.n_swa > 0) pc.cb = max(pc.cb, max(0, pc.pmin - a.n_swa + 1) & ~(kTile - 1));
-    pc.mode = p.n_split > 1 ? 2 : 0;
+    pc.wcb = pc.cb;
+    pc.wce = pc.ce;
+    if (a.causal) pc.wce = min(pc.wce, max(pc.pmax + 1, 0));
+    if (a.n_swa > 0) pc.wcb = max(pc.wcb, max(0, pc.pmin - a.n_swa + 1) & ~(kTile - 1));
+    if (pc.row0 >= pc.M) pc.wce = pc.wcb;
+    if (!staged) {
+        pc.cb = pc.wcb;
+        pc.ce = pc.wce;
+    }
+    pc.mode = a.n_split > 1 ? 2 : 0;
     pc.rec = z;
     return true;
 }
 
 template <int KT, int VT, int NK, int NV>
 __global__ __launch_bounds__(kGmWaves * 64, NK <= 4 ? 2 : 1) void pa_gen_mfma_kernel(GenMfmaParams p) {
+    extern __shared__ __attribute__((aligned(16))) char gm_lds[];
     const bool pre = (int) blockIdx.x >= p.n_dec_wgs;
     const int worker = __builtin_amdgcn_readfirstlane(blockIdx.x * kGmWaves + (threadIdx.x >> 6));
     GmPiece pc;
+    if constexpr (gm_staged_types(KT, VT)) {
+        if (pre && p.staged) {
+            if (gm_prefill_piece(p, blockIdx.x - p.n_dec_wgs, true, pc)) gm_piece<KT, VT, NK, NV, true>(p, pc, gm_lds);
+            return;
+        }
+    }
     GmPieceIter it;
     bool go;
     if (pre) {
-        go = gm_prefill_piece(p, blockIdx.x - p.n_dec_wgs, pc);
+        go = gm_prefill_piece(p, blockIdx.x - p.n_dec_wgs, false, pc);
     } else {
         it.init(p.a, worker);
         go = it.next(p.a, worker, pc);
     }
     while (go) {
-        gm_piece<KT, VT, NK, NV>(p, pc);
+        gm_piece<KT, VT, NK, NV, false>(p, pc, nullptr);
         go = !pre && it.next(p.a, worker, pc);
     }
 }
 
+template <int KT, int VT, int NK, int NV>
+static hipError_t launch_gen_mfma_n(const GenMfmaParams &p, unsigned wgs, hipStream_t stream) {
+    size_t lds = 0;
+    if (p.staged)
+        lds = 2 * gm_tile(VT) * (size_t) (gm_k_stride(KT, NK) + gm_v_stride(VT, NV));
+    if (lds > 64 * 1024) {   // head sizes near 256: the opt-in for more dynamic LDS
+        const hipError_t e = hipFuncSetAttribute((const void *) pa_gen_mfma_kernel<KT, VT, NK, NV>,
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds);
+        if (e != hipSuccess) return e;
+    }
+    hipLaunchKernelGGL((pa_gen_mfma_kernel<KT, VT, NK, NV>), dim3(wgs), dim3(kGmWaves * 64), lds, stream, p);
+    return hipGetLastError();
+}
+
 template <int KT, int VT>
 static hipError_t launch_gen_mfma_v(const GenMfmaParams &p, unsigned wgs, hipStream_t stream) {
-    const dim3 grid(wgs), block(kGmWaves * 64);
     switch (gen_mfma_chunks(p.D, p.Dv)) {
-        case 2: hipLaunchKernelGGL((pa_gen_mfma_kernel<KT, VT, 2, 1>), grid, block, 0, stream, p); break;
-        case 3: hipLaunchKernelGGL((pa_gen_mfma_kernel<KT, VT, 3, 2>), grid, block, 0, stream, p); break;
-        case 4: hipLaunchKernelGGL((pa_gen_mfma_kernel<KT, VT, 4, 2>), grid, block, 0, stream, p); break;
-        case 8: hipLaunchKernelGGL((pa_gen_mfma_kernel<KT, VT, 8, 4>), grid, block, 0, stream, p); break;
+        case 2: return launch_gen_mfma_n<KT, VT, 2, 1>(p, wgs, stream);
+        case 3: return launch_gen_mfma_n<KT, VT, 3, 2>(p, wgs, stream);
+        case 4: return launch_gen_mfma_n<KT, VT, 4, 2>(p, wgs, stream);
+        case 8: return launch_gen_mfma_n<KT, VT, 8, 4>(p, wgs, stream);
         default: return hipErrorInvalidValue;
     }
-    return hipGetLastError();
 }
 
 template <int KT>

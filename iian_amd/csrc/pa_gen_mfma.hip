@@ -43,18 +43,20 @@ __global__ __launch_bounds__(256) void pa_gen_merge_kernel(GenMfmaParams p, int 
     const int q0 = min(max(a.qsl[lo], 0), a.T), nq = min(max(a.qsl[lo + 1], q0), a.T) - q0;
     // rows of a decode sequence, and of none, have no split records
     if (t < q0 || t >= q0 + nq || (int64_t) nq * a.gqa <= a.decode_rows) return;
-    merge_row<1>(p.split_o + row * p.n_split * p.Dv, p.Dv, p.split_ml + 2 * row * p.n_split, 2, p.n_split, p.Dv,
-                 a.out + row * p.Dv, comb);
+    merge_split_row(a, row, p.Dv, 4 * (threadIdx.x & 63));
 }
 
-hipError_t launch_gen_mfma(const GenMfmaParams &p, int type_k, int type_v, int64_t n_prefill_wgs, hipStream_t stream) {
+hipError_t launch_gen_mfma(const GenMfmaParams &params, int type_k, int type_v, int64_t n_prefill_wgs,
+                           hipStream_t stream) {
+    GenMfmaParams p = params;
+    p.staged = n_prefill_wgs > 0 && gm_staged(type_k, type_v, p.Dv);
     const int64_t wgs = p.n_dec_wgs + n_prefill_wgs;
     const int64_t seg = p.n_dec_wgs ? (int64_t) p.a.S * p.a.Hkv : 0;
     // few segments: their records are many (on average more than 16 each)
     const bool wide = seg * 16 <= p.a.sk_workers;
     const int seg_rows = (int) std::min<int64_t>(kGmRows, (int64_t) p.a.max_q * p.a.gqa);
     const int64_t seg_wgs = wide ? seg * seg_rows : seg;
-    const int64_t row_wgs = n_prefill_wgs && p.n_split > 1 ? ((int64_t) p.a.T * p.a.H + 3) / 4 : 0;
+    const int64_t row_wgs = n_prefill_wgs && p.a.n_split > 1 ? ((int64_t) p.a.T * p.a.H + 3) / 4 : 0;
     if (wgs <= 0 || wgs > INT32_MAX || seg_wgs + row_wgs > INT32_MAX) return hipErrorInvalidValue;
     hipError_t e;
     switch (type_k) {

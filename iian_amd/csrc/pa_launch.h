@@ -32,14 +32,13 @@ struct GenParams {
 
 // Everything the matrix-core general kernels (pa_gen_mfma.h) read, by value.
 struct GenMfmaParams {
-    AttnParams a;               // k_row, the decode rows' records, segment table; bs_log2 and qscale unused
+    AttnParams a;               // k_row, the decode rows' records, segment table, the prefill rows' ranges
+                                // (a.n_split of every row block); bs_log2 and qscale unused
     int64_t v_row;              // bytes per V pool row (a.k_row: K's)
-    float *split_o;             // prefill split records: [T*H][n_split][Dv]
-    float *split_ml;            // [T*H][n_split] of (m in log2 units, l)
     int32_t D, Dv, block_size;
     int32_t bs_log2;            // -1: block_size is not a power of two
     int32_t n_dec_wgs;          // leading workgroups that hold stream-K workers (a.sk_workers / 4)
-    int32_t n_split;            // ranges per prefill row block
+    int32_t staged;             // prefill workgroups stage their tiles in LDS (set by the launcher)
     float sscale;               // of the dot product: scale (before a softcap) or scale * log2 e
 };
 

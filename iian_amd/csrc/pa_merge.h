@@ -94,4 +94,28 @@ __device__ __forceinline__ void merge_row(const float *o0, int64_t o_stride, con
     *(float4 *) (out + d) = make_float4(acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv);
 }
 
+// Output row `row` of a split prefill row block (split_range, pa_common.h), dims
+// d .. d+3 by this lane: out = sum_z 2^(m_z - m) O_z / sum_z 2^(m_z - m) l_z over
+// its ranges, range 0's O taken from `out` itself.
+__device__ __forceinline__ void merge_split_row(const AttnParams &p, int64_t row, int D, int d) {
+    float mx = -INFINITY;
+    for (int z = 0; z < p.n_split; z++) mx = fmaxf(mx, split_ml_at(p, row, z)->x);
+    if (d >= D) return;
+    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+    float ls = 0.f;
+    for (int z = 0; z < p.n_split; z++) {
+        const float2 ml = *split_ml_at(p, row, z);
+        if (ml.x == -INFINITY) continue;   // no visible cell, or no such range: its O may hold anything
+        const float w = __builtin_amdgcn_exp2f(ml.x - mx);
+        const float4 v = *(const float4 *) (split_o_at(p, row, z, D) + d);
+        ls = fmaf(w, ml.y, ls);
+        acc.x = fmaf(w, v.x, acc.x);
+        acc.y = fmaf(w, v.y, acc.y);
+        acc.z = fmaf(w, v.z, acc.z);
+        acc.w = fmaf(w, v.w, acc.w);
+    }
+    const float inv = ls > 0.f ? 1.f / ls : 0.f;
+    *(float4 *) (p.out + row * D + d) = make_float4(acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv);
+}
+
 }  // namespace iian_pa

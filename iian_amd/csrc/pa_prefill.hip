@@ -39,6 +39,7 @@
 #include "pa_launch.h"
 #include "pa_mfma.h"
 #include "pa_decode_body.h"
+#include "pa_merge.h"
 
 #include <algorithm>
 
@@ -645,9 +646,7 @@ __global__ __launch_bounds__(NW * 64, PrefillOcc<D>::kWavesPerSimd) void pa_pref
     }
 }
 
-// The split row blocks' merge: out = sum_z 2^(m_z - m) O_z / sum_z 2^(m_z - m)
-// l_z over the ranges of each row of a prefill sequence, range 0's O taken from
-// `out` itself.  One round trip of (m, l) and one of the O rows; a lane holds 4
+// The split row blocks' merge (merge_split_row).  One round trip of (m, l) and one of the O rows; a lane holds 4
 // dims, so a row takes lpr = 16, 32 or 64 lanes and a wave 64 / lpr rows.  Rows
 // the launch did not cover (past cover_rows of a sequence) are left alone.
 __global__ __launch_bounds__(256) void pa_split_merge_kernel(AttnParams p, int D, int lpr, int cover_rows) {
@@ -665,24 +664,7 @@ __global__ __launch_bounds__(256) void pa_split_merge_kernel(AttnParams p, int D
     }
     const int q0 = min(max(p.qsl[lo], 0), p.T), nq = min(max(p.qsl[lo + 1], q0), p.T) - q0;
     if (t < q0 || t >= q0 + nq || nq * p.gqa <= p.decode_rows || (t - q0) * p.gqa + h % p.gqa >= cover_rows) return;
-    float mx = -INFINITY;
-    for (int z = 0; z < p.n_split; z++) mx = fmaxf(mx, split_ml_at(p, row, z)->x);
-    if (d >= D) return;
-    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-    float ls = 0.f;
-    for (int z = 0; z < p.n_split; z++) {
-        const float2 ml = *split_ml_at(p, row, z);
-        if (ml.x == -INFINITY) continue;   // no visible cell, or no such range: its O may hold anything
-        const float w = __builtin_amdgcn_exp2f(ml.x - mx);
-        const float4 v = *(const float4 *) (split_o_at(p, row, z, D) + d);
-        ls = fmaf(w, ml.y, ls);
-        acc.x = fmaf(w, v.x, acc.x);
-        acc.y = fmaf(w, v.y, acc.y);
-        acc.z = fmaf(w, v.z, acc.z);
-        acc.w = fmaf(w, v.w, acc.w);
-    }
-    const float inv = ls > 0.f ? 1.f / ls : 0.f;
-    *(float4 *) (p.out + row * D + d) = make_float4(acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv);
+    merge_split_row(p, row, D, d);
 }
 
 hipError_t launch_split_merge(const AttnParams &p, int head_dim, int cover_rows, hipStream_t stream) {
