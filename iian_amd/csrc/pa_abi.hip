@@ -63,6 +63,7 @@ constexpr int kGenPrefillWgsPerCu = 2;
 // a launch of about one round is cut into, and the most ranges per row block.
 constexpr int kSplitRoundsD256 = 3;
 constexpr int kMaxSplits = 16;
+constexpr int kOrderMinCells = 1024;     // prefill_order_entries
 constexpr int kQ8DecodeWavesPerCu = 8;
 constexpr int kMaxWavesPerCu = kQ8DecodeWavesPerCu;
 constexpr int kDefaultCus = 256;   // an MI355X, when the device cannot be queried
@@ -318,6 +319,30 @@ int prefill_splits(AttnParams &p, int head_dim, bool mixed_one_launch, int64_t m
     const size_t out_rows = (size_t) p.T * p.H;
     while (ns > 1 && split_bytes(out_rows, ns, head_dim) > room) ns--;
     return (int) std::max<int64_t>(ns, 1);
+}
+
+// Entries of the order list of a prefill launch (launch_prefill_order), 0 for a
+// launch in batch order.  A new prompt's row blocks grow from one tile to its
+// whole length, and in batch order the longest of them start last: the list
+// starts them first, for a launch of about 5 us more.  It pays when the launch
+// takes more than a round of workgroup slots and its row blocks are that
+// uneven, which the host sees when the longest prompt may make up half of the
+// longest table (H32/Hkv8/D128, new prompts: 2243 + 2552 + 752 tokens 184 ->
+// 171 us with the KV write, one of 2637 123 -> 106, one of 4096 224 -> 198, one
+// of 8192 738 -> 681; 4 of 1000 87 either way).  At D = 256 the three
+// prompts 252 -> 229, one of 8192 1055 -> 908.  Short prompts (8 of 510: 69 ->
+// 80), chunks over long contexts and windows, whose row blocks are alike, stay
+// in batch order, which keeps a sequence's row blocks together (2-6% at 8
+// chunks over 2K cells, a 1024-cell window, and 8 chunks beside 64 decodes).
+int prefill_order_entries(const AttnParams &p, int head_dim, bool mixed_one_launch, int32_t block_size, int cus) {
+    const int64_t rows = (int64_t) p.T * p.gqa, blocks = rows / kPrefillBlockRows;
+    const int64_t cells = (int64_t) p.max_blocks * block_size;
+    const int64_t slots = head_dim == 256 ? cus : 2 * cus - (mixed_one_launch ? p.sk_workers / 4 : 0);
+    const int64_t n = blocks + std::min<int64_t>(p.S, rows / (p.decode_rows + 1));
+    if (4 * blocks * p.Hkv < 5 * slots || cells < kOrderMinCells || 2 * (int64_t) p.max_q < cells ||
+        (p.n_swa > 0 && p.n_swa < cells) || p.S > kOrderMaxSeqs || n * p.Hkv >= INT32_MAX / 2)
+        return 0;
+    return (int) n;
 }
 
 // Any head size the general kernel stages (1 .. 1024; the reference's op
@@ -698,14 +723,24 @@ int run_attention(hipStream_t st, const float *q, const void *k_pool, const void
     p.n_split = 1;
     if (!decode_only) {
         const size_t cap = src.scratch ? kScratchBytes : wl.total;
-        p.n_split = prefill_splits(p, head_dim, mixed_one_launch, max_rows, block_size, cus,
-                                   cap - std::min(split_at, cap));
-        if (p.n_split > 1) need = split_at + split_bytes((size_t) n_tokens * n_head, p.n_split, head_dim_v);
+        p.n_order = prefill_order_entries(p, head_dim, mixed_one_launch, block_size, cus);
+        if (split_at + p.n_order * sizeof(int2) > cap) p.n_order = 0;
+        if (p.n_order > 0) {   // the list lies where split records would
+            need = split_at + p.n_order * sizeof(int2);
+        } else {
+            p.n_split = prefill_splits(p, head_dim, mixed_one_launch, max_rows, block_size, cus,
+                                       cap - std::min(split_at, cap));
+            if (p.n_split > 1) need = split_at + split_bytes((size_t) n_tokens * n_head, p.n_split, head_dim_v);
+        }
     }
     const int rc = ws_resolve(src, st, need, &ws);
     if (rc) return rc;
     p.split_o = (float *) (ws + split_at);
     p.split_ml = (float *) (ws + split_at + split_o_bytes((size_t) n_tokens * n_head, p.n_split, head_dim_v));
+    if (p.n_order > 0) {
+        p.order = (const int2 *) (ws + split_at);
+        if (launch_prefill_order(p, (int2 *) (ws + split_at), max_rows, st) != hipSuccess) return IIAN_PA_ERR_HIP;
+    }
     p.part_o = (float *) (ws + xl.o);
     p.part_ml = (float *) (ws + xl.ml);
     p.seg_info = (int2 *) (ws + xl.seg);

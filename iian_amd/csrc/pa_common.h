@@ -63,6 +63,9 @@ struct AttnParams {
     int32_t split_balance;      // cut for balance only: not when the batch is even (pa_prefill16_kernel)
     float *split_o;             // their records past the first: [T*H][n_split - 1][D] (the first is in `out`)
     float *split_ml;            // [T*H][n_split] of (m in log2 units, l)
+    const int2 *order;          // nullable: (sequence, row block) of the launch's prefill row blocks, most cells
+                                // first, then (-1, 0) (pa_prefill_order_kernel)
+    int32_t n_order;            // its entries
 };
 
 __device__ __forceinline__ float wave_max(float v) {

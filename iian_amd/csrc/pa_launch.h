@@ -64,11 +64,18 @@ hipError_t launch_prefill(const AttnParams &p, int head_dim, int kv_type, int ma
 // workgroups plus the decode rows' stream-K workers, which merge their split
 // segments themselves.
 hipError_t launch_mixed_f16(const AttnParams &p, int head_dim, int max_rows, hipStream_t stream);
+// How a prefill launch's workgroups map to row blocks (a template parameter of
+// both prefill kernels: a run-time branch cost the plain form 0.3-1.4%).
+enum PrefillMode { kPrefillPlain = 0, kPrefillSplit = 1, kPrefillOrdered = 2 };
 // Query rows per prefill workgroup (both prefill kernels).
 constexpr int kPrefillBlockRows = 128;
 // Merge of the split prefill row blocks (p.n_split > 1); rows past cover_rows
 // of a sequence were not attended by the launch.
 hipError_t launch_split_merge(const AttnParams &p, int head_dim, int cover_rows, hipStream_t stream);
+// Writes the order list (p.order, p.n_order entries) of a prefill launch of at
+// most kOrderMaxSeqs sequences.
+constexpr int kOrderMaxSeqs = 1024;
+hipError_t launch_prefill_order(const AttnParams &p, int2 *order, int max_rows, hipStream_t stream);
 // The 16-row-tile prefill kernel (pa_prefill16.hip), used at head size 256.
 hipError_t launch_prefill16(const AttnParams &p, int head_dim, int kv_type, int max_rows, hipStream_t stream);
 

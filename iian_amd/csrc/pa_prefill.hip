@@ -72,10 +72,12 @@ struct PrefillOcc {
 // the decode workers finish long before the prefill workgroups, so the merge
 // costs the launch nothing, and the call is one launch.
 //
-// SPLIT: row blocks cut into ranges of their tiles (split_range, pa_common.h).
-template <int D, int NW, int KVT, bool MIXED, bool SPLIT>
+// MODE (PrefillMode): row blocks in batch order, cut into ranges of their tiles
+// (split_range, pa_common.h), or in the order of a list (pa_prefill_order_kernel).
+template <int D, int NW, int KVT, bool MIXED, int MODE>
 __global__ __launch_bounds__(NW * 64, PrefillOcc<D>::kWavesPerSimd) void pa_prefill_kernel(AttnParams p, int n_rb,
                                                                                           int n_dec) {
+    constexpr bool SPLIT = MODE == kPrefillSplit;
     int bid = blockIdx.x;
     if constexpr (MIXED) {
         if (bid < n_dec) {
@@ -122,15 +124,28 @@ __global__ __launch_bounds__(NW * 64, PrefillOcc<D>::kWavesPerSimd) void pa_pref
     // 173.5-173.7 us).  Per pair, so every row block is taken once.
     // (a cut row block's ranges lie n_rb slots apart: the row blocks of one
     // range, which read the same cells, stay together)
-    const int slot = bid >> 3;
-    const int per_pair = SPLIT ? n_rb * p.n_split : n_rb;
-    const int pair_x = slot / per_pair;
-    const int pair = (bid & 7) + 8 * pair_x;
-    const int rb = (((pair_x * n_rb) / p.cus_per_xcd) & 1) ? n_rb - 1 - slot % n_rb : slot % n_rb;
-    const int z = SPLIT ? slot % per_pair / n_rb : 0;
-    if (pair >= p.S * p.Hkv) return;
-    const int s = pair / p.Hkv;
-    const int hk = pair % p.Hkv;
+    // With an order list (launches of more than one round of slots), a
+    // workgroup takes a row block's next kv head instead: the heads of a list
+    // entry go to consecutive XCDs, so with a multiple of 8 heads each head
+    // stays on its XCD, and the row blocks with the most cells start first.
+    int s, hk, rb, z = 0;
+    if constexpr (MODE == kPrefillOrdered) {
+        hk = bid % p.Hkv;
+        const int2 e = p.order[bid / p.Hkv];
+        s = __builtin_amdgcn_readfirstlane(e.x);
+        rb = __builtin_amdgcn_readfirstlane(e.y);
+        if (s < 0) return;
+    } else {
+        const int slot = bid >> 3;
+        const int per_pair = SPLIT ? n_rb * p.n_split : n_rb;
+        const int pair_x = slot / per_pair;
+        const int pair = (bid & 7) + 8 * pair_x;
+        rb = (((pair_x * n_rb) / p.cus_per_xcd) & 1) ? n_rb - 1 - slot % n_rb : slot % n_rb;
+        if (SPLIT) z = slot % per_pair / n_rb;
+        if (pair >= p.S * p.Hkv) return;
+        s = pair / p.Hkv;
+        hk = pair % p.Hkv;
+    }
 
     // wave index in a scalar register: the DMA rows, block ids and LDS
     // addresses derived from it then stay in SALU (-1.5% at the Qwen3-8B
@@ -677,23 +692,77 @@ hipError_t launch_split_merge(const AttnParams &p, int head_dim, int cover_rows,
     return hipGetLastError();
 }
 
+// The order list of a prefill launch: entry r is the row block with the r-th
+// most cells to attend, by the engine's position layout (a sequence's tokens
+// are its last cells; other positions only cost balance).  One thread per
+// list entry: it finds its row block (s, b) and counts, sequence by sequence,
+// the row blocks that come before it; a sequence's row blocks grow with b, so
+// that is one division each.  Equal ones keep batch order.
+__global__ __launch_bounds__(256) void pa_prefill_order_kernel(AttnParams p, int2 *order, int n_rb) {
+    __shared__ int nb[kOrderMaxSeqs], prior[kOrderMaxSeqs], toks[kOrderMaxSeqs];
+    for (int s = threadIdx.x; s < p.S; s += 256) {
+        const int q0 = min(max(p.qsl[s], 0), p.T);
+        const int nq = min(max(p.qsl[s + 1], q0), p.T) - q0;
+        const int M = nq * p.gqa;
+        nb[s] = M > p.decode_rows ? min(n_rb, (M + kPrefillBlockRows - 1) / kPrefillBlockRows) : 0;
+        prior[s] = max(p.seq_lens[s], nq) - nq;
+        toks[s] = nq;
+    }
+    __syncthreads();
+    const int idx = blockIdx.x * 256 + threadIdx.x;
+    if (idx >= p.n_order) return;
+    int s = 0, b = idx;
+    while (s < p.S && b >= nb[s]) b -= nb[s++];
+    if (s == p.S) {
+        order[idx] = make_int2(-1, 0);
+        return;
+    }
+    const int window = p.n_swa > 0 ? p.n_swa + kPrefillBlockRows / p.gqa + 1 : INT32_MAX;
+    const int v = min(window, prior[s] + min(toks[s], ((b + 1) * kPrefillBlockRows + p.gqa - 1) / p.gqa));
+    // row blocks of sequence j with more than c cells
+    auto above = [&](int j, int c) {
+        const int t = c - prior[j];
+        if (c >= window || toks[j] <= t) return 0;
+        return max(0, nb[j] - (t < 0 ? 0 : (int) ((int64_t) t * p.gqa / kPrefillBlockRows)));
+    };
+    int rank = 0;
+    for (int j = 0; j < s; j++) rank += above(j, v - 1);
+    rank += above(s, v) + b - (nb[s] - above(s, v - 1));
+    for (int j = s + 1; j < p.S; j++) rank += above(j, v);
+    order[rank] = make_int2(s, b);
+}
+
+hipError_t launch_prefill_order(const AttnParams &p, int2 *order, int max_rows, hipStream_t stream) {
+    if (p.S > kOrderMaxSeqs || p.n_order <= 0) return hipErrorInvalidValue;
+    const int n_rb = (max_rows + kPrefillBlockRows - 1) / kPrefillBlockRows;
+    hipLaunchKernelGGL(pa_prefill_order_kernel, dim3((p.n_order + 255) / 256), dim3(256), 0, stream, p, order, n_rb);
+    return hipGetLastError();
+}
+
 template <int D, int NW, int KVT, bool MIXED>
 static hipError_t launch_prefill_t(const AttnParams &p, int max_rows, hipStream_t stream) {
     constexpr int ROWS = NW * 32;
     const int n_rb = (max_rows + ROWS - 1) / ROWS;
     const int pairs_per_xcd = (p.S * p.Hkv + 7) / 8;
     static_assert(ROWS == kPrefillBlockRows, "the host plans 128-row blocks");
-    const int64_t n_pf = 8 * (int64_t) pairs_per_xcd * n_rb * std::max(1, p.n_split);
+    const int64_t n_pf = p.order ? (int64_t) p.n_order * p.Hkv
+                                 : 8 * (int64_t) pairs_per_xcd * n_rb * std::max(1, p.n_split);
     const int64_t n_dec = MIXED ? ((p.sk_workers + NW - 1) / NW + 7) / 8 * 8 : 0;
     const int64_t nwg = n_dec + n_pf;
     if (nwg > INT32_MAX) return hipErrorInvalidValue;
     const dim3 grid((unsigned) nwg), block(NW * 64);
     if (p.n_split > 1) {
-        hipLaunchKernelGGL((pa_prefill_kernel<D, NW, KVT, MIXED, true>), grid, block, 0, stream, p, n_rb, (int) n_dec);
+        hipLaunchKernelGGL((pa_prefill_kernel<D, NW, KVT, MIXED, kPrefillSplit>), grid, block, 0, stream, p, n_rb,
+                           (int) n_dec);
         const hipError_t e = hipGetLastError();
         return e != hipSuccess ? e : launch_split_merge(p, D, n_rb * ROWS, stream);
     }
-    hipLaunchKernelGGL((pa_prefill_kernel<D, NW, KVT, MIXED, false>), grid, block, 0, stream, p, n_rb, (int) n_dec);
+    if (p.order)
+        hipLaunchKernelGGL((pa_prefill_kernel<D, NW, KVT, MIXED, kPrefillOrdered>), grid, block, 0, stream, p, n_rb,
+                           (int) n_dec);
+    else
+        hipLaunchKernelGGL((pa_prefill_kernel<D, NW, KVT, MIXED, kPrefillPlain>), grid, block, 0, stream, p, n_rb,
+                           (int) n_dec);
     return hipGetLastError();
 }
 

@@ -70,12 +70,14 @@ __device__ __forceinline__ f16x8 lds_tr_b16x8_16(const char *p0, const char *p1)
 // values in f16 plus the block scales d as f32 in LDS, applied per cell after
 // each QK^T k-step MFMA (k-step = block), so q*d enters the scores exactly;
 // V as f16(q*d), the correctly rounded dequantised value.
-// SPLIT: row blocks cut into ranges of their tiles (split_range, pa_common.h).
-template <int D, int NRT, int NW, int KVT, bool SPLIT>
+// MODE (PrefillMode): row blocks in batch order, cut into ranges of their tiles
+// (split_range, pa_common.h), or in the order of a list (pa_prefill.hip).
+template <int D, int NRT, int NW, int KVT, int MODE>
 // Waves per SIMD asked of the register allocator: four for f16 at D = 128 (two
 // 8-wave workgroups per CU in 128 VGPRs), else two up to D = 128, one at 256.
 __global__ __launch_bounds__(NW * 64, (D == 128 && KVT == 1) ? 4 : (D <= 128 ? 2 : 1)) void pa_prefill16_kernel(
     AttnParams p, int n_rb) {
+    constexpr bool SPLIT = MODE == kPrefillSplit, ordered = MODE == kPrefillOrdered;
     using SH = PrefillShape16<D>;
     constexpr int KS = SH::KS, NPV = SH::NPV, KSTRIDE = SH::KSTRIDE, VSTRIDE = SH::VSTRIDE;
     constexpr bool Q8 = KVT == 8;
@@ -100,8 +102,9 @@ __global__ __launch_bounds__(NW * 64, (D == 128 && KVT == 1) ? 4 : (D <= 128 ? 2
     // range, which read the same cells, stay together)
     const int per_pair = SPLIT ? n_rb * p.n_split : n_rb;
     const int pair = (bid & 7) + 8 * (slot / per_pair);
-    const int rb = slot % n_rb, z = SPLIT ? slot % per_pair / n_rb : 0;
-    if (pair >= p.S * p.Hkv) return;
+    int rb = slot % n_rb;
+    const int z = SPLIT ? slot % per_pair / n_rb : 0;
+    if (!ordered && pair >= p.S * p.Hkv) return;
 
     // wave index in a scalar register, so that the tile-load rows derived from
     // it stay in SALU (cfg5 global prefill 4947-5022 against 5015-5085 us)
@@ -115,10 +118,16 @@ __global__ __launch_bounds__(NW * 64, (D == 128 && KVT == 1) ? 4 : (D <= 128 ? 2
     // 64 sequences; past that, and with a window, which bounds every row
     // block's cells, the batch order stands: the ranking's round trip and
     // shuffles cost the window-bounded prefill 2-3%).
-    const int hk = pair % p.Hkv;
+    const int hk = ordered ? bid % p.Hkv : pair % p.Hkv;
     int s = pair / p.Hkv, L, q0, nq;
+    if (ordered) {
+        const int2 e = p.order[bid / p.Hkv];
+        s = __builtin_amdgcn_readfirstlane(e.x);
+        rb = __builtin_amdgcn_readfirstlane(e.y);
+        if (s < 0) return;
+    }
     int n_split = SPLIT ? p.n_split : 1;   // ranges a row block may be cut into
-    if (p.S <= 64 && p.n_swa <= 0) {
+    if (p.S <= 64 && p.n_swa <= 0 && !ordered) {
         int ll = 0, a = 0, nql = 0, key = -1;
         if (lane < p.S) {
             ll = p.seq_lens[lane];
@@ -508,15 +517,17 @@ static hipError_t launch_prefill16_t(const AttnParams &p, int max_rows, hipStrea
     constexpr int ROWS = NW * NRT * 16;
     const int n_rb = (max_rows + ROWS - 1) / ROWS;
     const int pairs_per_xcd = (p.S * p.Hkv + 7) / 8;
-    const int64_t nwg = 8 * (int64_t) pairs_per_xcd * n_rb * std::max(1, p.n_split);
+    const int64_t nwg = p.order ? (int64_t) p.n_order * p.Hkv
+                                : 8 * (int64_t) pairs_per_xcd * n_rb * std::max(1, p.n_split);
     if (nwg > INT32_MAX) return hipErrorInvalidValue;
     const dim3 grid((unsigned) nwg), block(NW * 64);
     if (p.n_split > 1) {
-        hipLaunchKernelGGL((pa_prefill16_kernel<D, NRT, NW, KVT, true>), grid, block, 0, stream, p, n_rb);
+        hipLaunchKernelGGL((pa_prefill16_kernel<D, NRT, NW, KVT, kPrefillSplit>), grid, block, 0, stream, p, n_rb);
         const hipError_t e = hipGetLastError();
         return e != hipSuccess ? e : launch_split_merge(p, D, n_rb * ROWS, stream);
     }
-    hipLaunchKernelGGL((pa_prefill16_kernel<D, NRT, NW, KVT, false>), grid, block, 0, stream, p, n_rb);
+    if (p.order) hipLaunchKernelGGL((pa_prefill16_kernel<D, NRT, NW, KVT, kPrefillOrdered>), grid, block, 0, stream, p, n_rb);
+    else hipLaunchKernelGGL((pa_prefill16_kernel<D, NRT, NW, KVT, kPrefillPlain>), grid, block, 0, stream, p, n_rb);
     return hipGetLastError();
 }
 
