@@ -134,7 +134,8 @@ __global__ __launch_bounds__(NW * 64, PrefillOcc<D>::kWavesPerSimd) void pa_pref
         const int2 e = p.order[bid / p.Hkv];
         s = __builtin_amdgcn_readfirstlane(e.x);
         rb = __builtin_amdgcn_readfirstlane(e.y);
-        if (s < 0) return;
+        // (past the list; or unwritten, where query_start_loc's ranges overlap)
+        if ((uint32_t) s >= (uint32_t) p.S || (uint32_t) rb >= (uint32_t) n_rb) return;
     } else {
         const int slot = bid >> 3;
         const int per_pair = SPLIT ? n_rb * p.n_split : n_rb;
@@ -729,7 +730,8 @@ __global__ __launch_bounds__(256) void pa_prefill_order_kernel(AttnParams p, int
     for (int j = 0; j < s; j++) rank += above(j, v - 1);
     rank += above(s, v) + b - (nb[s] - above(s, v - 1));
     for (int j = s + 1; j < p.S; j++) rank += above(j, v);
-    order[rank] = make_int2(s, b);
+    // overlapping query_start_loc ranges hold more row blocks than n_order
+    if (rank < p.n_order) order[rank] = make_int2(s, b);
 }
 
 hipError_t launch_prefill_order(const AttnParams &p, int2 *order, int max_rows, hipStream_t stream) {

@@ -124,7 +124,8 @@ __global__ __launch_bounds__(NW * 64, (D == 128 && KVT == 1) ? 4 : (D <= 128 ? 2
         const int2 e = p.order[bid / p.Hkv];
         s = __builtin_amdgcn_readfirstlane(e.x);
         rb = __builtin_amdgcn_readfirstlane(e.y);
-        if (s < 0) return;
+        // (past the list; or unwritten, where query_start_loc's ranges overlap)
+        if ((uint32_t) s >= (uint32_t) p.S || (uint32_t) rb >= (uint32_t) n_rb) return;
     }
     int n_split = SPLIT ? p.n_split : 1;   // ranges a row block may be cut into
     if (p.S <= 64 && p.n_swa <= 0 && !ordered) {
