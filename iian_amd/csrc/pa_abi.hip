@@ -60,9 +60,8 @@ constexpr int kGenDecodeWavesPerCuWide = 4;
 constexpr int kGenPrefillWgsPerCuF16 = 1;
 constexpr int kGenPrefillWgsPerCu = 2;
 // Split prefill row blocks (prefill_splits): the rounds of D = 256 workgroups
-// a launch of about one round is cut into, and the most ranges per row block.
+// a launch of about one round is cut into.
 constexpr int kSplitRoundsD256 = 3;
-constexpr int kMaxSplits = 16;
 constexpr int kOrderMinCells = 1024;     // prefill_order_entries
 constexpr int kQ8DecodeWavesPerCu = 8;
 constexpr int kMaxWavesPerCu = kQ8DecodeWavesPerCu;
@@ -535,7 +534,7 @@ int run_attention(hipStream_t st, const float *q, const void *k_pool, const void
             const int64_t max_tiles = ((int64_t) max_blocks * block_size + kTile - 1) / kTile;
             const bool f16 = type_k == IIAN_PA_TYPE_F16 && type_v == IIAN_PA_TYPE_F16;
             int64_t ns = ((int64_t) (f16 ? kGenPrefillWgsPerCuF16 : kGenPrefillWgsPerCu) * cus + full - 1) / full;
-            ns = std::min<int64_t>({ns, std::max<int64_t>(1, max_tiles / 8), 16});
+            ns = std::min<int64_t>({ns, std::max<int64_t>(1, max_tiles / 8), kMaxSplits});
             const size_t out_rows = (size_t) n_tokens * n_head;
             split_at = align256(xl.total);
             const size_t room = cap - std::min(split_at, cap);

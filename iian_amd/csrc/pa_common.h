@@ -247,6 +247,7 @@ __device__ __forceinline__ float *rec_ml(const AttnParams &p, int rec, int hr, i
 // n_split.  A row block of up to kSplitMinCells cells is never cut, so its rows do
 // not depend on the batch or on how the launch was planned.
 constexpr int kSplitMinCells = 1024;
+constexpr int kMaxSplits = 16;   // p.n_split at most: a row's (m, l) pairs fit the lanes of split_merge_rows
 
 struct SplitRange {
     int n;        // ranges of this row block

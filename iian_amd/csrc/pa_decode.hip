@@ -34,6 +34,8 @@
 #include "pa_decode_body.h"
 #include "pa_merge.h"
 
+#include <algorithm>
+
 namespace iian_pa {
 
 // 1.5 waves per SIMD are launched at D <= 128 (kF16DecodeWaves in pa_abi.hip),
@@ -54,7 +56,7 @@ __global__ __launch_bounds__(64, (D * NRT <= 128) ? 2 : 1) void pa_decode_f16_ke
 // WPR = 1: one workgroup per (sequence, kv head or head group), wave i merging
 // rows i, i+4, ...  WPR = 4: one workgroup per row, blockIdx.z, whose 4 waves
 // share its records, for calls with few segments and so many records in each.
-template <int WPR>
+template <int WPR, int LPR>
 __global__ __launch_bounds__(256) void pa_merge_kernel(AttnParams p, int D) {
     __shared__ __attribute__((aligned(16))) float comb[WPR > 1 ? 4 * 258 : 4];
     // blockIdx.y: the kv head, or the head group of head_group kv heads
@@ -72,30 +74,39 @@ __global__ __launch_bounds__(256) void pa_merge_kernel(AttnParams p, int D) {
     if ((nq <= 0) | (M > p.decode_rows) | (info.y <= 1)) return;
     const int hr = grouped ? hg : 0;
     const int rows = M * p.head_group;
-    for (int r = WPR > 1 ? (int) blockIdx.z : (int) (threadIdx.x >> 6); r < rows; r += WPR > 1 ? rows : 4) {
+    for (int r = WPR > 1 ? (int) blockIdx.z : (int) (threadIdx.x >> 6); r < rows; r += WPR > 1 ? (int) gridDim.z : 4) {
+        if (WPR > 1) __syncthreads();   // the row before it has left comb
         const int hl = r / M, rh = r - hl * M;
         const int t = q0 + rh / p.gqa, h = (hg * p.head_group + hl) * p.gqa + rh % p.gqa;
-        merge_row<WPR>(rec_o(p, info.x, hr, r, D), p.rec_stride, rec_ml(p, info.x, hr, r),
-                       2 * (int64_t) p.rec_heads * p.rec_rows, info.y, D, p.out + ((int64_t) t * p.H + h) * D, comb);
+        merge_row<WPR, LPR>(rec_o(p, info.x, hr, r, D), p.rec_stride, rec_ml(p, info.x, hr, r),
+                            2 * (int64_t) p.rec_heads * p.rec_rows, info.y, D, p.out + ((int64_t) t * p.H + h) * D,
+                            comb);
     }
 }
 
-// A workgroup per row where the call has at most one segment per 8 stream-K
-// workers, and so 8 records or more per segment on average: merge_row's batch
+// A workgroup per row where the call has at most one segment per 12 stream-K
+// workers, and so 12 records or more per segment on average: merge_row's batch
 // covers 8 records of a row with one wave, 32 with four.  Measured at H32/Hkv8/
 // D128 f16, whole calls (before: one wave per row, 8 records a batch, at any
-// count): 2 sequences of 26K-30K cells 57.8 -> 53.4 us (the merge 10.2 -> 5.8),
-// 4 of 512-8192 cells 22.7 -> 19.2, 16 37.9 -> 37.6 (38.5 with a wave per row),
-// 24 and more unchanged; 4 Q8_0 spec-verify sequences of 4K 40.6 -> 28.9 us.
+// count): 2 sequences of 26K-30K cells 57.8 -> 52.6 us (the merge 10.2 -> 5.5),
+// 4 of 512-8192 cells 22.7 -> 19.2, 16 37.9 -> 37.6 (38.5 with a wave per row);
+// 4 Q8_0 spec-verify sequences of 4K 40.6 -> 28.9 us.  Beyond it the
+// workgroups cost more than the shorter chain gives (Q8_0 decodes of 2000
+// cells: 16 sequences 30.0 -> 29.8 us, 24 35.1 -> 35.4, 32 46.9 -> 47.5).
 hipError_t launch_merge(const AttnParams &p, int head_dim, hipStream_t stream) {
     if (head_dim % 4 || head_dim > 256) return hipErrorInvalidValue;
     const int groups = p.Hkv / p.head_group;
     const int64_t segs = p.rec_heads > 1 ? p.S : (int64_t) p.S * groups;
     const dim3 block(256);
-    if (segs * 8 <= p.sk_workers)
-        hipLaunchKernelGGL(pa_merge_kernel<4>, dim3(p.S, groups, p.rec_rows), block, 0, stream, p, head_dim);
-    else
-        hipLaunchKernelGGL(pa_merge_kernel<1>, dim3(p.S, groups), block, 0, stream, p, head_dim);
+    const int lpr = merge_lpr(head_dim);
+    if (segs * 12 <= p.sk_workers) {
+        const int rows = (int) std::min<int64_t>(p.rec_rows, (int64_t) p.max_q * p.gqa * p.head_group);
+        const auto kernel = lpr == 16 ? pa_merge_kernel<4, 16> : lpr == 32 ? pa_merge_kernel<4, 32> : pa_merge_kernel<4, 64>;
+        hipLaunchKernelGGL(kernel, dim3(p.S, groups, std::max(rows, 1)), block, 0, stream, p, head_dim);
+    } else {
+        const auto kernel = lpr == 16 ? pa_merge_kernel<1, 16> : lpr == 32 ? pa_merge_kernel<1, 32> : pa_merge_kernel<1, 64>;
+        hipLaunchKernelGGL(kernel, dim3(p.S, groups), block, 0, stream, p, head_dim);
+    }
     return hipGetLastError();
 }
 

@@ -10,8 +10,8 @@ namespace iian_pa {
 // the decode segments: WPR = 1, a workgroup per segment and a wave per row;
 // WPR = 4, a workgroup per row, its waves sharing the row's records (chosen
 // when the call has few segments, whose records are then many).  The rest take
-// the split prefill rows, a wave each.
-template <int WPR>
+// the split prefill rows.
+template <int WPR, int LPR>
 __global__ __launch_bounds__(256) void pa_gen_merge_kernel(GenMfmaParams p, int n_seg_wgs, int seg_rows) {
     __shared__ __attribute__((aligned(16))) float comb[WPR > 1 ? 4 * 258 : 4];
     const AttnParams &a = p.a;
@@ -27,23 +27,12 @@ __global__ __launch_bounds__(256) void pa_gen_merge_kernel(GenMfmaParams p, int 
         // (WPR = 4: one row per workgroup, so its barrier is met once)
         for (int r = WPR > 1 ? blockIdx.x % seg_rows : wave; r < M; r += WPR > 1 ? kGmRows : 4) {
             const int64_t orow = (int64_t) (q0 + r / a.gqa) * a.H + hk * a.gqa + r % a.gqa;
-            merge_row<WPR>(rec_o(a, info.x, 0, r, p.Dv), a.rec_stride, rec_ml(a, info.x, 0, r), 2 * (int64_t) a.rec_rows,
-                           info.y, p.Dv, a.out + orow * p.Dv, comb);
+            merge_row<WPR, LPR>(rec_o(a, info.x, 0, r, p.Dv), a.rec_stride, rec_ml(a, info.x, 0, r),
+                                2 * (int64_t) a.rec_rows, info.y, p.Dv, a.out + orow * p.Dv, comb);
         }
         return;
     }
-    const int64_t row = (int64_t) (blockIdx.x - n_seg_wgs) * 4 + wave;
-    if (row >= (int64_t) a.T * a.H) return;
-    const int t = (int) (row / a.H);
-    int lo = 0, hi = a.S - 1;   // the last s with qsl[s] <= t
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (a.qsl[mid] <= t) lo = mid; else hi = mid - 1;
-    }
-    const int q0 = min(max(a.qsl[lo], 0), a.T), nq = min(max(a.qsl[lo + 1], q0), a.T) - q0;
-    // rows of a decode sequence, and of none, have no split records
-    if (t < q0 || t >= q0 + nq || (int64_t) nq * a.gqa <= a.decode_rows) return;
-    merge_split_row(a, row, p.Dv, 4 * (threadIdx.x & 63));
+    split_merge_rows<LPR>(a, ((int64_t) (blockIdx.x - n_seg_wgs) * 4 + wave) * (64 / LPR), p.Dv, INT32_MAX);
 }
 
 hipError_t launch_gen_mfma(const GenMfmaParams &params, int type_k, int type_v, int64_t n_prefill_wgs,
@@ -56,7 +45,10 @@ hipError_t launch_gen_mfma(const GenMfmaParams &params, int type_k, int type_v, 
     const bool wide = seg * 16 <= p.a.sk_workers;
     const int seg_rows = (int) std::min<int64_t>(kGmRows, (int64_t) p.a.max_q * p.a.gqa);
     const int64_t seg_wgs = wide ? seg * seg_rows : seg;
-    const int64_t row_wgs = n_prefill_wgs && p.a.n_split > 1 ? ((int64_t) p.a.T * p.a.H + 3) / 4 : 0;
+    const int lpr = merge_lpr(p.Dv), rows_per_wg = 4 * (64 / lpr);
+    const int64_t row_wgs =
+        n_prefill_wgs && p.a.n_split > 1 ? ((int64_t) p.a.T * p.a.H + rows_per_wg - 1) / rows_per_wg : 0;
+    if (p.a.n_split > kMaxSplits) return hipErrorInvalidValue;
     if (wgs <= 0 || wgs > INT32_MAX || seg_wgs + row_wgs > INT32_MAX) return hipErrorInvalidValue;
     hipError_t e;
     switch (type_k) {
@@ -67,8 +59,13 @@ hipError_t launch_gen_mfma(const GenMfmaParams &params, int type_k, int type_v, 
     }
     if (e != hipSuccess || seg_wgs + row_wgs == 0) return e;
     const dim3 grid((unsigned) (seg_wgs + row_wgs));
-    if (wide) hipLaunchKernelGGL(pa_gen_merge_kernel<4>, grid, dim3(256), 0, stream, p, (int) seg_wgs, seg_rows);
-    else hipLaunchKernelGGL(pa_gen_merge_kernel<1>, grid, dim3(256), 0, stream, p, (int) seg_wgs, seg_rows);
+    const auto kernel = wide ? (lpr == 16   ? pa_gen_merge_kernel<4, 16>
+                                : lpr == 32 ? pa_gen_merge_kernel<4, 32>
+                                            : pa_gen_merge_kernel<4, 64>)
+                             : (lpr == 16   ? pa_gen_merge_kernel<1, 16>
+                                : lpr == 32 ? pa_gen_merge_kernel<1, 32>
+                                            : pa_gen_merge_kernel<1, 64>);
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, p, (int) seg_wgs, seg_rows);
     return hipGetLastError();
 }
 

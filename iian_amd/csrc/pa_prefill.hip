@@ -662,34 +662,22 @@ __global__ __launch_bounds__(NW * 64, PrefillOcc<D>::kWavesPerSimd) void pa_pref
     }
 }
 
-// The split row blocks' merge (merge_split_row).  One round trip of (m, l) and one of the O rows; a lane holds 4
-// dims, so a row takes lpr = 16, 32 or 64 lanes and a wave 64 / lpr rows.  Rows
-// the launch did not cover (past cover_rows of a sequence) are left alone.
-__global__ __launch_bounds__(256) void pa_split_merge_kernel(AttnParams p, int D, int lpr, int cover_rows) {
-    const int lane = threadIdx.x & 63, sub = lane / lpr, d = 4 * (lane & (lpr - 1));
-    const int64_t row = ((int64_t) blockIdx.x * 4 + (threadIdx.x >> 6)) * (64 / lpr) + sub;
-    if (row >= (int64_t) p.T * p.H) return;
-    // an uncut row block wrote the finished row (looked at first: rows the
-    // launch did not cover hold anything here, and are left alone below)
-    if (split_ml_at(p, row, 0)->y < 0.f) return;
-    const int t = (int) (row / p.H), h = (int) (row - (int64_t) t * p.H);
-    int lo = 0, hi = p.S - 1;   // the last s with qsl[s] <= t
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (p.qsl[mid] <= t) lo = mid; else hi = mid - 1;
-    }
-    const int q0 = min(max(p.qsl[lo], 0), p.T), nq = min(max(p.qsl[lo + 1], q0), p.T) - q0;
-    if (t < q0 || t >= q0 + nq || nq * p.gqa <= p.decode_rows || (t - q0) * p.gqa + h % p.gqa >= cover_rows) return;
-    merge_split_row(p, row, D, d);
+// The split row blocks' merge.
+template <int LPR>
+__global__ __launch_bounds__(256) void pa_split_merge_kernel(AttnParams p, int D, int cover_rows) {
+    split_merge_rows<LPR>(p, ((int64_t) blockIdx.x * 4 + (threadIdx.x >> 6)) * (64 / LPR), D, cover_rows);
 }
 
 hipError_t launch_split_merge(const AttnParams &p, int head_dim, int cover_rows, hipStream_t stream) {
-    const int lpr = head_dim <= 64 ? 16 : head_dim <= 128 ? 32 : 64;
-    if (head_dim % 4 || head_dim > 256) return hipErrorInvalidValue;
+    const int lpr = merge_lpr(head_dim);
+    if (head_dim % 4 || head_dim > 256 || p.n_split > kMaxSplits) return hipErrorInvalidValue;
     const int64_t rows_per_wg = 4 * (64 / lpr);
     const int64_t wgs = ((int64_t) p.T * p.H + rows_per_wg - 1) / rows_per_wg;
     if (wgs > INT32_MAX) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(pa_split_merge_kernel, dim3((unsigned) wgs), dim3(256), 0, stream, p, head_dim, lpr, cover_rows);
+    const auto kernel = lpr == 16   ? pa_split_merge_kernel<16>
+                        : lpr == 32 ? pa_split_merge_kernel<32>
+                                    : pa_split_merge_kernel<64>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned) wgs), dim3(256), 0, stream, p, head_dim, cover_rows);
     return hipGetLastError();
 }
 

@@ -8,7 +8,7 @@ import numpy as np
 import pytest
 import torch
 
-from helpers import F16, Q8_0, make_case, row_rel_err
+from helpers import F16, F32, Q8_0, make_case, row_rel_err
 from test_gpu_parity import TOL, banner, gpu_attention, oracle_attention, to_device
 
 pytestmark = pytest.mark.gpu
@@ -55,6 +55,25 @@ def test_split_prefill_matches_oracle(pa, oracle, name):
     print(f"[gpu] {name}: max row rel err {e.max():.3e}", flush=True)
     assert int(err.item()) == 0 and np.isfinite(got).all()
     assert e.max() <= TOL, (name, e.max())
+
+
+@pytest.mark.parametrize("S", [1, 2, 62, 63, 64, 90])
+@pytest.mark.parametrize("H,Hkv,D,k_type", [(8, 2, 64, F16), (5, 1, 128, F16), (4, 2, 256, F16), (7, 7, 80, F16),
+                                            (5, 5, 96, F32)])
+def test_split_rows_among_many_sequences(pa, oracle, S, H, Hkv, D, k_type):
+    """The merge finds each row's sequence in one read below 64 sequences and
+    by bisection from there: chunks first, last and in the middle of decodes
+    and empty sequences, row counts that leave the last wave partly idle."""
+    banner(f"split prefill S={S} H={H} D={D} type {k_type}")
+    rng = np.random.default_rng(S * 1000 + D)
+    lens, nq = [int(x) for x in rng.integers(5, 70, S)], [int(x) for x in rng.integers(0, 2, S)]
+    for s in sorted({0, S // 2, S - 1}):
+        lens[s], nq[s] = int(rng.integers(2100, 3300)), int(rng.integers(33, 60))
+    c = make_case(rng, H, Hkv, D, lens, nq, k_type=k_type, v_type=k_type)
+    err = torch.zeros(1, dtype=torch.int32, device="cuda")
+    got = gpu_attention(pa, c, err)
+    assert int(err.item()) == 0 and np.isfinite(got).all()
+    assert row_rel_err(got, oracle_attention(oracle, c)).max() <= (2e-5 if D in (80, 96) else TOL)
 
 
 @pytest.mark.parametrize("k_type,D", [(F16, 128), (F16, 256), (Q8_0, 128)])
