@@ -18,15 +18,16 @@ inline int merge_lpr(int dv) { return dv <= 64 ? 16 : dv <= 128 ? 32 : 64; }
 //
 // Bound by dependent round trips, not by bytes: a lane takes 4 dims, so a
 // record's row fills LPR = 16, 32 or 64 lanes and a wave holds 64/LPR records
-// side by side, four such groups in flight per batch.  LPR (merge_lpr) is a
+// side by side, several such groups in flight per batch: 8 records with one
+// wave per row, whose segments have few (16 at D = 64 cost 64 Q8_0 verify
+// sequences of 5 tokens 49.0 -> 49.9 us a call), four groups with four.  LPR (merge_lpr) is a
 // template parameter: with run-time loops a merge took 0.1-0.8 us longer (2
 // sequences of 26K-30K cells, whole call, 53.3 against 52.6 us).
 template <int WPR, int LPR>
 __device__ __forceinline__ void merge_row(const float *o0, int64_t o_stride, const float *ml0, int64_t ml_stride,
                                           int np, int dv, float *out, float *comb) {
-    constexpr int U = 4;
+    constexpr int rpw = 64 / LPR, U = WPR > 1 ? 4 : 8 / rpw;
     const int lane = threadIdx.x & 63, wave = WPR > 1 ? (int) (threadIdx.x >> 6) : 0;
-    constexpr int rpw = 64 / LPR;
     const int sub = lane / LPR, d = 4 * (lane & (LPR - 1));
     const bool live = d < dv;
     constexpr int step = WPR * rpw;
