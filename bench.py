@@ -33,7 +33,7 @@ WORKLOADS = {
     "cfg1": "Qwen2.5-0.5B paged decode, H14/Hkv2/D64, 8 seqs, ctx U[64,1024], 1024-block f16 pool",
     "cfg2": "Llama-3-8B paged decode, H32/Hkv8/D128, 64 seqs, ctx log-uniform [512,8192], "
             "16-token f16 blocks in a 65536-block pool, + KV write of 64 tokens",
-    "cfg2_f32": "Llama-3-8B paged decode as cfg2 with F32 K/V pools (the general fp32 kernel), + KV write "
+    "cfg2_f32": "Llama-3-8B paged decode as cfg2 with F32 K/V pools (the matrix-core general kernel), + KV write "
                 "of 64 tokens",
     "cfg3": "Qwen3-8B mixed batch, H32/Hkv8/D128: 4 prefill chunks x 512 over prior U[1024,4096] "
             "(1024-token shared prefix) + 32 decode tokens, f16 KV",
@@ -73,7 +73,7 @@ def launch_kernels(sp, pa, max_blocks: int, block_size: int, cus: int) -> str:
         return "pa_decode_f16_kernel<96> + pa_merge_kernel<96>"
     if (sp.D not in (64, 96, 128, 256) or (sp.D == 96 and sp.kv_type != pa.GGML_TYPE_F16)
             or sp.kv_type not in (pa.GGML_TYPE_F16, pa.GGML_TYPE_Q8_0)):
-        return "pa_general_kernel + pa_general_merge_kernel"
+        return "pa_gen_mfma_kernel + pa_gen_merge_kernel"
     has_dec = any(0 < r <= 32 for r in rows)
     has_pf = any(r > 32 for r in rows)
     d = sp.D
