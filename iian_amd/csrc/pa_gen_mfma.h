@@ -197,8 +197,9 @@ __device__ __forceinline__ void gm_piece(const GenMfmaParams &p, const GmPiece &
     constexpr bool KF16 = KT == 1, VF16 = VT == 1;
     constexpr int NT = VF16 ? 2 : 1;       // 16-cell steps per tile: the f16 PV wants 32 cells per MFMA
     constexpr int TC = 16 * NT, CV = 4 * NT;   // cells per tile, and V cells per lane
-    // D > 32 (NK - 1) and Dv > 64 (NV - 1) except in the wide kernels (NK = 8,
-    // D > 128), whose later chunks and blocks are skipped when past the size
+    // D > 32 (NK - 1) except in the wide kernels (NK = 8, D > 128), whose later
+    // chunks are skipped when past D, as their V blocks are when past Dv (no
+    // kernel has a lower limit on Dv: gm_v_offset)
     constexpr int JOPT = NK == 8 ? 4 : NK, BOPT = NK == 8 ? 1 : NV;
     const int lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15;
     const int D = p.D, Dv = p.Dv;
@@ -305,13 +306,11 @@ __device__ __forceinline__ void gm_piece(const GenMfmaParams &p, const GmPiece &
     // lane offsets inside a row: K dims 8g of chunk 0 and of the last chunk
     // (lanes past D reread its last 8 dims, and their K is taken as zero)
     const int kd_last = min(32 * (NK - 1) + 8 * g, D - 8);
-    const uint32_t k_lane = KT == 8 ? pc.hk * (D / 32) * 34 + 2 + 8 * g : (pc.hk * D + 8 * g) * KE;
-    const uint32_t k_last = KT == 8 ? 0 : (pc.hk * D + kd_last) * KE;
+    const uint32_t k_lane = gm_k_offset(KT, pc.hk, D, 0, g);
+    const uint32_t k_last = KT == 8 ? 0 : gm_k_offset(KT, pc.hk, D, NK - 1, g);
     // V dims 4n of block 0 and of the last block (columns past Dv are never stored)
     const int vd_last = min(64 * (NV - 1) + 4 * n, Dv - 4);
-    const uint32_t v_head = VT == 8 ? pc.hk * (Dv / 32) * 34 : pc.hk * Dv * VE;
-    const uint32_t v_lane = VT == 8 ? v_head + 34 * (n >> 3) : v_head + 4 * n * VE;
-    const uint32_t v_last = VT == 8 ? v_head + 34 * (vd_last >> 5) : v_head + vd_last * VE;
+    const uint32_t v_lane = gm_v_offset(VT, pc.hk, Dv, 0, n), v_last = gm_v_offset(VT, pc.hk, Dv, NV - 1, n);
     auto load_k = [&](const Step (&st)[NT]) {
 #pragma unroll
         for (int t = 0; t < NT; t++) {
@@ -329,7 +328,7 @@ __device__ __forceinline__ void gm_piece(const GenMfmaParams &p, const GmPiece &
                     const bool edge = j == NK - 1 && JOPT == NK;
                     const uint32_t off = edge ? c + k_last : c + k_lane + 32 * j * KE;
                     if constexpr (JOPT < NK) {   // wide kernels: any chunk may be the last
-                        const uint32_t o2 = j >= JOPT ? c + (pc.hk * D + min(32 * j + 8 * g, D - 8)) * KE : off;
+                        const uint32_t o2 = j >= JOPT ? c + gm_k_offset(KT, pc.hk, D, j, g) : off;
                         kr[t][j].a = gm_ld<u32x4>(base, o2);
                         if constexpr (KT == 0) kr[t][j].b = gm_ld<u32x4>(base, o2 + 16);
                     } else {
@@ -351,16 +350,11 @@ __device__ __forceinline__ void gm_piece(const GenMfmaParams &p, const GmPiece &
                 for (int b = 0; b < NV; b++) {
                     GmV<VT> &v = vr[4 * t + i][b];
                     if (b >= BOPT && 64 * b >= Dv) continue;   // wave-uniform
+                    const uint32_t off = c + (b == 0 ? v_lane : b == NV - 1 ? v_last : gm_v_offset(VT, pc.hk, Dv, b, n));
                     if constexpr (VT == 8) {
-                        const int vd = min(64 * b + 4 * n, Dv - 4);
-                        const uint32_t off = b == NV - 1 ? c + v_last
-                                             : BOPT < NV ? c + v_head + 34 * (vd >> 5) : c + v_lane + 68 * b;
                         v.d = gm_ld<uint16_t>(base, off);
                         v.x = gm_ld<u32_a2>(base, off + 2 + ((4 * n) & 31)).x;
                     } else {
-                        const uint32_t off = b == NV - 1 ? c + v_last
-                                             : BOPT < NV ? c + v_head + min(64 * b + 4 * n, Dv - 4) * VE
-                                                         : c + v_lane + 64 * b * VE;
                         if constexpr (VT == 0) v.a = gm_ld<u32x4>(base, off);
                         else v.a = gm_ld<u32x2>(base, off);
                     }
@@ -870,10 +864,10 @@ static hipError_t launch_gen_mfma_n(const GenMfmaParams &p, unsigned wgs, hipStr
 template <int KT, int VT>
 static hipError_t launch_gen_mfma_v(const GenMfmaParams &p, unsigned wgs, hipStream_t stream) {
     switch (gen_mfma_chunks(p.D, p.Dv)) {
-        case 2: return launch_gen_mfma_n<KT, VT, 2, 1>(p, wgs, stream);
-        case 3: return launch_gen_mfma_n<KT, VT, 3, 2>(p, wgs, stream);
-        case 4: return launch_gen_mfma_n<KT, VT, 4, 2>(p, wgs, stream);
-        case 8: return launch_gen_mfma_n<KT, VT, 8, 4>(p, wgs, stream);
+        case 2: return launch_gen_mfma_n<KT, VT, 2, gen_mfma_blocks(2)>(p, wgs, stream);
+        case 3: return launch_gen_mfma_n<KT, VT, 3, gen_mfma_blocks(3)>(p, wgs, stream);
+        case 4: return launch_gen_mfma_n<KT, VT, 4, gen_mfma_blocks(4)>(p, wgs, stream);
+        case 8: return launch_gen_mfma_n<KT, VT, 8, gen_mfma_blocks(8)>(p, wgs, stream);
         default: return hipErrorInvalidValue;
     }
 }

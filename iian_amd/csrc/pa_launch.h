@@ -2,6 +2,7 @@
 #pragma once
 
 #include "pa_common.h"
+#include "pa_gen_layout.h"
 
 namespace iian_pa {
 
@@ -123,16 +124,9 @@ int general_tile_cells(int D, int Dv);
 int general_rows_per_block(int max_rows);
 
 // Matrix-core general path (pa_gen_mfma.hip): any K/V types, blocks of a
-// multiple of 16 cells.  gen_mfma_chunks: the 32-dim K chunks of the kernel
-// that takes head sizes D (a multiple of 8) and Dv (of 4), or 0: D in (32, 64],
-// (64, 96], (96, 128] or (128, 256], Dv up to 64, 128, 128 or 256.
+// multiple of 16 cells, the head sizes of gen_mfma_chunks (pa_gen_layout.h).
 // n_prefill_wgs: prefill workgroups (64-row blocks x kv heads x n_split), 0
 // when no sequence can have more than 16 rows.
-inline int gen_mfma_chunks(int D, int Dv) {
-    if (D % 8 || Dv % 4 || D <= 32 || D > 256) return 0;
-    const int nk = D <= 64 ? 2 : D <= 96 ? 3 : D <= 128 ? 4 : 8;
-    return Dv <= (nk == 2 ? 64 : nk == 8 ? 256 : 128) ? nk : 0;
-}
 hipError_t launch_gen_mfma(const GenMfmaParams &p, int type_k, int type_v, int64_t n_prefill_wgs, hipStream_t stream);
 hipError_t launch_gen_mfma_f32(const GenMfmaParams &p, int type_v, unsigned wgs, hipStream_t stream);
 hipError_t launch_gen_mfma_q8(const GenMfmaParams &p, int type_v, unsigned wgs, hipStream_t stream);

@@ -51,6 +51,9 @@ CASES = {
     "f32_d160_bs80": (8, 2, 160, [500, 161], [40, 1], {"k_type": F32, "bs": 80}),
     "f32k_q8v_d96": (8, 2, 96, [300, 64], [40, 1], {"k_type": F32, "v_type": Q8_0}),
     "q8k_f32v_d128_dv40": (8, 2, 128, [300, 64], [40, 1], {"k_type": Q8_0, "v_type": F32, "Dv": 40}),
+    "q8_d128_dv32": (8, 2, 128, [300, 64, 33], [40, 1, 17], {"k_type": Q8_0, "Dv": 32}),
+    "f16_d96_dv20": (8, 2, 96, [300, 64], [40, 1], {"Dv": 20}),
+    "f32_d104_dv4": (8, 2, 104, [300, 64], [40, 1], {"k_type": F32, "Dv": 4}),
     "q8k_f16v_d160": (8, 2, 160, [300, 64], [40, 1], {"k_type": Q8_0, "v_type": F16, "Dv": 96}),
     "q8_d96_tile_edges": (8, 2, 96, EDGE_LENS, [1] * 9, {"k_type": Q8_0}),
     "q8_d224": (8, 2, 224, [300, 64], [40, 1], {"k_type": Q8_0}),
