@@ -3,6 +3,7 @@
 
 #include "pa_common.h"
 #include "pa_gen_layout.h"
+#include "pa_prefill_order.h"
 
 namespace iian_pa {
 
@@ -68,8 +69,6 @@ hipError_t launch_mixed_f16(const AttnParams &p, int head_dim, int max_rows, hip
 // How a prefill launch's workgroups map to row blocks (a template parameter of
 // both prefill kernels: a run-time branch cost the plain form 0.3-1.4%).
 enum PrefillMode { kPrefillPlain = 0, kPrefillSplit = 1, kPrefillOrdered = 2 };
-// Query rows per prefill workgroup (both prefill kernels).
-constexpr int kPrefillBlockRows = 128;
 // Merge of the split prefill row blocks (p.n_split > 1); rows past cover_rows
 // of a sequence were not attended by the launch.
 hipError_t launch_split_merge(const AttnParams &p, int head_dim, int cover_rows, hipStream_t stream);

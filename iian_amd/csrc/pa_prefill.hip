@@ -706,20 +706,9 @@ __global__ __launch_bounds__(256) void pa_prefill_order_kernel(AttnParams p, int
         order[idx] = make_int2(-1, 0);
         return;
     }
-    const int window = p.n_swa > 0 ? p.n_swa + kPrefillBlockRows / p.gqa + 1 : INT32_MAX;
-    const int v = min(window, prior[s] + min(toks[s], ((b + 1) * kPrefillBlockRows + p.gqa - 1) / p.gqa));
-    // row blocks of sequence j with more than c cells
-    auto above = [&](int j, int c) {
-        const int t = c - prior[j];
-        if (c >= window || toks[j] <= t) return 0;
-        return max(0, nb[j] - (t < 0 ? 0 : (int) ((int64_t) t * p.gqa / kPrefillBlockRows)));
-    };
-    int rank = 0;
-    for (int j = 0; j < s; j++) rank += above(j, v - 1);
-    rank += above(s, v) + b - (nb[s] - above(s, v - 1));
-    for (int j = s + 1; j < p.S; j++) rank += above(j, v);
+    const int rank = order_rank({nb, prior, toks, p.S, p.gqa, order_window(p.n_swa, p.gqa)}, s, b);
     // overlapping query_start_loc ranges hold more row blocks than n_order
-    if (rank < p.n_order) order[rank] = make_int2(s, b);
+    if ((uint32_t) rank < (uint32_t) p.n_order) order[rank] = make_int2(s, b);
 }
 
 hipError_t launch_prefill_order(const AttnParams &p, int2 *order, int max_rows, hipStream_t stream) {

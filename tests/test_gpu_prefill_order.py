@@ -35,6 +35,7 @@ CASES = {
     "f16_d96_mha": (32, 32, 96, [1100, 500], [1100, 400], {}),
     "f16_d256": (16, 8, 256, [1500, 1200, 90], [1500, 1200, 90], {}),
     "q8_d128": (32, 8, 128, [1600, 1200], [1600, 1200], {"k_type": Q8_0}),
+    "window_above_every_context": (32, 8, 128, [1500, 1100], [1500, 1100], {"n_swa": 2 ** 31 - 1}),
     "hkv3": (36, 3, 64, [2100, 1500], [2100, 1500], {}),
     "random_positions": (32, 8, 128, [1500, 1200], [1500, 1200], {"pos_mode": "random"}),
 }
