@@ -544,6 +544,27 @@ __device__ __forceinline__ void gm_piece(const GenMfmaParams &p, const GmPiece &
                 const CellWindow cw = cell_window(tile, TC, pc.ce, prow, a.causal, a.n_swa);
 #pragma unroll
                 for (int e = 0; e < CV; e++) x[e] = cell_visible(cw, 16 * (e >> 2) + 4 * g + (e & 3)) ? x[e] : -INFINITY;
+                // V of cells that no row of the wave attends (before its window, after
+                // its last position, the repeats past the last cell) may be infinite or
+                // NaN, and P = 0 must not meet it
+                const int v_lo = a.n_swa > 0 ? max(0, pc.pmin - a.n_swa + 1) : 0;
+                const int v_hi = a.causal ? min(pc.ce, pc.pmax + 1) : pc.ce;
+                if (tile < v_lo || tile + TC > v_hi) {
+#pragma unroll
+                    for (int c = 0; c < CV; c++) {
+                        const int cell = tile + 16 * (c >> 2) + 4 * g + (c & 3);
+                        const bool in = cell >= v_lo && cell < v_hi;
+#pragma unroll
+                        for (int b = 0; b < NV; b++) {
+                            if constexpr (VT == 8) {
+                                vr[c][b].d = in ? vr[c][b].d : (uint16_t) 0;
+                            } else {
+#pragma unroll
+                                for (int w = 0; w < VE; w++) vr[c][b].a[w] = in ? vr[c][b].a[w] : 0u;
+                            }
+                        }
+                    }
+                }
             }
             float mx = x[0];
 #pragma unroll

@@ -124,3 +124,45 @@ def test_noalloc_without_room_for_decode_records(pa, oracle):
     assert call_noalloc(pa._lib.load(), c, q, k, v, batch, out, err) == 0
     torch.cuda.synchronize()
     assert row_rel_err(out.cpu().numpy(), oracle_attention(oracle, c)).max() <= TOL and int(err.item()) == 0
+
+
+@pytest.mark.parametrize("value", [np.inf, np.nan])
+@pytest.mark.parametrize("D,k_type,v_type", [(80, F16, F16), (128, F32, F32), (128, F16, F32), (96, Q8_0, Q8_0),
+                                             (96, F32, Q8_0), (160, F16, F16)])
+def test_values_of_cells_not_attended_are_not_used(pa, oracle, D, k_type, v_type, value):
+    """Infinite or NaN V in the cells just before a decode row's window (inside
+    its first tile), in the cells after its position, and, alone, in the last
+    cell of a sequence, which a partial tile repeats: the rows that do not
+    attend them keep their values, as the reference skips masked cells, and over
+    F32 a row that attends an infinite one is infinite, not NaN (over F16 one of
+    P's two terms may be zero)."""
+    banner(f"general mfma unattended V D={D} types {k_type} {v_type} {value}")
+    kw = dict(k_type=k_type, v_type=v_type, quantize=oracle.quantize_q8_0)
+    def poison(c, s, cells):
+        for cell in cells:
+            row = c.v_pool[c.bt[s, cell // c.bs] * c.bs + cell % c.bs]
+            if c.v_type == Q8_0:   # the blocks' scales
+                row.reshape(-1, 34)[:, :2] = np.array([value], np.float16).view(np.uint8)
+            else:
+                row.view(np.float16 if c.v_type == F16 else np.float32)[:] = value
+    # one decode, one verify and one prefill sequence over a window whose first cell is not a tile's
+    c = make_case(np.random.default_rng(8), 4, 2, D, [300, 211, 150], [1, 5, 40], n_swa=75, **kw)
+    for s, (L, n) in enumerate(((300, 1), (211, 5), (150, 40))):
+        poison(c, s, range(max(0, L - n - 75 - 30), L - n - 75 + 1))
+    got, want = gpu_attention(pa, c), oracle_attention(oracle, c)
+    assert np.isfinite(want).all() and np.isfinite(got).all()
+    assert row_rel_err(got, want).max() <= TOL
+    # causal, a query before the sequence's end
+    c = make_case(np.random.default_rng(9), 4, 2, D, [300, 90], [1, 1], **kw)
+    c.pos[:] = (250, 17)
+    poison(c, 0, range(251, 300))
+    poison(c, 1, range(18, 90))
+    got, want = gpu_attention(pa, c), oracle_attention(oracle, c)
+    assert np.isfinite(want).all() and np.isfinite(got).all()
+    assert row_rel_err(got, want).max() <= TOL
+    # the last cell, attended, in a tile that repeats it
+    c = make_case(np.random.default_rng(10), 4, 2, D, [33, 97], [1, 1], **kw)
+    poison(c, 0, [32])
+    poison(c, 1, [96])
+    got = gpu_attention(pa, c)
+    assert np.all(got == np.inf) if value == np.inf and v_type == F32 else not np.isfinite(got).any()
