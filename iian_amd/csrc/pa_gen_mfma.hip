@@ -24,8 +24,9 @@ __global__ __launch_bounds__(256) void pa_gen_merge_kernel(GenMfmaParams p, int 
         const int nq = min(max(a.qsl[s + 1], q0), a.T) - q0;
         if (nq <= 0 || (int64_t) nq * a.gqa > a.decode_rows || info.y <= 1) return;
         const int M = nq * a.gqa;
-        // (WPR = 4: one row per workgroup, so its barrier is met once)
-        for (int r = WPR > 1 ? blockIdx.x % seg_rows : wave; r < M; r += WPR > 1 ? kGmRows : 4) {
+        // (a sequence with more tokens than the caller's max_query_len has more rows than seg_rows)
+        for (int r = WPR > 1 ? blockIdx.x % seg_rows : wave; r < M; r += WPR > 1 ? seg_rows : 4) {
+            if (WPR > 1) __syncthreads();   // the row before it has left comb
             const int64_t orow = (int64_t) (q0 + r / a.gqa) * a.H + hk * a.gqa + r % a.gqa;
             merge_row<WPR, LPR>(rec_o(a, info.x, 0, r, p.Dv), a.rec_stride, rec_ml(a, info.x, 0, r),
                                 2 * (int64_t) a.rec_rows, info.y, p.Dv, a.out + orow * p.Dv, comb);

@@ -9,8 +9,8 @@ import numpy as np
 import pytest
 import torch
 
-from helpers import Q8_0, make_case, row_rel_err
-from test_gpu_parity import TOL, banner, gpu_attention, oracle_attention
+from helpers import F16, F32, Q8_0, make_case, row_rel_err
+from test_gpu_parity import TOL, banner, gpu_attention, oracle_attention, to_device
 
 pytestmark = pytest.mark.gpu
 
@@ -47,3 +47,20 @@ def test_merge_matches_oracle(pa, oracle, name):
     got = gpu_attention(pa, c)
     e = row_rel_err(got, oracle_attention(oracle, c))
     assert np.isfinite(got).all() and e.max() <= TOL, (name, e.max())
+
+
+@pytest.mark.parametrize("D,k_type", [(128, F32), (128, F16), (80, F16)])
+def test_rows_past_the_declared_length_are_merged_too(pa, oracle, D, k_type):
+    """A decode sequence of more tokens than max_query_len, its rows still one
+    tile: bit 2 is set, and every row that was attended is merged, in the form
+    with a workgroup per row as in the others."""
+    banner(f"merge understated max_query_len D={D} type {k_type}")
+    c = make_case(np.random.default_rng(33), 8, 2, D, [9000, 40], [3, 1], k_type=k_type)
+    k, v, batch = to_device(pa, c)
+    batch.max_query_len = 2    # 8 of the 12 rows
+    out = torch.full((c.T, c.H, c.Dv), 7.0, device="cuda")
+    err = torch.zeros(1, dtype=torch.int32, device="cuda")
+    pa.build_paged_attn(torch.as_tensor(c.q).cuda(), k, v, c.Hkv, pa.PagedAttnParams(scale=c.scale), batch, out=out,
+                        err_flag=err)
+    assert int(err.item()) == 4
+    assert row_rel_err(out.cpu().numpy(), oracle_attention(oracle, c)).max() <= TOL
