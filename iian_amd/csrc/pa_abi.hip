@@ -5,6 +5,7 @@
 #include "../../include/iian_pa.h"
 #include "pa_common.h"
 #include "pa_launch.h"
+#include "pa_plan.h"
 
 #include <algorithm>
 #include <atomic>
@@ -59,10 +60,6 @@ constexpr int kGenMixedDecodeWavesPerCu = 3;
 constexpr int kGenDecodeWavesPerCuWide = 4;
 constexpr int kGenPrefillWgsPerCuF16 = 1;
 constexpr int kGenPrefillWgsPerCu = 2;
-// Split prefill row blocks (prefill_splits): the rounds of D = 256 workgroups
-// a launch of about one round is cut into.
-constexpr int kSplitRoundsD256 = 3;
-constexpr int kOrderMinCells = 1024;     // prefill_order_entries
 constexpr int kQ8DecodeWavesPerCu = 8;
 constexpr int kMaxWavesPerCu = kQ8DecodeWavesPerCu;
 constexpr int kDefaultCus = 256;   // an MI355X, when the device cannot be queried
@@ -285,65 +282,6 @@ size_t split_bytes(size_t out_rows, int64_t ns, int head_dim_v) {
     return split_o_bytes(out_rows, ns, head_dim_v) + out_rows * (size_t) ns * 2 * sizeof(float);
 }
 
-// Ranges a prefill row block is cut into at most (split_range, pa_common.h),
-// with `room` bytes of workspace left for their records.  A launch whose row
-// blocks take at most half of the device's workgroup slots is cut to fill
-// them; more ranges than that only add starts and records (one 256-token chunk
-// over 10K cells at H16/Hkv8/D256: 481 us uncut, 87 with one workgroup per CU,
-// 136 with two rounds of them).  D <= 128 kernels hold two workgroups per CU,
-// less the decode workers of a mixed launch (4 chunks' worth of slots taken
-// from 2 chunks of 512 beside 32 decodes cost 365 -> 390 us).  At D = 256,
-// where a workgroup has its CU alone and the longest one decides a launch of
-// about one round, such a launch is planned for 3 rounds and the kernel cuts it
-// when the batch is uneven (8 chunks of 256 over 4K-16K cells 784 -> 614 us; 2
-// rounds 0-3% either way on other lengths).  Measured besides, whole calls: 8 Q8_0
-// kv heads, chunks of 504 and 361 tokens over 1.6K-2.7K cells beside 24
-// decodes, two layers, 394 -> 301 us; one chunk of 250 tokens over 8.5K cells at
-// H32/Hkv8/D128 231 -> 96 us; full launches unchanged.
-int prefill_splits(AttnParams &p, int head_dim, bool mixed_one_launch, int64_t max_rows, int32_t block_size,
-                   int cus, size_t room) {
-    const int64_t rows = (int64_t) p.T * p.gqa;
-    const int64_t blocks = std::max<int64_t>(1, rows / kPrefillBlockRows) * p.Hkv;
-    // slots: the workgroups of this kernel the device holds at once
-    const int64_t slots = head_dim == 256 ? cus : 2 * cus - (mixed_one_launch ? p.sk_workers / 4 : 0);
-    int64_t ns = slots / blocks;
-    p.split_balance = 0;
-    if (head_dim == 256 && 2 * blocks > slots && p.n_swa <= 0 && p.S <= 64) {
-        ns = kSplitRoundsD256 * slots / blocks;
-        p.split_balance = 1;   // the kernel looks whether the batch is uneven
-    }
-    int64_t cells = (int64_t) p.max_blocks * block_size;
-    if (p.n_swa > 0) cells = std::min<int64_t>(cells, (int64_t) p.n_swa + max_rows / p.gqa);
-    ns = std::min<int64_t>({ns, cells / kSplitMinCells, kMaxSplits});
-    const size_t out_rows = (size_t) p.T * p.H;
-    while (ns > 1 && split_bytes(out_rows, ns, head_dim) > room) ns--;
-    return (int) std::max<int64_t>(ns, 1);
-}
-
-// Entries of the order list of a prefill launch (launch_prefill_order), 0 for a
-// launch in batch order.  A new prompt's row blocks grow from one tile to its
-// whole length, and in batch order the longest of them start last: the list
-// starts them first, for a launch of about 5 us more.  It pays when the launch
-// takes more than a round of workgroup slots and its row blocks are that
-// uneven, which the host sees when the longest prompt may make up half of the
-// longest table (H32/Hkv8/D128, new prompts: 2243 + 2552 + 752 tokens 184 ->
-// 171 us with the KV write, one of 2637 123 -> 106, one of 4096 224 -> 198, one
-// of 8192 738 -> 681; 4 of 1000 87 either way).  At D = 256 the three
-// prompts 252 -> 229, one of 8192 1055 -> 908.  Short prompts (8 of 510: 69 ->
-// 80), chunks over long contexts and windows, whose row blocks are alike, stay
-// in batch order, which keeps a sequence's row blocks together (2-6% at 8
-// chunks over 2K cells, a 1024-cell window, and 8 chunks beside 64 decodes).
-int prefill_order_entries(const AttnParams &p, int head_dim, bool mixed_one_launch, int32_t block_size, int cus) {
-    const int64_t rows = (int64_t) p.T * p.gqa, blocks = rows / kPrefillBlockRows;
-    const int64_t cells = (int64_t) p.max_blocks * block_size;
-    const int64_t slots = head_dim == 256 ? cus : 2 * cus - (mixed_one_launch ? p.sk_workers / 4 : 0);
-    const int64_t n = blocks + std::min<int64_t>(p.S, rows / (p.decode_rows + 1));
-    if (4 * blocks * p.Hkv < 5 * slots || cells < kOrderMinCells || 2 * (int64_t) p.max_q < cells ||
-        (p.n_swa > 0 && p.n_swa < cells) || p.S > kOrderMaxSeqs || n * p.Hkv >= INT32_MAX / 2)
-        return 0;
-    return (int) n;
-}
-
 // Any head size the general kernel stages (1 .. 1024; the reference's op
 // takes any, paged_attn.cpp:96-100); a Q8_0 head slice is whole 32-value
 // blocks.
@@ -426,7 +364,7 @@ int run_attention(hipStream_t st, const float *q, const void *k_pool, const void
                   int32_t max_query_len, int32_t n_head, int32_t n_head_kv, int32_t head_dim, int32_t head_dim_v,
                   int32_t block_size, float scale, float softcap, int32_t causal, int32_t n_swa, float *out,
                   const WsSource &src, int32_t *err_flag, const float *k_new = nullptr,
-                  const float *v_new = nullptr) {
+                  const float *v_new = nullptr, const StepLengths *step = nullptr) {
     if (n_tokens < 0 || n_seqs < 0 || max_query_len < 0) return IIAN_PA_ERR_ARG;
     if (n_tokens == 0 || n_seqs == 0) return IIAN_PA_OK;
     if (!q || !k_pool || !v_pool || !block_tables || !seq_lens || !query_start_loc || !pos || !out)
@@ -450,6 +388,9 @@ int run_attention(hipStream_t st, const float *q, const void *k_pool, const void
         return IIAN_PA_ERR_ARG;
     const int bs_log2 = log2_exact(block_size);
     const int gqa = n_head / n_head_kv;
+    // what the launch is planned for: the step's contexts, or as much as the table holds
+    CallLengths len = {(int64_t) max_blocks * block_size, false, false};
+    if (step) len = {std::min<int64_t>(len.cells, step->longest), true, step->uneven};
 
     // f16 pools at head size 96 (Phi-3) take the MFMA kernels too: the decode
     // kernel when every sequence of the call is a decode or spec-verify row
@@ -531,7 +472,7 @@ int run_attention(hipStream_t st, const float *q, const void *k_pool, const void
             // kGenPrefillWgsPerCu workgroups per CU, each range at least 8
             // tiles of the longest table, the records inside the workspace
             const int64_t full = std::max<int64_t>(1, rows / 64) * n_head_kv;
-            const int64_t max_tiles = ((int64_t) max_blocks * block_size + kTile - 1) / kTile;
+            const int64_t max_tiles = (len.cells + kTile - 1) / kTile;
             const bool f16 = type_k == IIAN_PA_TYPE_F16 && type_v == IIAN_PA_TYPE_F16;
             int64_t ns = ((int64_t) (f16 ? kGenPrefillWgsPerCuF16 : kGenPrefillWgsPerCu) * cus + full - 1) / full;
             ns = std::min<int64_t>({ns, std::max<int64_t>(1, max_tiles / 8), kMaxSplits});
@@ -722,13 +663,19 @@ int run_attention(hipStream_t st, const float *q, const void *k_pool, const void
     p.n_split = 1;
     if (!decode_only) {
         const size_t cap = src.scratch ? kScratchBytes : wl.total;
-        p.n_order = prefill_order_entries(p, head_dim, mixed_one_launch, block_size, cus);
+        const PrefillCall c = {n_tokens, n_seqs, n_head_kv, gqa, n_swa, max_query_len, p.decode_rows, p.sk_workers,
+                               head_dim, cus, mixed_one_launch, type_k == IIAN_PA_TYPE_Q8_0, len};
+        p.n_order = prefill_order_entries(c);
         if (split_at + p.n_order * sizeof(int2) > cap) p.n_order = 0;
         if (p.n_order > 0) {   // the list lies where split records would
             need = split_at + p.n_order * sizeof(int2);
         } else {
-            p.n_split = prefill_splits(p, head_dim, mixed_one_launch, max_rows, block_size, cus,
-                                       cap - std::min(split_at, cap));
+            const SplitPlan sp = prefill_splits(c);
+            const size_t room = cap - std::min(split_at, cap);
+            p.n_split = sp.ranges;
+            while (p.n_split > 1 && split_bytes((size_t) n_tokens * n_head, p.n_split, head_dim) > room) p.n_split--;
+            p.split_balance = sp.balance;
+            p.split_blocks = sp.row_blocks;
             if (p.n_split > 1) need = split_at + split_bytes((size_t) n_tokens * n_head, p.n_split, head_dim_v);
         }
     }
@@ -774,6 +721,23 @@ int run_attention(hipStream_t st, const float *q, const void *k_pool, const void
 }
 
 }  // namespace
+
+namespace iian_pa {
+
+int attention_of_step(void *stream, const float *q, const void *k_pool, const void *v_pool, int type_k, int type_v,
+                      int32_t num_blocks, const int32_t *block_tables, int32_t max_blocks, const int32_t *seq_lens,
+                      const int32_t *query_start_loc, const int32_t *pos, int32_t n_tokens, int32_t n_seqs,
+                      int32_t max_query_len, int32_t n_head, int32_t n_head_kv, int32_t head_dim, int32_t head_dim_v,
+                      int32_t block_size, float scale, float softcap, int32_t causal, int32_t n_swa, float *out,
+                      void *workspace, size_t workspace_bytes, int32_t *err_flag, const StepLengths &step) {
+    const WsSource src = {workspace, workspace_bytes, false};
+    return run_attention((hipStream_t) stream, q, k_pool, v_pool, type_k, type_v, num_blocks, block_tables,
+                         max_blocks, seq_lens, query_start_loc, pos, n_tokens, n_seqs, max_query_len, n_head,
+                         n_head_kv, head_dim, head_dim_v, block_size, scale, softcap, causal, n_swa, out, src,
+                         err_flag, nullptr, nullptr, &step);
+}
+
+}  // namespace iian_pa
 
 extern "C" {
 

@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "pa_split.h"
+
 namespace iian_pa {
 
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
@@ -63,6 +65,7 @@ struct AttnParams {
     int32_t split_balance;      // cut for balance only: not when the batch is even (pa_prefill16_kernel)
     float *split_o;             // their records past the first: [T*H][n_split - 1][D] (the first is in `out`)
     float *split_ml;            // [T*H][n_split] of (m in log2 units, l)
+    int32_t split_blocks;       // prefill row blocks the launch has workgroups for
     const int2 *order;          // nullable: (sequence, row block) of the launch's prefill row blocks, most cells
                                 // first, then (-1, 0) (pa_prefill_order_kernel)
     int32_t n_order;            // its entries
@@ -244,24 +247,64 @@ __device__ __forceinline__ float *rec_ml(const AttnParams &p, int rec, int hr, i
 // longest one.  Its row blocks are then cut into equal ranges of their tiles,
 // one workgroup each, whose partial results a launch after it merges
 // (pa_split_merge_kernel): as many as kSplitMinCells cells each allow, at most
-// n_split.  A row block of up to kSplitMinCells cells is never cut, so its rows do
-// not depend on the batch or on how the launch was planned.
-constexpr int kSplitMinCells = 1024;
-constexpr int kMaxSplits = 16;   // p.n_split at most: a row's (m, l) pairs fit the lanes of split_merge_rows
+// n_split.  Workgroups look their range up (find_range), so that a batch of few
+// prefill sequences among many leaves few of them without work (n_split times
+// the grid of a launch without ranges cost a Q8_0 step of one chunk and 300
+// decodes 82 -> 117 us), and the ranges of few kv heads spread over all XCDs
+// (one prompt of 2300 tokens at H14/Hkv2/D64 106 -> 73 us).
+// A row block of up to kSplitMinCells cells is never cut, so its rows do not
+// depend on the batch or on how the launch was planned.  The ranges of a longer
+// one round P to f16 against their own reference maximum, and its rows follow
+// the cut within that rounding.
+// Row blocks (block_rows rows, at most n_rb) of sequence s, 0 for one the
+// prefill launch does not attend.
+__device__ __forceinline__ int prefill_row_blocks(const AttnParams &p, int s, int block_rows, int n_rb) {
+    if (s >= p.S) return 0;
+    const int q0 = min(max(p.qsl[s], 0), p.T);
+    const int64_t M = (int64_t) (min(max(p.qsl[s + 1], q0), p.T) - q0) * p.gqa;
+    return M > p.decode_rows ? (int) min((int64_t) n_rb, (M + block_rows - 1) / block_rows) : 0;
+}
 
-struct SplitRange {
-    int n;        // ranges of this row block
-    int lo, hi;   // cells of range z (empty when z >= n)
+// Range `item` of a cut launch: the sequences in order, of each its ranges z <
+// n_split, of each range its row blocks (which read the same cells), the last
+// rows, which see the most cells, first.  find_range_at: among 64 sequences
+// whose row blocks lane i holds, those before it counted in `before`.
+struct RangeItem {
+    int seq, z, rb;   // seq: index of the sequence among the lanes
 };
-// Range z of the cells [c_lo, c_hi) in whole tiles of `tile` cells.
-__device__ __forceinline__ SplitRange split_range(int c_lo, int c_hi, int z, int n_split, int tile) {
-    const int cells = max(c_hi - c_lo, 0);
-    SplitRange r;
-    r.n = min(n_split, max(1, (cells + kSplitMinCells - 1) / kSplitMinCells));
-    const int nt = (cells + tile - 1) / tile, per = (nt + r.n - 1) / r.n;
-    r.lo = min(c_hi, c_lo + z * per * tile);
-    r.hi = z < r.n ? min(c_hi, c_lo + (z + 1) * per * tile) : r.lo;
-    return r;
+__device__ __forceinline__ bool find_range_at(int nb, int n_split, int item, int &before, RangeItem &r) {
+    int incl = nb * n_split;
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int u = __shfl_up(incl, o);
+        if (lane >= o) incl += u;
+    }
+    const uint64_t hit = __builtin_amdgcn_ballot_w64(before + incl > item);
+    if (!hit) {
+        before += __builtin_amdgcn_readfirstlane(__shfl(incl, 63));
+        return false;
+    }
+    r.seq = __builtin_ctzll(hit);
+    const int n = __builtin_amdgcn_readfirstlane(__shfl(nb, r.seq));
+    const int off = item - before - (__builtin_amdgcn_readfirstlane(__shfl(incl, r.seq)) - n * n_split);
+    r.z = off / n;
+    r.rb = n - 1 - off % n;
+    return true;
+}
+// Called by a whole wave; the answer is wave-uniform, false past the last range.
+__device__ __forceinline__ bool find_range(const AttnParams &p, int block_rows, int n_rb, int item, int &s, int &z,
+                                           int &rb) {
+    int before = 0;
+    RangeItem r;
+    for (int base = 0; base < p.S; base += 64)
+        if (find_range_at(prefill_row_blocks(p, base + (threadIdx.x & 63), block_rows, n_rb), p.n_split, item, before, r)) {
+            s = base + r.seq;
+            z = r.z;
+            rb = r.rb;
+            return true;
+        }
+    return false;
 }
 
 // The (m, l) of output row `orow`, range z.  Range 0 of an uncut row block

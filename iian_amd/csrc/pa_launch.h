@@ -3,6 +3,7 @@
 
 #include "pa_common.h"
 #include "pa_gen_layout.h"
+#include "pa_plan.h"
 #include "pa_prefill_order.h"
 
 namespace iian_pa {
@@ -66,6 +67,19 @@ hipError_t launch_prefill(const AttnParams &p, int head_dim, int kv_type, int ma
 // workgroups plus the decode rows' stream-K workers, which merge their split
 // segments themselves.
 hipError_t launch_mixed_f16(const AttnParams &p, int head_dim, int max_rows, hipStream_t stream);
+// What the host knows of a step's contexts (the runtime, which is given them).
+struct StepLengths {
+    int32_t longest;   // cells of the longest
+    bool uneven;       // prefill_uneven of its prefill sequences
+};
+// iian_pa_attention, planned for them instead of for the table's width.
+int attention_of_step(void *stream, const float *q, const void *k_pool, const void *v_pool, int type_k, int type_v,
+                      int32_t num_blocks, const int32_t *block_tables, int32_t max_blocks, const int32_t *seq_lens,
+                      const int32_t *query_start_loc, const int32_t *pos, int32_t n_tokens, int32_t n_seqs,
+                      int32_t max_query_len, int32_t n_head, int32_t n_head_kv, int32_t head_dim, int32_t head_dim_v,
+                      int32_t block_size, float scale, float softcap, int32_t causal, int32_t n_swa, float *out,
+                      void *workspace, size_t workspace_bytes, int32_t *err_flag, const StepLengths &step);
+
 // How a prefill launch's workgroups map to row blocks (a template parameter of
 // both prefill kernels: a run-time branch cost the plain form 0.3-1.4%).
 enum PrefillMode { kPrefillPlain = 0, kPrefillSplit = 1, kPrefillOrdered = 2 };
@@ -74,7 +88,6 @@ enum PrefillMode { kPrefillPlain = 0, kPrefillSplit = 1, kPrefillOrdered = 2 };
 hipError_t launch_split_merge(const AttnParams &p, int head_dim, int cover_rows, hipStream_t stream);
 // Writes the order list (p.order, p.n_order entries) of a prefill launch of at
 // most kOrderMaxSeqs sequences.
-constexpr int kOrderMaxSeqs = 1024;
 hipError_t launch_prefill_order(const AttnParams &p, int2 *order, int max_rows, hipStream_t stream);
 // The 16-row-tile prefill kernel (pa_prefill16.hip), used at head size 256.
 hipError_t launch_prefill16(const AttnParams &p, int head_dim, int kv_type, int max_rows, hipStream_t stream);

@@ -101,7 +101,7 @@ __device__ __forceinline__ void merge_row(const float *o0, int64_t o_stride, con
 }
 
 
-// One wave's output rows of split prefill row blocks (split_range, pa_common.h):
+// One wave's output rows of split prefill row blocks (split_range, pa_split.h):
 // rows row0 .. row0 + 64/LPR - 1, LPR lanes each:
 //   out = sum_z 2^(m_z - m) O_z / sum_z 2^(m_z - m) l_z
 // over the row's ranges, range 0's O taken from `out` itself.  Rows of a decode

@@ -73,7 +73,7 @@ struct PrefillOcc {
 // costs the launch nothing, and the call is one launch.
 //
 // MODE (PrefillMode): row blocks in batch order, cut into ranges of their tiles
-// (split_range, pa_common.h), or in the order of a list (pa_prefill_order_kernel).
+// (split_range, pa_split.h), or in the order of a list (pa_prefill_order_kernel).
 template <int D, int NW, int KVT, bool MIXED, int MODE>
 __global__ __launch_bounds__(NW * 64, PrefillOcc<D>::kWavesPerSimd) void pa_prefill_kernel(AttnParams p, int n_rb,
                                                                                           int n_dec) {
@@ -122,12 +122,11 @@ __global__ __launch_bounds__(NW * 64, PrefillOcc<D>::kWavesPerSimd) void pa_pref
     // early ones and get the CU to themselves sooner (Qwen3-8B chunked prefill
     // 133.3-134.0 against 137.2-137.3 us; with decode rows 164.8-165.9 against
     // 173.5-173.7 us).  Per pair, so every row block is taken once.
-    // (a cut row block's ranges lie n_rb slots apart: the row blocks of one
-    // range, which read the same cells, stay together)
     // With an order list (launches of more than one round of slots), a
     // workgroup takes a row block's next kv head instead: the heads of a list
     // entry go to consecutive XCDs, so with a multiple of 8 heads each head
     // stays on its XCD, and the row blocks with the most cells start first.
+    // The ranges of a cut launch are dealt like that too.
     int s, hk, rb, z = 0;
     if constexpr (MODE == kPrefillOrdered) {
         hk = bid % p.Hkv;
@@ -136,13 +135,14 @@ __global__ __launch_bounds__(NW * 64, PrefillOcc<D>::kWavesPerSimd) void pa_pref
         rb = __builtin_amdgcn_readfirstlane(e.y);
         // (past the list; or unwritten, where query_start_loc's ranges overlap)
         if ((uint32_t) s >= (uint32_t) p.S || (uint32_t) rb >= (uint32_t) n_rb) return;
+    } else if constexpr (SPLIT) {
+        hk = bid % p.Hkv;
+        if (!find_range(p, ROWS, n_rb, bid / p.Hkv, s, z, rb)) return;
     } else {
         const int slot = bid >> 3;
-        const int per_pair = SPLIT ? n_rb * p.n_split : n_rb;
-        const int pair_x = slot / per_pair;
+        const int pair_x = slot / n_rb;
         const int pair = (bid & 7) + 8 * pair_x;
         rb = (((pair_x * n_rb) / p.cus_per_xcd) & 1) ? n_rb - 1 - slot % n_rb : slot % n_rb;
-        if (SPLIT) z = slot % per_pair / n_rb;
         if (pair >= p.S * p.Hkv) return;
         s = pair / p.Hkv;
         hk = pair % p.Hkv;
@@ -724,8 +724,9 @@ static hipError_t launch_prefill_t(const AttnParams &p, int max_rows, hipStream_
     const int n_rb = (max_rows + ROWS - 1) / ROWS;
     const int pairs_per_xcd = (p.S * p.Hkv + 7) / 8;
     static_assert(ROWS == kPrefillBlockRows, "the host plans 128-row blocks");
-    const int64_t n_pf = p.order ? (int64_t) p.n_order * p.Hkv
-                                 : 8 * (int64_t) pairs_per_xcd * n_rb * std::max(1, p.n_split);
+    const int64_t n_pf = p.order         ? (int64_t) p.n_order * p.Hkv
+                         : p.n_split > 1 ? (int64_t) p.split_blocks * p.n_split * p.Hkv
+                                         : 8 * (int64_t) pairs_per_xcd * n_rb;
     const int64_t n_dec = MIXED ? ((p.sk_workers + NW - 1) / NW + 7) / 8 * 8 : 0;
     const int64_t nwg = n_dec + n_pf;
     if (nwg > INT32_MAX) return hipErrorInvalidValue;

@@ -28,8 +28,6 @@
 #include "pa_launch.h"
 #include "pa_mfma.h"
 
-#include <algorithm>
-
 namespace iian_pa {
 
 // The lo product of q in bf8 (f16 pools; pa_mfma.h): one
@@ -71,7 +69,7 @@ __device__ __forceinline__ f16x8 lds_tr_b16x8_16(const char *p0, const char *p1)
 // each QK^T k-step MFMA (k-step = block), so q*d enters the scores exactly;
 // V as f16(q*d), the correctly rounded dequantised value.
 // MODE (PrefillMode): row blocks in batch order, cut into ranges of their tiles
-// (split_range, pa_common.h), or in the order of a list (pa_prefill.hip).
+// (split_range, pa_split.h), or in the order of a list (pa_prefill.hip).
 template <int D, int NRT, int NW, int KVT, int MODE>
 // Waves per SIMD asked of the register allocator: four for f16 at D = 128 (two
 // 8-wave workgroups per CU in 128 VGPRs), else two up to D = 128, one at 256.
@@ -98,13 +96,9 @@ __global__ __launch_bounds__(NW * 64, (D == 128 && KVT == 1) ? 4 : (D <= 128 ? 2
     // few sequences of a batch are prefill chunks) land on different XCDs.
     const int bid = blockIdx.x;
     const int slot = bid >> 3;
-    // (a cut row block's ranges lie n_rb slots apart: the row blocks of one
-    // range, which read the same cells, stay together)
-    const int per_pair = SPLIT ? n_rb * p.n_split : n_rb;
-    const int pair = (bid & 7) + 8 * (slot / per_pair);
-    int rb = slot % n_rb;
-    const int z = SPLIT ? slot % per_pair / n_rb : 0;
-    if (!ordered && pair >= p.S * p.Hkv) return;
+    const int pair = (bid & 7) + 8 * (slot / n_rb);
+    int rb = slot % n_rb, z = 0;
+    if (!ordered && !SPLIT && pair >= p.S * p.Hkv) return;
 
     // wave index in a scalar register, so that the tile-load rows derived from
     // it stay in SALU (cfg5 global prefill 4947-5022 against 5015-5085 us)
@@ -118,7 +112,9 @@ __global__ __launch_bounds__(NW * 64, (D == 128 && KVT == 1) ? 4 : (D <= 128 ? 2
     // 64 sequences; past that, and with a window, which bounds every row
     // block's cells, the batch order stands: the ranking's round trip and
     // shuffles cost the window-bounded prefill 2-3%).
-    const int hk = ordered ? bid % p.Hkv : pair % p.Hkv;
+    // With an order list, or cut into ranges, a workgroup takes the next kv head
+    // of the same row block, so the heads go to consecutive XCDs.
+    const int hk = ordered || SPLIT ? bid % p.Hkv : pair % p.Hkv;
     int s = pair / p.Hkv, L, q0, nq;
     if (ordered) {
         const int2 e = p.order[bid / p.Hkv];
@@ -142,12 +138,6 @@ __global__ __launch_bounds__(NW * 64, (D == 128 && KVT == 1) ? 4 : (D <= 128 ? 2
             rank += (kj > key || (kj == key && j < lane)) ? 1 : 0;
         }
         if (SPLIT && p.split_balance) {
-            // The call has about as many workgroups as CUs: uncut, it takes the
-            // longest of them, or its rounds of average ones.  Cut only when
-            // that is well above an even share of the cells (records and the
-            // pieces' starts cost an even batch 12%: 8 chunks of 256 tokens
-            // over 6000 cells each 356 against 400 us; over 4K-16K cells 784
-            // us uncut, 627 cut).
             const float rows = key >= 0 ? (float) ((nql * p.gqa + ROWS - 1) / ROWS) : 0.f;
             float blocks = rows, cells = rows * (float) max(key, 0), longest = (float) max(key, 0);
 #pragma unroll
@@ -156,18 +146,29 @@ __global__ __launch_bounds__(NW * 64, (D == 128 && KVT == 1) ? 4 : (D <= 128 ? 2
                 cells += __shfl_xor(cells, o);
                 longest = fmaxf(longest, __shfl_xor(longest, o));
             }
-            const float cus = 8.f * (float) p.cus_per_xcd, wgs = blocks * (float) p.Hkv;
-            const float share = cells * (float) p.Hkv / cus;
-            const float uncut = fmaxf(longest, ceilf(wgs / cus) * (cells / fmaxf(blocks, 1.f)));
-            if (!__builtin_amdgcn_ballot_w64(uncut > 1.2f * share)) n_split = 1;
-            if (z >= n_split) return;
+            const bool cut = prefill_uneven(blocks, cells, longest, (float) p.Hkv, 8.f * (float) p.cus_per_xcd);
+            if (!__builtin_amdgcn_ballot_w64(cut)) n_split = 1;
         }
-        const uint64_t hit = __builtin_amdgcn_ballot_w64(lane < p.S && rank == s);
-        s = __builtin_amdgcn_readfirstlane(hit ? (int) __builtin_ctzll(hit) : s);
+        if constexpr (SPLIT) {   // the ranges of the longest sequence first
+            const int src = __builtin_amdgcn_ds_permute(4 * (lane < p.S ? rank : lane), lane);   // lane i: the i-th longest
+            int nb = key >= 0 ? min(n_rb, (nql * p.gqa + ROWS - 1) / ROWS) : 0;
+            nb = __shfl(nb, src);
+            RangeItem r;
+            int before = 0;
+            if (!find_range_at(nb, n_split, bid / p.Hkv, before, r)) return;
+            s = __builtin_amdgcn_readfirstlane(__shfl(src, r.seq));
+            z = r.z;
+            rb = r.rb;
+        } else {
+            const uint64_t hit = __builtin_amdgcn_ballot_w64(lane < p.S && rank == s);
+            s = __builtin_amdgcn_readfirstlane(hit ? (int) __builtin_ctzll(hit) : s);
+        }
         L = __builtin_amdgcn_readfirstlane(__shfl(ll, s));
         q0 = __builtin_amdgcn_readfirstlane(__shfl(a, s));
         nq = __builtin_amdgcn_readfirstlane(__shfl(nql, s));
     } else {
+        if constexpr (SPLIT)
+            if (!find_range(p, ROWS, n_rb, bid / p.Hkv, s, z, rb)) return;
         L = p.seq_lens[s];
         q0 = min(max(p.qsl[s], 0), p.T);
         nq = min(max(p.qsl[s + 1], q0), p.T) - q0;
@@ -518,8 +519,9 @@ static hipError_t launch_prefill16_t(const AttnParams &p, int max_rows, hipStrea
     constexpr int ROWS = NW * NRT * 16;
     const int n_rb = (max_rows + ROWS - 1) / ROWS;
     const int pairs_per_xcd = (p.S * p.Hkv + 7) / 8;
-    const int64_t nwg = p.order ? (int64_t) p.n_order * p.Hkv
-                                : 8 * (int64_t) pairs_per_xcd * n_rb * std::max(1, p.n_split);
+    const int64_t nwg = p.order         ? (int64_t) p.n_order * p.Hkv
+                        : p.n_split > 1 ? (int64_t) p.split_blocks * p.n_split * p.Hkv
+                                        : 8 * (int64_t) pairs_per_xcd * n_rb;
     if (nwg > INT32_MAX) return hipErrorInvalidValue;
     const dim3 grid((unsigned) nwg), block(NW * 64);
     if (p.n_split > 1) {

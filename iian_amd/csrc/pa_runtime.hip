@@ -17,10 +17,13 @@
 //               (iian_pa_build_batch)
 //   layer       RoPE + the K/V write (iian_pa_rope_kv_write, or
 //               iian_pa_kv_write_kv without RoPE) and paged attention
-//               (iian_pa_attention) for one layer's pools
+//               (iian_pa_attention) for one layer's pools, its launches planned
+//               for the step's contexts, which begin_step has seen
 // Nothing is allocated after creation.  One runtime serves one stream at a
 // time (its buffers are per step).
 #include "../../include/iian_pa.h"
+
+#include "pa_launch.h"
 
 #include <hip/hip_runtime.h>
 
@@ -28,9 +31,12 @@
 #include <cstring>
 #include <new>
 
+using namespace iian_pa;
+
 struct iian_pa_runtime {
     iian_pa_runtime_config cfg;
     int device = 0;
+    int cus = 0;
     // device buffers
     int32_t *d_req = nullptr;     // [block ids (max_total_blocks)][block_off (S+1)][num_computed (S)][n_new (S)]
     int32_t *d_bt = nullptr;      // [max_seqs][max_blocks_per_seq]
@@ -48,6 +54,7 @@ struct iian_pa_runtime {
     int next = 0;
     // the step in flight
     int32_t S = 0, T = 0, max_q = 0;
+    StepLengths lengths = {0, false};
     bool in_step = false;
 };
 
@@ -89,7 +96,8 @@ int iian_pa_runtime_create(const iian_pa_runtime_config *cfg, iian_pa_runtime **
     iian_pa_runtime *rt = new (std::nothrow) iian_pa_runtime();
     if (!rt) return IIAN_PA_ERR_HIP;
     rt->cfg = c;
-    if (hipGetDevice(&rt->device) != hipSuccess) {
+    if (hipGetDevice(&rt->device) != hipSuccess ||
+        hipDeviceGetAttribute(&rt->cus, hipDeviceAttributeMultiprocessorCount, rt->device) != hipSuccess) {
         release(rt);
         return IIAN_PA_ERR_HIP;
     }
@@ -172,6 +180,22 @@ int iian_pa_runtime_begin_step(iian_pa_runtime *rt, void *stream, const int32_t 
     if (rc) return rc;
     rt->S = n_seqs;
     rt->T = (int32_t) T;
+    // the step's contexts, for the launches' plans: the table is as wide as the
+    // longest context of any step
+    rt->lengths = {0, false};
+    float blocks = 0.f, cells = 0.f, longest = 0.f;   // of the prefill sequences
+    const int32_t gqa = c.n_head / c.n_head_kv;
+    for (int32_t s = 0; s < n_seqs; s++) {
+        const int32_t len = num_computed[s] + n_new[s];
+        const int64_t rows = (int64_t) n_new[s] * gqa;
+        rt->lengths.longest = std::max(rt->lengths.longest, len);
+        if (rows <= 16) continue;
+        const float nb = (float) ((rows + kPrefillBlockRows - 1) / kPrefillBlockRows);
+        blocks += nb;
+        cells += nb * (float) len;
+        longest = std::max(longest, (float) len);
+    }
+    rt->lengths.uneven = prefill_uneven(blocks, cells, longest, (float) c.n_head_kv, (float) rt->cus);
     rt->max_q = max_q;
     rt->in_step = true;
     return IIAN_PA_OK;
@@ -198,10 +222,10 @@ int iian_pa_runtime_layer(iian_pa_runtime *rt, void *stream, const float *q, flo
                                  c.type_v, rt->d_err);
     }
     if (rc) return rc;
-    return iian_pa_attention(stream, qa, k_pool, v_pool, c.type_k, c.type_v, c.num_blocks, rt->d_bt,
+    return attention_of_step(stream, qa, k_pool, v_pool, c.type_k, c.type_v, c.num_blocks, rt->d_bt,
                              c.max_blocks_per_seq, rt->d_lens, rt->d_qsl, rt->d_pos, rt->T, rt->S, rt->max_q,
                              c.n_head, c.n_head_kv, c.head_dim, c.head_dim_v, c.block_size, scale, softcap, causal,
-                             n_swa, out, rt->d_ws, rt->ws_bytes, rt->d_err);
+                             n_swa, out, rt->d_ws, rt->ws_bytes, rt->d_err, rt->lengths);
 }
 
 int iian_pa_runtime_errors(iian_pa_runtime *rt, void *stream, int32_t *host_err) {

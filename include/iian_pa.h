@@ -118,7 +118,11 @@ size_t iian_pa_workspace_size(int32_t n_tokens, int32_t n_seqs, int32_t n_head, 
  *   k_pool, v_pool  the cell pools of one layer, num_blocks*block_size rows
  *                   (at most 2^32 rows, each under 1 GiB: IIAN_PA_ERR_UNSUPPORTED
  *                   beyond)
- *   block_tables    int32 [S][max_blocks] physical block ids
+ *   block_tables    int32 [S][max_blocks] physical block ids.  The launches are
+ *                   planned for contexts of up to max_blocks*block_size cells
+ *                   (from 32768 cells on, for contexts the host knows nothing
+ *                   of): a table no wider than the batch's longest sequence
+ *                   gives the best plan, any table the same cells attended
  *   seq_lens        int32 [S] cells of each sequence, this step's included
  *                   (UBatch::SeqInfo::cells.size(), include/iian/graph.h:33-36)
  *   query_start_loc int32 [S+1] tokens of sequence s are

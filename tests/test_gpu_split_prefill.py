@@ -1,5 +1,5 @@
 """Prefill row blocks cut into ranges of their cells (split_range in
-pa_common.h, the rule prefill_splits in pa_abi.hip) and their merge: one or a
+pa_split.h, the rule prefill_splits in pa_plan.h) and their merge: one or a
 few chunks over contexts at the edges of the 1024-cell minimum, for every
 prefill kernel.  Bar: the 2e-3 of the f16 kernels against the oracle."""
 import zlib
@@ -76,6 +76,21 @@ def test_split_rows_among_many_sequences(pa, oracle, S, H, Hkv, D, k_type):
     assert row_rel_err(got, oracle_attention(oracle, c)).max() <= (2e-5 if D in (80, 96) else TOL)
 
 
+@pytest.mark.parametrize("lens", [[4300] * 6, [9000, 4200, 1100, 1100, 1100, 1100]])
+@pytest.mark.parametrize("k_type", [F16, Q8_0])
+def test_cut_for_balance_or_left_alone(pa, oracle, k_type, lens):
+    """About one workgroup per CU at head size 256, planned for balance: an even
+    batch, which the kernel leaves uncut, and an uneven one.  Every 29th row."""
+    banner(f"split prefill balance type {k_type} {lens}")
+    c = make_case(np.random.default_rng(35), 16, 8, 256, lens, [210] * 6, k_type=k_type, quantize=oracle.quantize_q8_0)
+    err = torch.zeros(1, dtype=torch.int32, device="cuda")
+    got = gpu_attention(pa, c, err).reshape(-1, 256)
+    items = np.arange(0, c.T * c.H, 29)
+    want = oracle_attention(oracle, c, items=items).reshape(-1, 256)[items]
+    assert int(err.item()) == 0 and np.isfinite(got).all()
+    assert row_rel_err(got[items], want).max() <= TOL
+
+
 @pytest.mark.parametrize("k_type,D", [(F16, 128), (F16, 256), (Q8_0, 128)])
 def test_ranges_do_not_read_stale_records(pa, oracle, k_type, D):
     """Every record the merge uses is written by the call: the same bits over a
@@ -118,3 +133,32 @@ def test_rows_past_the_declared_length_are_left_alone(pa, oracle):
     assert int(err.item()) & 4
     assert row_rel_err(got[:32], want[:32]).max() <= TOL and row_rel_err(got[130:], want[130:]).max() <= TOL
     assert np.all(got[32:130] == 7.0)
+
+
+@pytest.mark.parametrize("H,Hkv,D,k_type", [(32, 8, 128, Q8_0), (16, 8, 256, F16), (14, 2, 64, F16)])
+def test_a_wide_runtime_plans_as_a_tight_one(pa, oracle, H, Hkv, D, k_type):
+    """The runtime plans its launches for the step's contexts: with a table eight
+    times as wide as the longest of them the cuts, and so the bits, are the same."""
+    banner(f"split prefill runtime width D={D} type {k_type}")
+    lens, nq = [3000, 2100, 40, 1500, 900], [100, 230, 40, 1, 1]
+    c = make_case(np.random.default_rng(34), H, Hkv, D, lens, nq, k_type=k_type, quantize=oracle.quantize_q8_0)
+    n_blk = [(L + c.bs - 1) // c.bs for L in lens]
+    ids = [c.bt[s, :n].tolist() for s, n in enumerate(n_blk)]
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(4)
+    new = [torch.randn((c.T, Hkv * D), generator=gen, device="cuda") for _ in range(2)]
+    outs = []
+    for width in (max(n_blk), 8 * max(n_blk)):
+        k, v, _ = to_device(pa, c)
+        rt = pa.PagedAttnRuntime(len(lens), c.T, width, sum(n_blk), H, Hkv, D, D, c.bs, c.k_pool.shape[0] // c.bs,
+                                 k_type, k_type)
+        rt.begin_step(ids, np.array(lens, np.int32) - np.array(nq, np.int32), np.array(nq, np.int32))
+        out = torch.full((c.T, H, D), float("nan"), device="cuda")
+        rt.layer(torch.as_tensor(c.q).cuda(), new[0], new[1], k, v, pa.PagedAttnParams(scale=c.scale), out)
+        assert rt.errors() == 0
+        outs.append(out.cpu().numpy())
+        c2 = make_case(np.random.default_rng(34), H, Hkv, D, lens, nq, k_type=k_type, quantize=oracle.quantize_q8_0)
+        c2.k_pool, c2.v_pool = k.data.cpu().numpy(), v.data.cpu().numpy()
+        assert row_rel_err(outs[-1], oracle_attention(oracle, c2)).max() <= TOL
+        rt.close()
+    assert np.array_equal(outs[0].view(np.uint32), outs[1].view(np.uint32))
