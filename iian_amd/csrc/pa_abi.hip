@@ -662,7 +662,10 @@ int run_attention(hipStream_t st, const float *q, const void *k_pool, const void
     const size_t split_at = align256(xl.total);
     p.n_split = 1;
     if (!decode_only) {
-        const size_t cap = src.scratch ? kScratchBytes : wl.total;
+        // the same room for both entry points, so that they cut alike and give the
+        // same bits (8 chunks of 256 tokens over 4K-16K cells at D = 256 then have
+        // records for 2 ranges instead of 3: 635 -> 639 us, within the runs' spread)
+        const size_t cap = std::min(kScratchBytes, wl.total);
         const PrefillCall c = {n_tokens, n_seqs, n_head_kv, gqa, n_swa, max_query_len, p.decode_rows, p.sk_workers,
                                head_dim, cus, mixed_one_launch, type_k == IIAN_PA_TYPE_Q8_0, len};
         p.n_order = prefill_order_entries(c);

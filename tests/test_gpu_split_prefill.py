@@ -135,6 +135,22 @@ def test_rows_past_the_declared_length_are_left_alone(pa, oracle):
     assert np.all(got[32:130] == 7.0)
 
 
+def test_both_entry_points_cut_alike(pa, oracle):
+    """A batch whose workspace holds records for more ranges than the library's
+    scratch does: the entry point without a workspace still gives the same bits."""
+    banner("split prefill both entry points")
+    lens = [9000, 4200, 6000, 7000, 2600, 3300, 5000, 4700]
+    c = make_case(np.random.default_rng(36), 16, 8, 256, lens, [256] * 8)
+    k, v, batch = to_device(pa, c)
+    q = torch.as_tensor(c.q).cuda()
+    want = pa.build_paged_attn(q, k, v, c.Hkv, pa.PagedAttnParams(scale=c.scale), batch).cpu().numpy()
+    from test_zz_no_alloc import call_noalloc
+    out = torch.empty((c.T, c.H, c.Dv), device="cuda")
+    err = torch.zeros(1, dtype=torch.int32, device="cuda")
+    assert call_noalloc(pa._lib.load(), c, q, k, v, batch, out, err) == 0
+    assert np.array_equal(out.cpu().numpy().view(np.uint32), want.view(np.uint32))
+
+
 @pytest.mark.parametrize("H,Hkv,D,k_type", [(32, 8, 128, Q8_0), (16, 8, 256, F16), (14, 2, 64, F16)])
 def test_a_wide_runtime_plans_as_a_tight_one(pa, oracle, H, Hkv, D, k_type):
     """The runtime plans its launches for the step's contexts: with a table eight
