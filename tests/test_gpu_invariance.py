@@ -7,19 +7,23 @@ op's outputs directly:
 
 * chunked prefill: a prompt's query tokens attended in one call, or in two
   consecutive calls (the second over the cells the first chunk would have
-  written), give the same rows bit for bit.  A prefill row's cells are walked
-  in the same tile order either way and masked cells add exact zeros, so the
-  row block a token lands in does not change its arithmetic.  With a sliding
-  window a row block's tiles start at its own window's first cell, so the
-  cells are grouped into tiles differently; a row's reference max (the one
-  its exponentials are taken against, moved lazily) then moves at other
-  tiles, which changes the f16 rounding of P, and rows agree to the 2e-3 bar
-  (5.6e-4 measured) instead of bit for bit;
-* batch composition: a prefill chunk attended alone or beside other
-  sequences gives the same rows bit for bit.  Decode rows are split into
-  stream-K pieces along the whole call's line of tiles, and each piece takes
-  its exponentials against its own running max, so the f16 rounding of P
-  follows the split: they agree to the 2e-3 bar (2e-4 measured).
+  written), give the same rows bit for bit up to 1024 cells.  A prefill row's
+  cells are walked in the same tile order either way and masked cells add exact
+  zeros, so the row block a token lands in does not change its arithmetic.
+  With a sliding window a row block's tiles start at its own window's first
+  cell, so the cells are grouped into tiles differently; a row's reference max
+  (the one its exponentials are taken against, moved lazily) then moves at
+  other tiles, which changes the f16 rounding of P, and rows agree to the 2e-3
+  bar (5.6e-4 measured) instead of bit for bit.  So do the rows of row blocks
+  over more than 1024 cells: a launch that leaves CUs idle cuts them into
+  ranges (pa_split.h), each range takes its exponentials against its own
+  running max, and how many there are follows the launch (5.3e-4 measured);
+* batch composition: a prefill chunk over at most 1024 cells attended alone or
+  beside other sequences gives the same rows bit for bit, over more cells to
+  the 2e-3 bar.  Decode rows are split into stream-K pieces along the whole
+  call's line of tiles, and each piece takes its exponentials against its own
+  running max, so the f16 rounding of P follows the split: they agree to the
+  2e-3 bar (2e-4 measured).
 
 Every call is also checked against the CPU oracle at the usual 2e-3 bar.
 """
@@ -133,3 +137,31 @@ def test_batch_composition(pa, oracle, name):
     e = row_rel_err(dec, together[n0:]).max()
     print(f"[gpu] {name}: decode rows alone against in the batch: max row rel diff {e:.3e}", flush=True)
     assert e <= TOL, (name, e)
+
+
+LONG = {
+    # name: (H, Hkv, D, lens, nq, kwargs); sequence 0 is a prefill chunk over more than 1024 cells, cut
+    # differently alone, beside a long decode and beside more chunks
+    "f16_d128": (32, 8, 128, [3000, 16000, 2500, 1800], [256, 1, 300, 256], {}),
+    "f16_d64": (14, 2, 64, [5000, 9000, 2500], [200, 1, 150], {}),
+    "f16_d256": (16, 8, 256, [4500, 6000, 2100, 1500], [128, 1, 256, 256], {}),
+    "q8_d128": (32, 8, 128, [3000, 7000, 2500], [256, 1, 300], {"k_type": Q8_0}),
+}
+
+
+@pytest.mark.parametrize("name", sorted(LONG))
+def test_long_chunks_agree_however_they_are_cut(pa, oracle, name):
+    H, Hkv, D, lens, nq, kw = LONG[name]
+    banner(f"long chunk {name} H={H} Hkv={Hkv} D={D} lens={lens} nq={nq} {kw}")
+    c = make_case(np.random.default_rng(sum(map(ord, name)) + 11), H, Hkv, D, lens, nq,
+                  quantize=oracle.quantize_q8_0, **kw)
+    n0, L0 = nq[0], lens[0]
+    alone = checked(pa, oracle, sub_case(c, [(0, 0, n0, L0)]), f"{name} alone")
+    halves = np.concatenate([checked(pa, oracle, sub_case(c, [(0, 0, n0 // 2, L0 - n0 + n0 // 2)]), f"{name} first half"),
+                             checked(pa, oracle, sub_case(c, [(0, n0 // 2, n0, L0)]), f"{name} second half")])
+    beside = gpu_attention(pa, sub_case(c, [(0, 0, n0, L0), (1, 0, 1, lens[1])]))[:n0]
+    batch = gpu_attention(pa, c)[:n0]
+    for got, what in ((halves, "in two chunks"), (beside, "beside a decode"), (batch, "in the batch")):
+        e = row_rel_err(got, alone).max()
+        print(f"[gpu] {name}: {what} against alone: max row rel diff {e:.3e}", flush=True)
+        assert e <= TOL, (name, what, e)
