@@ -546,21 +546,25 @@ __device__ __forceinline__ void gm_piece(const GenMfmaParams &p, const GmPiece &
                 for (int e = 0; e < CV; e++) x[e] = cell_visible(cw, 16 * (e >> 2) + 4 * g + (e & 3)) ? x[e] : -INFINITY;
                 // V of cells that no row of the wave attends (before its window, after
                 // its last position, the repeats past the last cell) may be infinite or
-                // NaN, and P = 0 must not meet it
+                // NaN, and P = 0 must not meet it.  The mask is held in a register and
+                // has a branch of its own up to head size 96 only: otherwise scalar
+                // registers spill (the branch costs 4-11% of the call at D = 112 and
+                // 160, to do without it 7% at D = 80; like this 0-3%).
                 const int v_lo = a.n_swa > 0 ? max(0, pc.pmin - a.n_swa + 1) : 0;
                 const int v_hi = a.causal ? min(pc.ce, pc.pmax + 1) : pc.ce;
-                if (tile < v_lo || tile + TC > v_hi) {
+                if (NK > 3 || __builtin_expect(tile < v_lo || tile + TC > v_hi, 0)) {
+                    const CellWindow vw = {v_lo - tile, (uint32_t) max(v_hi - v_lo, 0)};
 #pragma unroll
                     for (int c = 0; c < CV; c++) {
-                        const int cell = tile + 16 * (c >> 2) + 4 * g + (c & 3);
-                        const bool in = cell >= v_lo && cell < v_hi;
+                        uint32_t in = cell_visible(vw, 16 * (c >> 2) + 4 * g + (c & 3)) ? ~0u : 0u;
+                        asm volatile("" : "+v"(in));
 #pragma unroll
                         for (int b = 0; b < NV; b++) {
                             if constexpr (VT == 8) {
-                                vr[c][b].d = in ? vr[c][b].d : (uint16_t) 0;
+                                vr[c][b].d &= (uint16_t) in;
                             } else {
 #pragma unroll
-                                for (int w = 0; w < VE; w++) vr[c][b].a[w] = in ? vr[c][b].a[w] : 0u;
+                                for (int w = 0; w < VE; w++) vr[c][b].a[w] &= in;
                             }
                         }
                     }
