@@ -50,16 +50,10 @@ constexpr int kF16DecodeWavesPerCuPairs = 4;
 // per SIMD at head sizes up to 128 and one above; beside prefill workgroups 3
 // measured best (2 chunks + 16 decodes, H32/Hkv8/D128 F32: 187 us at 2 and 3,
 // 195 at 4, 203 at 6, 207 at 8; H16/Hkv16/D96 F32 153, 140, 154, 160, 173;
-// H32/Hkv32/D80 F16 128, 122, 122, 132, 141).  Prefill workgroups per CU a
-// launch is split for: F16 chunks are quick, and their records cost more than
-// a second workgroup per CU gives (2 chunks of 500 at H32/Hkv32/D80: 82 us at
-// 1, 97 at 2, 110 at 4); over F32 two balance better (the step above 207 at 1,
-// 195 at 2 and 4, with 4 decode waves).
+// H32/Hkv32/D80 F16 128, 122, 122, 132, 141).
 constexpr int kGenDecodeWavesPerCu = 8;
 constexpr int kGenMixedDecodeWavesPerCu = 3;
 constexpr int kGenDecodeWavesPerCuWide = 4;
-constexpr int kGenPrefillWgsPerCuF16 = 1;
-constexpr int kGenPrefillWgsPerCu = 2;
 constexpr int kQ8DecodeWavesPerCu = 8;
 constexpr int kMaxWavesPerCu = kQ8DecodeWavesPerCu;
 constexpr int kDefaultCus = 256;   // an MI355X, when the device cannot be queried
@@ -404,7 +398,9 @@ int run_attention(hipStream_t st, const float *q, const void *k_pool, const void
                       (int64_t) max_query_len * gqa > kDecodeRowsMax ||
                       !(mfma_path(type_k, type_v, head_dim, head_dim_v, bs_log2) || f16_96)))
         return IIAN_PA_ERR_UNSUPPORTED;
-    if (!mfma_path(type_k, type_v, head_dim, head_dim_v, bs_log2) && !f16_96 &&
+    const GeneralCall gc = {n_tokens, n_seqs, n_head_kv, gqa, max_query_len, head_dim, head_dim_v, type_k, type_v, cus,
+                            len.cells};
+    if (!mfma_path(type_k, type_v, head_dim, head_dim_v, bs_log2) && !f16_96 && !general_prefers_valu(gc) &&
         gen_mfma_path(head_dim, head_dim_v, block_size, max_blocks, num_blocks, kr, vr,
                       (int64_t) n_tokens * gqa)) {
         GenMfmaParams g = {};
@@ -468,19 +464,12 @@ int run_attention(hipStream_t st, const float *q, const void *k_pool, const void
             // every sequence that is not a decode one
             const int64_t rows = (int64_t) n_tokens * gqa;
             const int64_t n_rb = rows / 64 + std::min<int64_t>(n_seqs, rows / (a.decode_rows + 1));
-            // Ranges per row block: until the launch holds about
-            // kGenPrefillWgsPerCu workgroups per CU, each range at least 8
-            // tiles of the longest table, the records inside the workspace
-            const int64_t full = std::max<int64_t>(1, rows / 64) * n_head_kv;
-            const int64_t max_tiles = (len.cells + kTile - 1) / kTile;
-            const bool f16 = type_k == IIAN_PA_TYPE_F16 && type_v == IIAN_PA_TYPE_F16;
-            int64_t ns = ((int64_t) (f16 ? kGenPrefillWgsPerCuF16 : kGenPrefillWgsPerCu) * cus + full - 1) / full;
-            ns = std::min<int64_t>({ns, std::max<int64_t>(1, max_tiles / 8), kMaxSplits});
+            int64_t ns = gen_prefill_ranges(gc, a.decode_rows > 0, merge_lpr(head_dim_v));
             const size_t out_rows = (size_t) n_tokens * n_head;
             split_at = align256(xl.total);
             const size_t room = cap - std::min(split_at, cap);
             while (ns > 1 && split_bytes(out_rows, ns, head_dim_v) > room) ns--;
-            a.n_split = (int) std::max<int64_t>(ns, 1);
+            a.n_split = (int) ns;
             pre_wgs = n_rb * n_head_kv * a.n_split;
             if (a.n_split > 1) need = split_at + split_bytes(out_rows, a.n_split, head_dim_v);
         }

@@ -704,15 +704,18 @@ struct GmPieceIter {
         const SeqWindow w0 = seq_window(a, lane);
         nt = w0.nt;
         int total = wave_sum_i(nt);
-        bool over = w0.nq > a.max_q;
+        bool over = w0.nq > a.max_q, many = nt > 1;
         for (int b = 64; b < a.S; b += 64) {
             const SeqWindow wb = seq_window(a, b + lane);
             total += wave_sum_i(wb.nt);
             over |= wb.nq > a.max_q;
+            many |= wb.nt > 1;
         }
         if (worker == 0 && __builtin_amdgcn_ballot_w64(over) && lane == 0 && a.err) atomicOr(a.err, 4);
         total = __builtin_amdgcn_readfirstlane(total) * a.Hkv;
-        per = max(kMinPieceTiles, (total + a.sk_workers - 1) / a.sk_workers);
+        // (segments of one tile are not worth pairing: a worker would take two in turn)
+        const int least = __builtin_amdgcn_ballot_w64(many) ? kMinPieceTiles : 1;
+        per = max(least, (total + a.sk_workers - 1) / a.sk_workers);
         start = worker * per;
         end = min(total, start + per);
         base = 0;

@@ -42,14 +42,17 @@ hipError_t launch_gen_mfma(const GenMfmaParams &params, int type_k, int type_v, 
     p.staged = n_prefill_wgs > 0 && gm_staged(type_k, type_v, p.Dv);
     const int64_t wgs = p.n_dec_wgs + n_prefill_wgs;
     const int64_t seg = p.n_dec_wgs ? (int64_t) p.a.S * p.a.Hkv : 0;
-    // few segments: their records are many (on average more than 16 each)
+    // few segments: their records are many (on average more than 16 each).  Up to
+    // one per 12 workers, as the f16 merge, costs 18-21 sequences of 2000 cells at 8
+    // kv heads 0.2-0.6 us (D = 64 F32 32.5 -> 33.0, D = 96 Q8_0 42.9 -> 43.2), up to
+    // one per 8 as much again at 24-32; above head size 128 it makes no difference.
     const bool wide = seg * 16 <= p.a.sk_workers;
     const int seg_rows = (int) std::min<int64_t>(kGmRows, (int64_t) p.a.max_q * p.a.gqa);
     const int64_t seg_wgs = wide ? seg * seg_rows : seg;
     const int lpr = merge_lpr(p.Dv), rows_per_wg = 4 * (64 / lpr);
     const int64_t row_wgs =
         n_prefill_wgs && p.a.n_split > 1 ? ((int64_t) p.a.T * p.a.H + rows_per_wg - 1) / rows_per_wg : 0;
-    if (p.a.n_split > kMaxSplits) return hipErrorInvalidValue;
+    if (p.a.n_split > lpr) return hipErrorInvalidValue;
     if (wgs <= 0 || wgs > INT32_MAX || seg_wgs + row_wgs > INT32_MAX) return hipErrorInvalidValue;
     hipError_t e;
     switch (type_k) {

@@ -6,9 +6,6 @@
 
 namespace iian_pa {
 
-// Lanes that take a row of dv floats, 4 each.
-inline int merge_lpr(int dv) { return dv <= 64 ? 16 : dv <= 128 ? 32 : 64; }
-
 // Merge of np records of one row by WPR waves of a workgroup (1, or 4 with the
 // workgroup's LDS slice `comb`, 4 * (dv + 2) floats):
 //   out = sum_j 2^(m_j - m) O_j / sum_j 2^(m_j - m) l_j,  m = max_j m_j

@@ -119,4 +119,64 @@ inline int prefill_order_entries(const PrefillCall &c) {
     return (int) n;
 }
 
+// ---- The general path: pools and head sizes of pa_general.hip and pa_gen_mfma.h ----
+
+struct GeneralCall {
+    int32_t T, S, Hkv, gqa, max_q, D, Dv, type_k, type_v, cus;
+    int64_t cells;   // no context is longer, as far as the host knows
+};
+
+// Whether a call that pa_gen_mfma.h takes runs faster on pa_general_kernel: the
+// smallest decode calls, which it answers in one launch of a short kernel, where
+// the matrix-core kernel and its merge are two launches of 20-80 KB of code (32
+// cells: 10 against 18 us at H32/Hkv8/D128 F32, 12.6 against 26 at H16/Hkv8/D160
+// F16).  Its workgroups (one per sequence, kv head and 4 or 16 rows) walk 32
+// cells a tile up to head size 128, and 16 above, where it stays ahead longer
+// (16 sequences of 200 cells at H16/Hkv8/D256 F32 26.2 against 28.5, 4 of 512
+// 24.4 against 28.7; 64 of 64 cells 31 against 27).  More rows than one per wave
+// cost it more (5 tokens over 32 cells at H32/Hkv32/D80 F16 14 against 19.5, over
+// 64 21 against 14).
+inline bool general_prefers_valu(const GeneralCall &c) {
+    const int64_t rows = (int64_t) c.max_q * c.gqa, wgs = (int64_t) c.S * c.Hkv, work = wgs * c.cells;
+    const bool f16 = c.type_k == 1 && c.type_v == 1, q8 = c.type_k == 8 && c.type_v == 8;
+    if (rows > 16) return false;
+    if (c.D <= 128 && c.Dv <= 128) {
+        if (rows > 4) return c.cells <= 32 && wgs <= 2 * c.cus;
+        if (c.cells > 96) return q8 && c.cells <= 128 && 2 * wgs <= c.cus;
+        return wgs <= (rows == 1 && c.cells > 32 ? 1 : 2) * c.cus;
+    }
+    if (rows <= 4) return c.cells <= (f16 ? 256 : 512) && work <= 27000;
+    // (three tiles are cut into two pieces, which the matrix-core kernel merges)
+    return work <= 16384 && (f16 ? c.cells <= 32 || (c.cells > 64 && c.cells <= 96) : c.cells <= 128);
+}
+
+// Ranges per 64-row prefill block of pa_gen_mfma.h, at most most_ranges (a
+// merge's lanes): until the launch holds about as many full workgroups as pay,
+// each range at least 8 tiles of the longest context.  F16 chunks are quick, and
+// their records cost more than a second workgroup per CU gives (2 chunks of 500
+// at H32/Hkv32/D80: 82 us at 1, 97 at 2, 110 at 4); over F32 two balance better (2
+// chunks + 16 decodes at H32/Hkv8/D128 207 at 1, 195 at 2 and 4, with 4 decode
+// waves per CU).
+// A launch of 64 workgroups or fewer waits for one tile after another of them,
+// and is cut to 2 tiles while that leaves each its place on the device (one above
+// head size 128, whose workgroups have a CU alone): 20 tokens over 512 cells, one
+// sequence, H32/Hkv8/D128 F32 37 -> 18 us, H16/Hkv8/D256 67 -> 26; 4 of them over
+// 1024 cells 39 -> 35, but 46 with more workgroups than fit.  Over 128 cells that
+// pays only above head size 128 off F16 (35 -> 25 us; 12.5 -> 14.4 at D = 80).
+constexpr int kGenPrefillWgsPerCuF16 = 1;
+constexpr int kGenPrefillWgsPerCu = 2;
+inline int gen_prefill_ranges(const GeneralCall &c, bool decode_rows, int most_ranges) {
+    const int64_t rows = (int64_t) c.T * c.gqa, tiles = (c.cells + 31) / 32;
+    const bool f16 = c.type_k == 1 && c.type_v == 1, wide = c.D > 128 || c.Dv > 128;
+    const int64_t target = (f16 ? kGenPrefillWgsPerCuF16 : kGenPrefillWgsPerCu) * c.cus;
+    const int64_t full = std::max<int64_t>(1, rows / 64) * c.Hkv;
+    int64_t ns = std::min<int64_t>({(target + full - 1) / full, tiles / 8, kMaxSplits});
+    // partly filled blocks too, where no sequence is a decode one
+    const int64_t wgs = decode_rows ? full
+                                    : c.Hkv * std::min<int64_t>(rows / 64 + c.S, c.S * (((int64_t) c.max_q * c.gqa + 63) / 64));
+    if (wgs <= c.cus / 4 && (c.cells >= 256 || (!f16 && wide)))
+        ns = std::max(ns, std::min((wide ? c.cus : target) / wgs, (tiles + (8 * wgs <= c.cus)) / 2));
+    return (int) std::max<int64_t>(1, std::min<int64_t>(ns, most_ranges));
+}
+
 }  // namespace iian_pa

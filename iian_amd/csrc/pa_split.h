@@ -10,7 +10,10 @@
 namespace iian_pa {
 
 constexpr int kSplitMinCells = 1024;
-constexpr int kMaxSplits = 16;   // p.n_split at most: a row's (m, l) pairs fit the lanes of split_merge_rows
+constexpr int kMaxSplits = 16;   // p.n_split at most, for any head size
+// Lanes of a merge that take a row of dv floats, 4 each; a row's (m, l) pairs
+// must fit them (split_merge_rows).
+inline int merge_lpr(int dv) { return dv <= 64 ? 16 : dv <= 128 ? 32 : 64; }
 
 // Whether a launch of workgroups that have their CU alone is worth cutting for
 // balance: uncut, it takes the longest of them, or its rounds of average ones,

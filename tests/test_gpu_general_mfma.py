@@ -61,6 +61,19 @@ CASES = {
     "f16k_f32v_d128_random_pos": (8, 2, 128, [300, 200], [6, 70], {"v_type": F32, "pos_mode": "random"}),
     "f32k_f16v_d128_random_pos": (8, 2, 128, [300, 200], [6, 70], {"k_type": F32, "v_type": F16,
                                                                    "pos_mode": "random", "n_swa": 50}),
+    # both sides of the rules that leave a call to pa_general_kernel and of the ranges of few row blocks (pa_plan.h)
+    "f32_d128_table_of_96": (32, 8, 128, [1, 16, 33, 96], [1] * 4, {"k_type": F32}),
+    "f32_d128_table_of_112": (32, 8, 128, [1, 16, 33, 97], [1] * 4, {"k_type": F32}),
+    "f16_d80_one_tile_rows": (32, 32, 80, [32, 5, 17], [5, 5, 5], {}),
+    "f16_d112_one_tile_segments": (16, 8, 112, [32 - s % 30 for s in range(80)], [1] * 80, {}),
+    "q8_d96_table_of_128": (32, 8, 96, [128, 40], [1, 1], {"k_type": Q8_0}),
+    "f32_d256_16_of_200": (16, 8, 256, [200] * 16, [1] * 16, {"k_type": F32}),
+    "f16_d160_rows_of_96": (16, 8, 160, [96, 70], [5, 5], {}),
+    "f32_d128_20_tokens_16_ranges": (32, 8, 128, [1040], [20], {"k_type": F32}),
+    "f32_d256_20_tokens_of_520": (16, 8, 256, [520, 130], [20, 20], {"k_type": F32}),
+    "f32_d128_mqa_32_ranges": (32, 1, 128, [9000], [1], {"k_type": F32}),
+    "f32_d64_mqa_16_ranges": (32, 1, 64, [9000, 500], [1, 1], {"k_type": F32}),
+    "f32_d256_mqa_64_ranges": (32, 1, 256, [9000], [1], {"k_type": F32}),
     "f16_d80_one_chunk_splits": (8, 2, 80, [4000], [40], {}),          # prefill rows split over ranges
     "f32_d128_one_long_decode": (8, 2, 128, [9000], [1], {"k_type": F32}),   # more than 16 records a segment
     "f16_d80_130_sequences": (4, 2, 80, [20 + s for s in range(130)], [1 if s % 40 else 20 for s in range(130)], {}),

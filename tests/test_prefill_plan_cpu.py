@@ -1,7 +1,8 @@
 """How a prefill launch is cut and ordered (pa_plan.h, pa_split.h), compiled for
 the host: the ranges of a row block are a partition of its cells, and a launch
 is planned for the batch's contexts, not for the width of its table, where the
-host knows them or the table is as wide as a model's limit."""
+host knows them or the table is as wide as a model's limit; and the general
+path's choice of kernel and ranges at the edges of its rules."""
 import subprocess
 
 from iian_amd import build as B
@@ -79,6 +80,31 @@ int main() {
     CHECK(prefill_order_entries(call(128, 32, 8, 2600, 2600, 2600, false)) > 0);
     CHECK(prefill_order_entries(call(128, 32, 8, 2600, 2600, 131072, true)) > 0);
     CHECK(prefill_order_entries(call(128, 32, 8, 2600, 2600, 131072, false)) == 0);
+    // the general path: the smallest decode calls run on the VALU kernel, others do not
+    auto gen = [](int S, int H, int Hkv, int D, int q, int64_t cells, int tk = 0, int tv = 0) {
+        return GeneralCall{S * q, S, Hkv, H / Hkv, q, D, D, tk, tv, 256, cells};
+    };
+    CHECK(general_prefers_valu(gen(1, 32, 8, 128, 1, 96)) && !general_prefers_valu(gen(1, 32, 8, 128, 1, 97)));
+    CHECK(general_prefers_valu(gen(64, 32, 8, 128, 1, 96)) && !general_prefers_valu(gen(65, 32, 8, 128, 1, 96)));
+    CHECK(general_prefers_valu(gen(4, 32, 8, 96, 1, 128, 8, 8)) && !general_prefers_valu(gen(64, 32, 8, 96, 1, 128, 8, 8)));
+    CHECK(general_prefers_valu(gen(1, 32, 32, 80, 5, 32, 1, 1)) && !general_prefers_valu(gen(1, 32, 32, 80, 5, 33, 1, 1)));
+    CHECK(general_prefers_valu(gen(4, 16, 8, 256, 1, 512)) && !general_prefers_valu(gen(64, 16, 8, 256, 1, 64)));
+    CHECK(general_prefers_valu(gen(4, 16, 8, 160, 1, 256, 1, 1)) && !general_prefers_valu(gen(4, 16, 8, 160, 1, 512, 1, 1)));
+    CHECK(!general_prefers_valu(gen(1, 32, 8, 128, 1, 32768)) && !general_prefers_valu(gen(1, 32, 8, 128, 5, 16)));
+    // ranges: at least one, at most a merge's lanes, none of short contexts, more for few blocks
+    for (int S : {1, 3, 20, 200})
+        for (int q : {5, 20, 64, 500})
+            for (int64_t cells : {16, 100, 500, 5000, 200000})
+                for (int D : {40, 96, 128, 256})
+                    for (int type : {0, 1, 8}) {
+                        const int n = gen_prefill_ranges(gen(S, 32, 8, D, q, cells, type, type), false, merge_lpr(D));
+                        CHECK(n >= 1 && n <= merge_lpr(D) && n <= (cells + 31) / 32);
+                        if (cells <= 100 && D <= 128) CHECK(n == 1);
+                    }
+    CHECK(gen_prefill_ranges(gen(1, 32, 8, 128, 20, 512), false, 32) == 8);
+    CHECK(gen_prefill_ranges(gen(1, 32, 1, 128, 1, 16384), false, 32) == 32);
+    CHECK(gen_prefill_ranges(gen(4, 16, 8, 256, 64, 1024), false, 64) == 4);
+    CHECK(gen_prefill_ranges(gen(1000, 32, 8, 128, 20, 8000), false, 32) == 1);
     printf("%d bad\n", bad);
     return bad != 0;
 }
