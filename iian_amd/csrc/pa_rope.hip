@@ -352,7 +352,7 @@ __global__ __launch_bounds__(kRopeWaves * 64, 8) void pa_rope_vec_kernel(RopePar
     }
 }
 
-// The vector kernel's form: every pair of whole heads rotated (n_dims = D =
+// Whether a step goes to the vector kernel.  Its form: every pair of whole heads rotated (n_dims = D =
 // Dv), 4-element pieces within each half (and whole Q8_0 blocks), 16-byte
 // aligned rows.  (An f16 pool's pieces are 8 bytes, which the ABI requires.)
 static bool rope_vec_ok(const RopeParams &p, int type_k, int type_v) {
@@ -360,7 +360,15 @@ static bool rope_vec_ok(const RopeParams &p, int type_k, int type_v) {
     uintptr_t al = (uintptr_t) p.k_rows | (uintptr_t) p.v_rows | (uintptr_t) p.q_in | (uintptr_t) p.q_out;
     if (type_k == 0) al |= (uintptr_t) p.k_pool;
     if (type_v == 0) al |= (uintptr_t) p.v_pool;
-    return p.n_dims == p.D && p.Dv == p.D && p.D % (q8 ? 64 : 8) == 0 && p.D <= 512 && al % 16 == 0;
+    if (p.n_dims != p.D || p.Dv != p.D || p.D % (q8 ? 64 : 8) || p.D > 512 || al % 16) return false;
+    // Where it is faster: a step of few rows is answered in one round trip either
+    // way, and the kernel above has a wave per row and a shorter code (8 tokens of
+    // H32/Hkv8/D128 f16 4.5 against 5.0 us, 32 4.7 against 5.0, 128 5.3 against 4.9);
+    // few long rows per token leave this one's waves idle behind the table of 128
+    // or 256 pairs (889 tokens of K and V, 4 heads of 512, 11.8 against 13.4).
+    const int64_t rpt = (p.q_in ? p.H : 0) + 2 * (int64_t) p.Hkv, rows = p.T * rpt;
+    if (q8) return p.D >= 256 ? rpt >= 8 || rows < 3000 : rows >= 4096 && rpt >= 4;
+    return p.D >= 256 ? (rpt >= 24 && rows >= 6144) || (rpt >= 16 && rows >= 24576) : rows >= 6144 && rpt >= 4;
 }
 
 template <int KT, int VT>

@@ -42,6 +42,14 @@ def shifted(a, off):
     (2500, 32, 8, 128, (F16, Q8_0), 0, 0, False),
     (300, 32, 8, 128, (F16, F16), 2, 2, True),      # 8-byte aligned rows
     (300, 40, 8, 128, (F32, F32), 0, 0, True),
+    # both sides of the sizes the vector kernel is chosen from
+    (900, 5, 1, 8, (F32, F32), 0, 0, True),         # one lane per row
+    (300, 14, 2, 64, (Q8_0, Q8_0), 0, 0, True),
+    (1024, 2, 2, 64, (F16, F16), 2, 0, True),
+    (1023, 2, 2, 64, (F16, F16), 2, 0, True),
+    (900, 16, 8, 256, (F16, F16), 2, 0, False),
+    (1600, 16, 8, 256, (F16, F32), 0, 0, False),
+    (1500, 2, 1, 512, (Q8_0, F16), 2, 0, False),
 ])
 def test_rope_forms_bit_exact(pa, oracle, T, H, Hkv, D, types, mode, off, with_q):
     print(f"\n[gpu] rope form T={T} H={H} Hkv={Hkv} D={D} types={types} mode={mode} off={off}", flush=True)
