@@ -64,24 +64,36 @@ def pmc_traffic(config: str):
     return None if rec is None else int(rec["traffic_bytes_per_launch"])
 
 
+def merge_kernel(d: int, segments: int, workers: int) -> str:
+    """The instantiation launch_merge (pa_decode.hip) picks: waves per row, lanes per row."""
+    return f"pa_merge_kernel<{4 if segments * 12 <= workers else 1}, {16 if d <= 64 else 32 if d <= 128 else 64}>"
+
+
 def launch_kernels(sp, pa, max_blocks: int, block_size: int, cus: int) -> str:
     """The kernels one iian_pa_attention call of this workload launches (as
-    run_attention in pa_abi.hip picks them on a device of `cus` CUs)."""
+    run_attention in pa_abi.hip picks them on a device of `cus` CUs; prefill
+    launches that pa_plan.h cuts into ranges add pa_split_merge_kernel, and the
+    smallest general calls stay on pa_general_kernel)."""
     gqa = sp.H // sp.Hkv
     rows = [int(n) * gqa for n in sp.n_q]
     if sp.D == 96 and sp.kv_type == pa.GGML_TYPE_F16 and max(rows) <= 32:
-        return "pa_decode_f16_kernel<96> + pa_merge_kernel<96>"
+        pairs = max(rows) <= 8 and sp.Hkv % 2 == 0
+        merge = merge_kernel(96, len(rows) * sp.Hkv // (2 if pairs else 1), (4 if pairs else 6) * cus)
+        return f"pa_decode_f16_kernel<96> + {merge}"
     if (sp.D not in (64, 96, 128, 256) or (sp.D == 96 and sp.kv_type != pa.GGML_TYPE_F16)
             or sp.kv_type not in (pa.GGML_TYPE_F16, pa.GGML_TYPE_Q8_0)):
-        return "pa_gen_mfma_kernel + pa_gen_merge_kernel"
+        if sp.D % 8 == 0 and 32 < sp.D <= 256 and block_size % 16 == 0:
+            return "pa_gen_mfma_kernel + pa_gen_merge_kernel"
+        return "pa_general_kernel + pa_general_merge_kernel"
     has_dec = any(0 < r <= 32 for r in rows)
     has_pf = any(r > 32 for r in rows)
     d = sp.D
     if sp.kv_type == pa.GGML_TYPE_Q8_0:
-        dec = f"pa_decode_q8_kernel<{d}> + pa_merge_kernel<{d}>"
+        waves = 2 if 16 < max(rows) <= 32 else 1
+        dec = f"pa_decode_q8_kernel<{d}> + {merge_kernel(d, len(rows), 8 * cus // (waves * sp.Hkv))}"
         pf = f"pa_prefill_kernel<{d}, Q8_0>" if d <= 128 else f"pa_prefill16_kernel<{d}, Q8_0>"
     else:
-        dec = f"pa_decode_f16_kernel<{d}> + pa_merge_kernel<{d}>"
+        dec = f"pa_decode_f16_kernel<{d}> + {merge_kernel(d, len(rows) * sp.Hkv, (3 if d == 256 else 6) * cus)}"
         pf = f"pa_prefill_kernel<{d}, f16>" if d <= 128 else f"pa_prefill16_kernel<{d}, f16>"
         if has_pf and d <= 128:   # the mixed-batch instantiation, also without decode rows
             extra = " (decode pieces in the same grid, merged there)" if has_dec else ""
@@ -100,6 +112,11 @@ def launch_kernels(sp, pa, max_blocks: int, block_size: int, cus: int) -> str:
     if has_dec and has_pf:
         return f"{pf} || {dec} (two streams)"
     return pf if has_pf else dec
+
+
+def arithmetic_type(kernels: str) -> str:
+    """f16 MFMA operands with fp32 sums, or 32 bits throughout on the general kernels."""
+    return "f32" if kernels.startswith(("pa_gen_mfma_kernel", "pa_general_kernel")) else "f16"
 
 
 # The host-core share of one GPU on the GPU boxes: worker pools are sized to
@@ -365,8 +382,7 @@ def main() -> int:
         "higher_is_better": True,
         "scaling": "weak",
         "vs_baseline": None,
-        # the arithmetic type: f16 MFMA operands (fp32 sums), or fp32 throughout on the general kernel
-        "dtype": "f32" if "general" in kernels else "f16",
+        "dtype": arithmetic_type(kernels),
         "data": "synthetic",
         "step_calls": step_calls,
         "two_call_ms_per_step": round(two_call_ms, 5) if two_call_ms else None,

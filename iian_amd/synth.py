@@ -11,7 +11,7 @@ Configurations (BASELINE.json ``configs``):
   cfg1            Qwen2.5-0.5B decode: H14/Hkv2/D64, 8 seqs, L~U[64,1024], 1024-block pool
   cfg2            Llama-3-8B decode: H32/Hkv8/D128, 64 seqs, L log-uniform [512,8192],
                   65536-block pool, plus the KV write of the 64 new tokens
-                  (cfg2_f32: the same with F32 K/V pools, the general fp32 kernel)
+                  (cfg2_f32: the same with F32 K/V pools, the matrix-core general kernel)
   cfg3            Qwen3-8B mixed batch: 4 prefill chunks of 512 tokens over a prior
                   context P~U[1024,4096] whose first 1024 tokens (64 blocks) are shared
                   by all 4 sequences, plus 32 decode tokens with L~U[1024,4096]
