@@ -1,8 +1,9 @@
-"""The merge launch of the decode kernels on both sides of its rule (a
-workgroup per row up to one segment per 8 stream-K workers, a wave per row
-above), for every head size and record layout: one head, head pairs at head
-size 96, grouped Q8_0 records, two 16-row tiles.  Bar: the 2e-3 of the f16
-kernels (P is rounded to f16 there), as the other decode tests."""
+"""The merge launches of the decode kernels on both sides of their rules (a
+workgroup per row up to one segment per 12 stream-K workers, or per 16 on the
+general path, a wave per row above), for every head size and record layout: one
+head, head pairs at head size 96, grouped Q8_0 records, two 16-row tiles.  Bar:
+the 2e-3 of the f16 kernels (P is rounded to f16 there), as the other decode
+tests."""
 import zlib
 
 import numpy as np
@@ -29,8 +30,16 @@ CASES = {
     "d96_verify": (8, 2, 96, [5000, 40], [5, 1], {}),
     "d128_verify5_two_tiles": (32, 8, 128, [7000, 2100], [5, 5], {}),
     "d128_few_records": (32, 8, 128, [90, 70], [1, 1], {}),
-    "d128_24_sequences": (8, 8, 128, [1000 + 40 * s for s in range(24)], [1] * 24, {}),   # 192 segments, 1536 workers
+    "d128_24_sequences": (8, 8, 128, [1000 + 40 * s for s in range(24)], [1] * 24, {}),   # 1536 workers
     "d128_25_sequences": (8, 8, 128, [1000 + 40 * s for s in range(25)], [1] * 25, {}),
+    "d128_16_sequences": (8, 8, 128, [1000 + 40 * s for s in range(16)], [1] * 16, {}),   # 128 segments: the last
+    "d128_17_sequences": (8, 8, 128, [1000 + 40 * s for s in range(17)], [1] * 17, {}),   # one with a workgroup per row
+    "q8_d128_21_sequences": (8, 8, 128, [600 + 10 * s for s in range(21)], [1] * 21, {"k_type": Q8_0}),   # 256 workers
+    "q8_d128_22_sequences": (8, 8, 128, [600 + 10 * s for s in range(22)], [1] * 22, {"k_type": Q8_0}),
+    "f32_d128_16_sequences": (8, 8, 128, [1000 + 40 * s for s in range(16)], [1] * 16, {"k_type": F32}),   # 2048 workers
+    "f32_d128_17_sequences": (8, 8, 128, [1000 + 40 * s for s in range(17)], [1] * 17, {"k_type": F32}),
+    "f16_d160_8_sequences": (8, 8, 160, [1000 + 40 * s for s in range(8)], [1] * 8, {}),                   # 1024
+    "f16_d160_9_sequences": (8, 8, 160, [1000 + 40 * s for s in range(9)], [1] * 9, {}),
     "d256_one_sequence": (16, 8, 256, [9000], [1], {}),
     "q8_d64_one_sequence": (14, 2, 64, [6000], [1], {"k_type": Q8_0}),
     "q8_d128_verify5": (32, 8, 128, [7000, 300], [5, 5], {"k_type": Q8_0}),
