@@ -3,18 +3,20 @@
 //
 // K and V each F32, F16 or Q8_0 in any pairing, head sizes up to 256 (D a
 // multiple of 8, Dv of 4, gen_mfma_chunks), blocks of a multiple of 16 cells,
-// Dv != D.  Precision is that of
-// pa_general_kernel, which keeps every other combination: nothing of the
-// computation drops below 32 bits.
+// Dv != D.  pa_general_kernel keeps every other combination and the smallest
+// decode calls (general_prefers_valu, pa_plan.h).  Scores and sums are held in 32
+// bits, as are probabilities except over F16 V (22).
 //
 //   K F32 or Q8_0  S^T = K Q^T on v_mfma_f32_16x16x4_f32; a Q8_0 value is
 //                  q * fp32(d), exactly dequantize_row_q8_0 (ggml-quants.c:553-567)
 //   K F16          K is exact in f16, and q goes in as three f16 terms (11 + 11
-//                  + 11 bits, each rounded toward zero: the whole fp32 value)
-//                  on v_mfma_f32_16x16x32_f16: 3 x 16 cycles per 32 dims where
-//                  the fp32 form takes 8 x 32
+//                  + 11 bits, each rounded toward zero: the fp32 value, down to
+//                  2^-38 of the row's largest element) on
+//                  v_mfma_f32_16x16x32_f16: 3 x 16 cycles per 32 dims where the
+//                  fp32 form takes 8 x 32
 //   V F32 or Q8_0  O += P V on the fp32 MFMA, P in fp32
-//   V F16          V exact, P as two f16 terms (22 bits), on the f16 MFMA
+//   V F16          V exact, P as two f16 terms (22 bits, or to 2^-31 of the row's
+//                  largest P where that is coarser), on the f16 MFMA
 //
 // Work split.  One wave owns 16 query rows (r = j*gqa + g) of one (sequence,
 // kv head) and walks 32-cell tiles (16 when V is not F16) through the block
@@ -44,7 +46,10 @@
 // 512-8192 cells over F32 pools, H32/Hkv8/D128, 215 -> 158 us (5.2 TB/s); those
 // 2 chunks and 16 decodes over F32 1448 -> 186 us; 2 chunks of 500 and 16
 // decodes over F16 at H32/Hkv32/D80 9030 -> 122 us.  Distance from a 64-bit
-// result there: 6.5e-7 -> 4.1e-7 (F32), 6.3e-7 -> 5.7e-7 (F16, D80).
+// result there: 6.5e-7 -> 4.1e-7 (F32), 6.3e-7 -> 5.7e-7 (F16, D80).  Over 116
+// rows and chunks of 600-60000 cells, flat to peaked, in five pairings: 1e-7 to
+// 2.0e-6, pa_general_kernel 4e-8 to 2.7e-6, the median ratio 0.99 (P's reference 4
+// or 6 log2 units lower changes none of it, and 6 costs F16 chunks 3-5%).
 #pragma once
 
 #include "pa_common.h"
@@ -127,11 +132,11 @@ struct GmPiece {
     int rec;
 };
 
-// x = h + m + l exactly, each f16 rounded toward zero.  x is scaled below
-// 2^15 by the caller.  m and l are kept non-zero (2^-24) where h alone is
-// exact, so that an infinite K element times the three terms gives one signed
-// infinity, as its fp32 product does, and never inf * 0.  The differences
-// pass through empty asm: folded into a mixed-precision FMA with a negated
+// x = h + m + l, each f16 rounded toward zero: exactly, as far as the third
+// term reaches (2^-24).  x is scaled below 2^15 by the caller.  m and l are kept
+// non-zero (+-2^-24, 2^-38 of the row's largest) where h alone is exact, so that
+// an infinite K element times the three terms gives one signed infinity, as its
+// fp32 product does, and never inf * 0.  The differences pass through empty asm: folded into a mixed-precision FMA with a negated
 // operand they have come out wrong (see split_f16x8).
 __device__ __forceinline__ void gm_split3(float x, _Float16 &h, _Float16 &m, _Float16 &l) {
     typedef __fp16 h2 __attribute__((ext_vector_type(2)));
@@ -437,8 +442,9 @@ __device__ __forceinline__ void gm_piece(const GenMfmaParams &p, const GmPiece &
     };
 
     // m_ref: the row's reference in log2 units, 7 below the largest score it
-    // was last moved to, so that P lies in [0, 2^15] (the range in which two
-    // f16 terms hold 22 bits of every P down to 2^-32 of the largest)
+    // was last moved to, so that P lies in [0, 2^15] and its largest in [2^7,
+    // 2^15]: two f16 terms leave out 2^-22 of a P, or 2^-24 (2^-31 of the
+    // largest) where that is more
     float m_ref = -INFINITY, m_sub = 0.f, l_run = 0.f;   // m_sub: m_ref, or 0 while no cell was visible
     f32x4 o[4 * NV];
 #pragma unroll

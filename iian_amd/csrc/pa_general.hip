@@ -3,7 +3,8 @@
 // 256] in multiples of 8 over blocks of a multiple of 16 cells): head sizes up
 // to 32, above 256 (up to 1024) or not a multiple of 8, and other block sizes,
 // over F32, F16 and Q8_0 pools in any pairing (Q8_0 in multiples of 32),
-// Dv != D.  Head sizes that are not multiples of 4 are staged in
+// Dv != D; and, of pa_gen_mfma.h's, the smallest decode calls, which it answers
+// sooner (general_prefers_valu, pa_plan.h).  Head sizes that are not multiples of 4 are staged in
 // LDS rows padded with zeros to the next multiple of 4 (the reference's
 // dot and axpy loops run to any D, paged_attn.cpp:39,50), with element-wise
 // global loads and stores, since their rows are not 16-byte aligned.

@@ -50,16 +50,16 @@ struct SplitPlan {
     int32_t row_blocks;   // row blocks the batch can hold
 };
 
-// A launch whose row
-// blocks take at most half of the device's workgroup slots is cut to fill
-// them; more ranges than that only add starts and records (one 256-token chunk
+// A launch whose row blocks take at most half of the device's workgroup slots is
+// cut to fill them; more ranges than that only add starts and records (one 256-token chunk
 // over 10K cells at H16/Hkv8/D256: 481 us uncut, 87 with one workgroup per CU,
 // 136 with two rounds of them).  D <= 128 kernels hold two workgroups per CU,
 // less the decode workers of a mixed launch (4 chunks' worth of slots taken
 // from 2 chunks of 512 beside 32 decodes cost 365 -> 390 us).  At D = 256,
 // where a workgroup has its CU alone and the longest one decides a launch of
 // about one round, such a launch is planned for 3 rounds and the kernel cuts it
-// when the batch is uneven (8 chunks of 256 over 4K-16K cells 784 -> 614 us; 2
+// when the batch is uneven (8 chunks of 256 over 4K-16K cells 782 -> 642 us with
+// the 2 ranges that the scratch holds of their rows, 628 with 3; planned for 2
 // rounds 0-3% either way on other lengths).  Measured besides, whole calls: 8 Q8_0
 // kv heads, chunks of 504 and 361 tokens over 1.6K-2.7K cells beside 24
 // decodes, two layers, 394 -> 301 us; one chunk of 250 tokens over 8.5K cells at
@@ -70,8 +70,8 @@ struct SplitPlan {
 // beside 16 159 -> 94.  Two ranges of little more than kSplitMinCells cells do
 // not pay over f16 pools when every XCD has its share of row blocks (8 chunks of
 // 256 tokens over 2100 cells at H14/Hkv2/D64 43.6 -> 45.1 us; at H32/Hkv32/D96
-// 4 of 256 over 3200 77.5 -> 80.5), as they do over Q8_0, whose tiles take longer (the same at H32/Hkv8/D128, 2 chunks beside 32
-// decodes, 123 -> 95).
+// 4 of 256 over 3200 77.5 -> 80.5), as they do over Q8_0, whose tiles take longer
+// (the same at H32/Hkv8/D128, 2 chunks beside 32 decodes, 123 -> 95).
 inline SplitPlan prefill_splits(const PrefillCall &c) {
     const int64_t rows = (int64_t) c.T * c.gqa;
     const int64_t blocks = std::max<int64_t>(1, rows / kPrefillBlockRows) * c.Hkv;

@@ -4,10 +4,10 @@ contexts at the edges of a 16- or 32-cell tile, row counts at the edges of a
 wave's 16 rows and a workgroup's 64, every type pairing, block sizes that are
 multiples of 16 but not powers of two, and non-finite K entries.
 
-Bar: 2e-5 of each row's largest value against the oracle.  Everything is held
-and summed in at least 24 bits: a score of a few tens is off by some 2^-24 of
-its size (4e-6 at 64), P by as much, and the oracle's own fp32 sums by the
-same again.
+Bar: 2e-5 of each row's largest value against the oracle.  A score is held and
+summed in 24 bits: one of a few tens is off by some 2^-24 of its size (4e-6 at
+64), P by as much and, over F16 V, by 2^-22 of its own (2.4e-7) from its two f16
+terms, and the oracle's own fp32 sums by the same again.
 """
 import zlib
 
