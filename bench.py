@@ -2,8 +2,8 @@
 
     python bench.py [--steps K] [--warmup W] [--config cfg2] [--no-cpu-baseline]
 
-A step is one layer-call of the path at Llama-3-8B decode shapes (BASELINE
-config 2): the slot-mapped KV write of the 64 new tokens (K and V pools) and
+A step is one layer-call of the path at Llama-3-8B decode shapes
+(cfg2): the slot-mapped KV write of the 64 new tokens (K and V pools) and
 paged GQA decode attention over the block pool, inputs resident in HBM.
 ``value`` is the achieved algorithmic HBM bandwidth of the whole step (GB/s);
 ``attn_tok_per_s`` the query tokens per second of one layer-call.
@@ -119,8 +119,8 @@ def arithmetic_type(kernels: str) -> str:
     return "f32" if kernels.startswith(("pa_gen_mfma_kernel", "pa_general_kernel")) else "f16"
 
 
-# The host-core share of one GPU on the GPU boxes: worker pools are sized to
-# it whatever nproc reports there.
+# The host-core share of one GPU: worker pools are sized to it whatever nproc
+# reports.
 CPU_SHARE = 16
 
 
@@ -427,7 +427,7 @@ def main() -> int:
                       f"median of 5 runs after 1 warm-up, {med * 1e3:.1f} ms/step on {t_share} threads",
             "cpu_model": model, "nproc": nproc, "cores_available": avail,
             "threads_policy": f"min(nproc, hardware_concurrency()/2 = {nproc // 2}) capped at the "
-                              f"{CPU_SHARE}-core host share of one GPU on this pool: {t_share} and {t_half} threads",
+                              f"{CPU_SHARE}-core host share of one GPU: {t_share} and {t_half} threads",
             "half_concurrency": {"threads": t_half, "value": round(b_step / med_half / 1e9, 2),
                                  "ms_per_step": round(med_half * 1e3, 1)},
             "single_thread": {"value": round(b_step / med1 / 1e9, 3), "ms_per_step": round(med1 * 1e3, 1)},

@@ -132,11 +132,12 @@ WorkspaceLayout exact_layout(const AttnParams &p) {
 // ---- Scratch of the no-allocation entry point (iian_pa_attention_noalloc) ----
 //
 // A file-scope device array, one copy per GPU, living until the process
-// ends.  kScratchBytes covers every BASELINE configuration's call (the
-// largest, Q8_0 spec-verify at 128 sequences x 8 kv heads, uses 34 MB).  On
-// the host, `scratch` names a stand-in, not device memory: its device
-// address is taken once per device with hipGetSymbolAddress (with that
-// device current) and only that address is ever handed to kernels.
+// ends.  kScratchBytes covers every benchmark configuration's call (the
+// largest, Q8_0 spec-verify at 128 sequences x 8 kv heads, needs 34 MB; records
+// of prefill rows cut into ranges take what is left).  On the host, `scratch`
+// names a stand-in, not device memory: its device address is taken once per
+// device with hipGetSymbolAddress (with that device current) and only that
+// address is ever handed to kernels.
 constexpr size_t kScratchBytes = (size_t) 64 << 20;
 static __device__ __align__(256) char scratch[kScratchBytes];
 

@@ -7,7 +7,7 @@ Block tables are seeded random permutations of the physical block ids, so a
 sequence's blocks are scattered over the pool as in a long-running engine
 (src/iian/kv_cache.cpp:214-229 hands out blocks from a free list).
 
-Configurations (BASELINE.json ``configs``):
+Configurations:
   cfg1            Qwen2.5-0.5B decode: H14/Hkv2/D64, 8 seqs, L~U[64,1024], 1024-block pool
   cfg2            Llama-3-8B decode: H32/Hkv8/D128, 64 seqs, L log-uniform [512,8192],
                   65536-block pool, plus the KV write of the 64 new tokens

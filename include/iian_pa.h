@@ -160,8 +160,9 @@ int iian_pa_attention(void *stream, const float *q, const void *k_pool, const vo
  * mixed batch that iian_pa_attention splits over a side stream runs its two
  * kernels in order on `stream` here).  Its first call on a device looks up
  * that device's copy of the array once.  A call needing more scratch than the
- * array holds returns IIAN_PA_ERR_SCRATCH before any launch (every BASELINE
- * configuration fits; the largest uses 34 MB).  Nothing in the array needs
+ * array holds returns IIAN_PA_ERR_SCRATCH before any launch (every benchmark
+ * configuration fits; the largest needs 34 MB, and records of prefill rows cut
+ * into ranges take what is left).  Nothing in the array needs
  * clearing between calls: every record is written before it is read within a
  * call, and the merge counters carry a per-call tag.  All calls on one GPU
  * share the array, so calls that overlap on one GPU (different streams, or

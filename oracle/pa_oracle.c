@@ -1,7 +1,7 @@
 /*
  * pa_oracle.c - CPU restatement of iian's paged-attention path (the oracle).
  *
- * TEST INFRASTRUCTURE ONLY: the checker the HIP kernels are compared against.
+ * TEST INFRASTRUCTURE ONLY: what the HIP kernels are compared against.
  * Only tests/, __graft_entry__.smoke() and bench.py's cpu_baseline leg may
  * load it; the product library never does.
  *

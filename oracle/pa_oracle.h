@@ -2,7 +2,7 @@
  * pa_oracle.h - CPU restatement of iian's paged-attention path.
  *
  * TEST INFRASTRUCTURE ONLY.  Nothing in the product (iian_amd/, include/) may
- * link, import or call this code.  It is the checker that the HIP kernels are
+ * link, import or call this code.  It is what the HIP kernels are
  * compared against: used by tests/, by __graft_entry__.smoke() and by the
  * cpu_baseline leg of bench.py, and nowhere else.
  *

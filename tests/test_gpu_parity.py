@@ -1,8 +1,8 @@
 """GPU parity: the gfx950 kernels (through the C ABI) against the CPU oracle.
 
 Bars: KV-write placement and Q8_0 values bit-exact; attention max relative
-error per (token, head) row, max|y - r| / max|r|, at most 2e-3 (BASELINE
-north star; fp32 accumulation in both).
+error per (token, head) row, max|y - r| / max|r|, at most 2e-3 (fp32
+accumulation in both).
 """
 import zlib
 

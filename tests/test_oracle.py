@@ -1,4 +1,4 @@
-"""Pins the CPU oracle (oracle/pa_oracle.c) before it is trusted as the checker.
+"""Pins the CPU oracle (oracle/pa_oracle.c) before it is trusted.
 
 * fp16 conversions against numpy's IEEE float16 casts;
 * Q8_0 quantise/dequantise bit for bit against ggml's own routines compiled
